@@ -5,17 +5,19 @@
 // losses.py:34-38 given the forward's lse and log-probs).
 //
 // Layout and schedule (gfx950, wave64):
-//   * A persistent grid of one 1024-lane workgroup per CU walks rows
-//     r = blockIdx.x, blockIdx.x + gridDim.x, ...
+//   * A persistent grid of NT-lane workgroups, as many as fit the CUs, walks
+//     rows r = blockIdx.x, blockIdx.x + gridDim.x, ...  NT runs from 64 (short
+//     rows, many of them per CU) to 1024 (one row per CU); see launch_variant.
 //   * A row of V 16-bit logits is held in VGPRs as SL slabs of one 16-byte
-//     vector per lane: slab k, lane j holds vector k*1024 + j.  V = 151936
-//     (bf16) is 18992 vectors, SL = 19 of the SL = 20 variant, i.e. 80 VGPRs.
+//     vector per lane: slab k, lane j holds vector k*NT + j.  V = 151936
+//     (bf16) is 18992 vectors, 19 slabs of the NT = 1024, SL = 20 variant,
+//     i.e. 80 VGPRs.
 //   * Per-row scalars (target, old log-prob, advantage, mask weight * 1/M)
 //     come from a packed 16-byte record per token (pack_records_kernel), read
 //     a row ahead through the scalar cache.
 //   * Sweep 1 (registers only): online max / sum of exp over the non-target
 //     columns per lane, slab by slab as the loads land, then one LDS combine
-//     across the 16 waves.
+//     across the workgroup's waves.
 //   * Sweep 2: each slab becomes g * (onehot - exp(x - lse)), is packed back to
 //     16 bits and stored with a non-temporal buffer store; once the whole row
 //     is stored, the same registers are refilled with the workgroup's next
@@ -33,7 +35,8 @@ namespace rrl {
 
 namespace {
 
-constexpr int RNT = 1024;                 // lanes per workgroup (16 waves)
+constexpr int kMaxSlabs = 20;       // slabs per lane: 80 VGPRs of the 128 at 4 waves per SIMD
+constexpr int kWavesPerSimd = 4;
 
 // Element access of one 16-byte vector per tag: EPV elements, their float
 // values, the packed form written back (round to nearest even for 16-bit),
@@ -241,8 +244,8 @@ __device__ __forceinline__ float exp_arg(float x, const ExpArg& q) {
     return __builtin_fmaf(x, kLog2e, q.cg);
 }
 
-template <class Tag, int SL, bool EXTRAS>
-__global__ __launch_bounds__(RNT) void resident_fused_kernel(RowArgs a, int32_t nvec) {
+template <class Tag, int NT, int SL, bool EXTRAS>
+__global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowArgs a, int32_t nvec) {
   using P = Pack16<Tag>;
   using S = typename Tag::S;
   constexpr int EPV = P::EPV;
@@ -250,8 +253,8 @@ __global__ __launch_bounds__(RNT) void resident_fused_kernel(RowArgs a, int32_t 
   // Double-buffered by combine parity: a wave can run at most one combine
   // ahead of the slowest (each combine has one barrier), so the buffer it
   // writes is never the one another wave is still reading.
-  __shared__ float sh_m[2][RNT / 64];
-  __shared__ float sh_s[2][RNT / 64];
+  __shared__ float sh_m[2][NT / 64];
+  __shared__ float sh_s[2][NT / 64];
   __shared__ float sh_xt[2];
   int buf = 0;
 
@@ -296,7 +299,7 @@ __global__ __launch_bounds__(RNT) void resident_fused_kernel(RowArgs a, int32_t 
     // loads), not for the whole row.
 #pragma unroll
     for (int k = 0; k < SL; ++k) {
-      x[k] = __builtin_amdgcn_raw_buffer_load_b128(src, voff, k * RNT * 16, kAuxLoad);
+      x[k] = __builtin_amdgcn_raw_buffer_load_b128(src, voff, k * NT * 16, kAuxLoad);
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (EXTRAS) {
@@ -322,7 +325,7 @@ __global__ __launch_bounds__(RNT) void resident_fused_kernel(RowArgs a, int32_t 
     if (has_next) rec_next = load_record(a.records, rn);
     const int32_t tgt = rec.target;
     const bool tgt_ok = tgt >= 0;
-    // Slab k of this lane holds the target iff rel == k * RNT; a target in
+    // Slab k of this lane holds the target iff rel == k * NT; a target in
     // the head or tail is the extra element of lane ei == tgt.
     const int32_t bt = tgt - (int32_t)g.head;
     const bool in_body = tgt_ok && (!EXTRAS || (bt >= 0 && bt < (int32_t)(g.nbody * EPV)));
@@ -338,7 +341,7 @@ __global__ __launch_bounds__(RNT) void resident_fused_kernel(RowArgs a, int32_t 
     // and slab that hold it.
     float m = -__builtin_huge_valf(), s = 0.0f;
     auto fold = [&](int k) {
-      if (lane < (int)g.nbody - k * RNT) {
+      if (lane < (int)g.nbody - k * NT) {
         float v[EPV];
         P::unpack(x[k], v);
         const float mn = fmaxf(m, vmax(v));
@@ -347,7 +350,7 @@ __global__ __launch_bounds__(RNT) void resident_fused_kernel(RowArgs a, int32_t 
 #pragma unroll
         for (int i = 0; i < EPV; ++i) e[i] = exp2_hw((v[i] - mg) * kLog2e);
         float se = vsum(e);
-        if (rel == k * RNT) {
+        if (rel == k * NT) {
           float xv = v[0], so = 0.0f;
 #pragma unroll
           for (int i = 0; i < EPV; ++i) {
@@ -383,7 +386,7 @@ __global__ __launch_bounds__(RNT) void resident_fused_kernel(RowArgs a, int32_t 
       if (!tgt_ok && tid == 0) sh_xt[buf] = -__builtin_huge_valf();
       // Workgroup combine, kept short: the next row's loads are not issued
       // until it ends.  Wave max, then the rescaled sum (one exponential per
-      // lane), then the 16 wave pairs through LDS with one barrier.
+      // lane), then the wave pairs through LDS with one barrier.
       const float Mw = wave_max_dpp(m);
       const float Sw = wave_sum_dpp(rescale(s, m, Mw));
       if ((tid & 63) == 0) {
@@ -391,17 +394,17 @@ __global__ __launch_bounds__(RNT) void resident_fused_kernel(RowArgs a, int32_t 
         sh_s[buf][tid >> 6] = Sw;
       }
       lds_barrier();
-      float mw[RNT / 64];
+      float mw[NT / 64];
 #pragma unroll
-      for (int i = 0; i < RNT / 64; ++i) mw[i] = sh_m[buf][i];
+      for (int i = 0; i < NT / 64; ++i) mw[i] = sh_m[buf][i];
       m = mw[0];
 #pragma unroll
-      for (int i = 1; i < RNT / 64; ++i) m = fmaxf(m, mw[i]);
-      float sp[RNT / 64];
+      for (int i = 1; i < NT / 64; ++i) m = fmaxf(m, mw[i]);
+      float sp[NT / 64];
 #pragma unroll
-      for (int i = 0; i < RNT / 64; ++i) sp[i] = rescale(sh_s[buf][i], mw[i], m);
+      for (int i = 0; i < NT / 64; ++i) sp[i] = rescale(sh_s[buf][i], mw[i], m);
 #pragma unroll
-      for (int w = RNT / 128; w > 0; w >>= 1)
+      for (int w = NT / 128; w > 0; w >>= 1)
 #pragma unroll
         for (int i = 0; i < w; ++i) sp[i] += sp[i + w];
       s = sp[0];
@@ -467,13 +470,13 @@ __global__ __launch_bounds__(RNT) void resident_fused_kernel(RowArgs a, int32_t 
       P::unpack(x[k], v);
 #pragma unroll
       for (int i = 0; i < EPV; ++i) d[i] = exp2_hw(exp_arg<Tag>(v[i], q));
-      if (rel == k * RNT) {
+      if (rel == k * NT) {
 #pragma unroll
         for (int i = 0; i < EPV; ++i) d[i] = (i == ti) ? tgt_pre : d[i];
       }
       u32x4 o = P::pack(d);
       o.x ^= sgn; o.y ^= sgn; o.z ^= sgn; o.w ^= sgn;
-      __builtin_amdgcn_raw_buffer_store_b128(o, dst, voff, k * RNT * 16, kAuxStoreNT);
+      __builtin_amdgcn_raw_buffer_store_b128(o, dst, voff, k * NT * 16, kAuxStoreNT);
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (EXTRAS) {
@@ -488,7 +491,7 @@ __global__ __launch_bounds__(RNT) void resident_fused_kernel(RowArgs a, int32_t 
     // 8-12% faster (5.7 against 5.1-5.3 TB/s for the same 1R + 1W bytes).
 #pragma unroll
     for (int k = 0; k < SL; ++k) {
-      x[k] = __builtin_amdgcn_raw_buffer_load_b128(src, voff, k * RNT * 16, kAuxLoad);
+      x[k] = __builtin_amdgcn_raw_buffer_load_b128(src, voff, k * NT * 16, kAuxLoad);
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (EXTRAS) {
@@ -535,8 +538,8 @@ __device__ __forceinline__ bool bwd_zero_row(const BwdRow& q) {
 // lane (plus the head and tail elements with EXTRAS), is written back as one
 // burst of stores and the registers are refilled with the workgroup's next
 // row as one burst of loads.  The waves never synchronise.
-template <class Tag, int SL, bool EXTRAS>
-__global__ __launch_bounds__(RNT) void resident_bwd_kernel(RowArgs a, int32_t nvec) {
+template <class Tag, int NT, int SL, bool EXTRAS>
+__global__ __launch_bounds__(NT, kWavesPerSimd) void resident_bwd_kernel(RowArgs a, int32_t nvec) {
   using P = Pack16<Tag>;
   using S = typename Tag::S;
   constexpr int EPV = P::EPV;
@@ -569,7 +572,7 @@ __global__ __launch_bounds__(RNT) void resident_bwd_kernel(RowArgs a, int32_t nv
     const __amdgpu_buffer_rsrc_t src = z0 ? row_rsrc(logits, 0u) : row_rsrc(p0 + g0.head, g0.nbody * 16);
 #pragma unroll
     for (int k = 0; k < SL; ++k) {
-      x[k] = __builtin_amdgcn_raw_buffer_load_b128(src, voff, k * RNT * 16, kAuxLoad);
+      x[k] = __builtin_amdgcn_raw_buffer_load_b128(src, voff, k * NT * 16, kAuxLoad);
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (EXTRAS)
@@ -626,7 +629,7 @@ __global__ __launch_bounds__(RNT) void resident_bwd_kernel(RowArgs a, int32_t nv
       // rows went through the arithmetic below.
 #pragma unroll
       for (int k = 0; k < SL; ++k) {
-        __builtin_amdgcn_raw_buffer_store_b128(zv, dst, voff, k * RNT * 16, kAuxStoreNT);
+        __builtin_amdgcn_raw_buffer_store_b128(zv, dst, voff, k * NT * 16, kAuxStoreNT);
         __builtin_amdgcn_sched_barrier(0);
       }
       if constexpr (EXTRAS) {
@@ -641,13 +644,13 @@ __global__ __launch_bounds__(RNT) void resident_bwd_kernel(RowArgs a, int32_t nv
         P::unpack(x[k], v);
 #pragma unroll
         for (int i = 0; i < EPV; ++i) d[i] = exp2_hw(__builtin_fmaf(v[i] - lse, kLog2e, lg));
-        if (rel == k * RNT) {
+        if (rel == k * NT) {
 #pragma unroll
           for (int i = 0; i < EPV; ++i) d[i] = (i == ti) ? tgt_pre : d[i];
         }
         u32x4 o = P::pack(d);
         o.x ^= sgn; o.y ^= sgn; o.z ^= sgn; o.w ^= sgn;
-        __builtin_amdgcn_raw_buffer_store_b128(o, dst, voff, k * RNT * 16, kAuxStoreNT);
+        __builtin_amdgcn_raw_buffer_store_b128(o, dst, voff, k * NT * 16, kAuxStoreNT);
         __builtin_amdgcn_sched_barrier(0);
       }
       if constexpr (EXTRAS) {
@@ -660,7 +663,7 @@ __global__ __launch_bounds__(RNT) void resident_bwd_kernel(RowArgs a, int32_t nv
     }
 #pragma unroll
     for (int k = 0; k < SL; ++k) {
-      x[k] = __builtin_amdgcn_raw_buffer_load_b128(src, voff, k * RNT * 16, kAuxLoad);
+      x[k] = __builtin_amdgcn_raw_buffer_load_b128(src, voff, k * NT * 16, kAuxLoad);
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (EXTRAS)
@@ -683,65 +686,117 @@ int cu_count_of_current_device(int* n_out) {
   return RRL_OK;
 }
 
-// Variants by slab count; a row needs ceil(nvec / 1024) slabs.
-template <class Tag, bool EXTRAS>
-int launch_resident(const RowArgs& a, int32_t nvec, hipStream_t stream) {
-  const int need = (nvec + RNT - 1) / RNT;
-  int cus = 0;
-  if (int rc = cu_count_of_current_device(&cus)) return rc;
-  const int64_t rows = a.B * a.T;
-  const unsigned pgrid = (unsigned)((rows + 255) / 256 < 65536 ? (rows + 255) / 256 : 65536);
-  hipLaunchKernelGGL(pack_records_kernel, dim3(pgrid), dim3(256), 0, stream, a);
-  if (int rc = check_launch("pack_records_kernel")) return rc;
-  const unsigned grid = (unsigned)(rows < cus ? rows : cus);
-#define RRL_RESIDENT_CASE(SLV)                                                                \
-  if (need <= SLV) {                                                                          \
-    hipLaunchKernelGGL((resident_fused_kernel<Tag, SLV, EXTRAS>), dim3(grid), dim3(RNT), 0,   \
-                       stream, a, nvec);                                                     \
-    return check_launch("resident_fused_kernel");                                             \
-  }
-  RRL_RESIDENT_CASE(4)
-  RRL_RESIDENT_CASE(8)
-  RRL_RESIDENT_CASE(12)
-  RRL_RESIDENT_CASE(16)
-  RRL_RESIDENT_CASE(20)
-#undef RRL_RESIDENT_CASE
-  set_error("resident_fused_kernel: row too long");
-  return RRL_EINVAL;
+// Workgroups per CU by slab count: the waves per SIMD that the kernels'
+// registers allow (4 SL of slabs and about 45 more), in NT-lane workgroups.
+template <int NT, int SL>
+constexpr int wgs_per_cu() {
+  constexpr int waves = SL <= 4 ? 7 : SL <= 8 ? 6 : SL <= 12 ? 5 : kWavesPerSimd;
+  return waves * 256 / NT > 0 ? waves * 256 / NT : 1;
 }
 
+template <class Tag, int NT, int SL, bool EXTRAS>
+int launch_resident(int mode, const RowArgs& a, int32_t nvec, int cus, hipStream_t stream) {
+  static_assert(!EXTRAS || NT >= kHeadLanes + Pack16<Tag>::EPV, "lanes for the head and the tail");
+  const int64_t rows = a.B * a.T;
+  const int64_t wgs = (int64_t)cus * wgs_per_cu<NT, SL>();
+  const unsigned grid = (unsigned)(rows < wgs ? rows : wgs);
+  if (mode == 1) {
+    hipLaunchKernelGGL((resident_bwd_kernel<Tag, NT, SL, EXTRAS>), dim3(grid), dim3(NT), 0, stream,
+                       a, nvec);
+    return check_launch("resident_bwd_kernel");
+  }
+  hipLaunchKernelGGL((resident_fused_kernel<Tag, NT, SL, EXTRAS>), dim3(grid), dim3(NT), 0, stream,
+                     a, nvec);
+  return check_launch("resident_fused_kernel");
+}
+
+// Lanes per row by its length.  A row's time is its loads' latency, the
+// reduction and finish_row's serial chain, then its stores; a CU hides that
+// only behind other rows, so a short row takes a small workgroup and the CU
+// holds many (24 rows of 4096 bf16 entries with one wave each).  Measured
+// with 8192 rows, us for the fused pass (lanes per row 64 / 128 / 256 / 512 /
+// 1024; 1024 lanes and slabs in steps of four for every row before):
+//   V =  4096 bf16 (  512 vectors)   26 /  32 /  43 /  70 / 145
+//   V =  8192 bf16 ( 1024)           52 /  50 /  54 /  76 / 163
+//   V = 16000 bf16 ( 2000)            - / 102 /  99 / 102 / 173
+//   V = 24000 bf16 ( 3000)            - /   - / 150 / 143 / 221
+//   V = 32000 bf16 ( 4000)            - /   - / 204 / 190 / 218
+//   V = 50304 bf16 ( 6288)            - /   - /   - / 301 / 300
+//   V = 65536 bf16 ( 8192, 4096 rows) - /   - /   - / 186 / 204
+//   V = 20000 f32  ( 5000)            - /   - / 248 / 236 / 242
+//   V = 32000 f32  ( 8000, 4096 rows) - /   - /   - / 189 / 184
+// A slab past the row's end costs its issue slots though it moves nothing:
+// 4000 vectors took 228 us with 13 slabs of 512 lanes against 190 with 8, so
+// the slab counts step by at most a sixth from 5 up.  With fewer than 2048
+// rows one- and two-wave workgroups leave the chip idle, and 256 lanes finish
+// each row sooner (512 rows of V = 8192: 11.5 / 10.7 / 9.1 / 10.1 / 15.3 us).
 template <class Tag, bool EXTRAS>
-int launch_resident_bwd(const RowArgs& a, int32_t nvec, hipStream_t stream) {
-  const int need = (nvec + RNT - 1) / RNT;
+int launch_variant(int mode, const RowArgs& a, int32_t nvec, hipStream_t stream) {
   int cus = 0;
   if (int rc = cu_count_of_current_device(&cus)) return rc;
   const int64_t rows = a.B * a.T;
-  const unsigned grid = (unsigned)(rows < cus ? rows : cus);
-#define RRL_RESIDENT_CASE(SLV)                                                                \
-  if (need <= SLV) {                                                                          \
-    hipLaunchKernelGGL((resident_bwd_kernel<Tag, SLV, EXTRAS>), dim3(grid), dim3(RNT), 0,     \
-                       stream, a, nvec);                                                     \
-    return check_launch("resident_bwd_kernel");                                               \
+  if (mode == 2) {
+    const unsigned pgrid = (unsigned)((rows + 255) / 256 < 65536 ? (rows + 255) / 256 : 65536);
+    hipLaunchKernelGGL(pack_records_kernel, dim3(pgrid), dim3(256), 0, stream, a);
+    if (int rc = check_launch("pack_records_kernel")) return rc;
   }
-  RRL_RESIDENT_CASE(4)
-  RRL_RESIDENT_CASE(8)
-  RRL_RESIDENT_CASE(12)
-  RRL_RESIDENT_CASE(16)
-  RRL_RESIDENT_CASE(20)
+  const bool many = rows >= 2048;
+#define RRL_RESIDENT_CASE(NTV, SLV) \
+  if (nvec <= NTV * SLV) return launch_resident<Tag, NTV, SLV, EXTRAS>(mode, a, nvec, cus, stream);
+  if (many) {
+    if constexpr (EXTRAS) {
+      RRL_RESIDENT_CASE(128, 4)  // one wave has no lanes for the tail
+    } else {
+      RRL_RESIDENT_CASE(64, 2)
+      RRL_RESIDENT_CASE(64, 4)
+      RRL_RESIDENT_CASE(64, 6)
+      RRL_RESIDENT_CASE(64, 8)
+    }
+    RRL_RESIDENT_CASE(128, 5)
+    RRL_RESIDENT_CASE(128, 6)
+    RRL_RESIDENT_CASE(128, 8)
+    RRL_RESIDENT_CASE(128, 10)
+    RRL_RESIDENT_CASE(128, 12)
+  }
+  RRL_RESIDENT_CASE(256, 2)
+  RRL_RESIDENT_CASE(256, 4)
+  RRL_RESIDENT_CASE(256, 6)
+  RRL_RESIDENT_CASE(256, 7)
+  RRL_RESIDENT_CASE(256, 8)
+  RRL_RESIDENT_CASE(256, 10)
+  RRL_RESIDENT_CASE(256, 12)
+  RRL_RESIDENT_CASE(512, 7)
+  RRL_RESIDENT_CASE(512, 8)
+  RRL_RESIDENT_CASE(512, 10)
+  RRL_RESIDENT_CASE(512, 12)
+  RRL_RESIDENT_CASE(512, 13)
+  RRL_RESIDENT_CASE(512, 14)
+  if constexpr (Pack16<Tag>::EPV == 8) {
+    RRL_RESIDENT_CASE(512, 16)
+  } else {
+    RRL_RESIDENT_CASE(1024, 8)
+  }
+  RRL_RESIDENT_CASE(1024, 9)
+  RRL_RESIDENT_CASE(1024, 10)
+  RRL_RESIDENT_CASE(1024, 12)
+  RRL_RESIDENT_CASE(1024, 13)
+  RRL_RESIDENT_CASE(1024, 14)
+  RRL_RESIDENT_CASE(1024, 16)
+  RRL_RESIDENT_CASE(1024, 18)
+  RRL_RESIDENT_CASE(1024, 19)
+  RRL_RESIDENT_CASE(1024, 20)
 #undef RRL_RESIDENT_CASE
-  set_error("resident_bwd_kernel: row too long");
+  set_error("resident row kernel: row too long");
   return RRL_EINVAL;
 }
 
 template <class Tag>
 int dispatch_resident(int mode, bool extras, const RowArgs& a, int32_t nvec, hipStream_t st) {
-  if (mode == 1)
-    return extras ? launch_resident_bwd<Tag, true>(a, nvec, st)
-                  : launch_resident_bwd<Tag, false>(a, nvec, st);
-  return extras ? launch_resident<Tag, true>(a, nvec, st) : launch_resident<Tag, false>(a, nvec, st);
+  return extras ? launch_variant<Tag, true>(mode, a, nvec, st)
+                : launch_variant<Tag, false>(mode, a, nvec, st);
 }
 
-constexpr int64_t kMaxResidentVec = 20 * RNT;  // SL = 20 fits 128 VGPRs without spills
+constexpr int64_t kMaxResidentVec = kMaxSlabs * 1024;  // SL = 20 fits 128 VGPRs without spills
 
 }  // namespace
 
