@@ -24,6 +24,7 @@ LIB_PATH = PKG_DIR / LIB_NAME
 SOURCES = [
     "rrl_host.hip",
     "logprob.hip",
+    "logprob_fwd.hip",
     "logprob_resident.hip",
     "objectives.hip",
     "estimators.hip",

@@ -197,6 +197,7 @@ int validate_logits(const void* logits, int dt, int64_t B, int64_t T, int64_t V,
 
 int maybe_launch_resident(const RowArgs& a, int mode, int logits_dtype, hipStream_t stream,
                           bool* launched);
+int maybe_launch_fwd(const RowArgs& a, int logits_dtype, hipStream_t stream, bool* launched);
 
 }  // namespace rrl
 
@@ -219,6 +220,9 @@ extern "C" int rrl_logprob_fwd(const void* logits, int32_t logits_dtype, int64_t
   a.tgt = to_view(targets);
   a.logp = logp_out; a.logp_dt = logp_dtype; a.lse_out = lse_out;
   a.status = status;
+  bool launched = false;
+  rc = maybe_launch_fwd(a, logits_dtype, as_stream(stream), &launched);
+  if (rc || launched) return rc;
   return dispatch_row<MODE_FWD>(a, logits_dtype, as_stream(stream));
 }
 
@@ -240,6 +244,9 @@ extern "C" int rrl_logprob_fwd_masked(const void* logits, int32_t logits_dtype, 
   a.mask = to_view(mask);
   a.logp = logp_out; a.logp_dt = logp_dtype; a.lse_out = lse_out;
   a.status = status;
+  bool launched = false;
+  rc = maybe_launch_fwd(a, logits_dtype, as_stream(stream), &launched);
+  if (rc || launched) return rc;
   return dispatch_row<MODE_FWD>(a, logits_dtype, as_stream(stream));
 }
 

@@ -28,8 +28,7 @@
 #include <hip/hip_runtime.h>
 
 #include "policy_math.hpp"
-#include "row_common.hpp"
-#include "wave_common.hpp"
+#include "slab_common.hpp"
 
 namespace rrl {
 
@@ -37,137 +36,6 @@ namespace {
 
 constexpr int kMaxSlabs = 20;       // slabs per lane: 80 VGPRs of the 128 at 4 waves per SIMD
 constexpr int kWavesPerSimd = 4;
-
-// Element access of one 16-byte vector per tag: EPV elements, their float
-// values, the packed form written back (round to nearest even for 16-bit),
-// the sign bit of every element of a dword, and the single-element loads and
-// non-temporal stores of a row's unaligned head and tail.
-template <class Tag> struct Pack16;
-template <> struct Pack16<TagBF16> {
-  static constexpr int EPV = 8, LOG2_EPV = 3;
-  static constexpr uint32_t SGN2 = 0x80008000u, SGN1 = 0x8000u;
-  static __device__ __forceinline__ void unpack(const u32x4& u, float (&x)[8]) {
-    x[0] = __uint_as_float(u.x << 16); x[1] = __uint_as_float(u.x & 0xffff0000u);
-    x[2] = __uint_as_float(u.y << 16); x[3] = __uint_as_float(u.y & 0xffff0000u);
-    x[4] = __uint_as_float(u.z << 16); x[5] = __uint_as_float(u.z & 0xffff0000u);
-    x[6] = __uint_as_float(u.w << 16); x[7] = __uint_as_float(u.w & 0xffff0000u);
-  }
-  static __device__ __forceinline__ u32x4 pack(const float (&d)[8]) {
-    u32x4 o;
-    o.x = f32x2_to_bf16x2_bits(d[0], d[1]);
-    o.y = f32x2_to_bf16x2_bits(d[2], d[3]);
-    o.z = f32x2_to_bf16x2_bits(d[4], d[5]);
-    o.w = f32x2_to_bf16x2_bits(d[6], d[7]);
-    return o;
-  }
-  static __device__ __forceinline__ float one(uint32_t b) { return __uint_as_float(b << 16); }
-  static __device__ __forceinline__ uint32_t pack_one(float d) { return f32_to_bf16_bits(d); }
-  static __device__ __forceinline__ uint32_t load_one(__amdgpu_buffer_rsrc_t r, int off) {
-    return __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0);
-  }
-  static __device__ __forceinline__ void store_one(uint32_t b, __amdgpu_buffer_rsrc_t r, int off) {
-    __builtin_amdgcn_raw_buffer_store_b16((unsigned short)b, r, off, 0, kAuxStoreNT);
-  }
-};
-template <> struct Pack16<TagF16> {
-  static constexpr int EPV = 8, LOG2_EPV = 3;
-  static constexpr uint32_t SGN2 = 0x80008000u, SGN1 = 0x8000u;
-  static __device__ __forceinline__ void unpack(const u32x4& u, float (&x)[8]) {
-    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      x[2 * i] = f16_bits_to_f32((uint16_t)(w[i] & 0xffffu));
-      x[2 * i + 1] = f16_bits_to_f32((uint16_t)(w[i] >> 16));
-    }
-  }
-  static __device__ __forceinline__ u32x4 pack(const float (&d)[8]) {
-    uint32_t w[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      w[i] = (uint32_t)f32_to_f16_bits(d[2 * i]) | ((uint32_t)f32_to_f16_bits(d[2 * i + 1]) << 16);
-    u32x4 o;
-    o.x = w[0]; o.y = w[1]; o.z = w[2]; o.w = w[3];
-    return o;
-  }
-  static __device__ __forceinline__ float one(uint32_t b) {
-    return f16_bits_to_f32((uint16_t)(b & 0xffffu));
-  }
-  static __device__ __forceinline__ uint32_t pack_one(float d) { return f32_to_f16_bits(d); }
-  static __device__ __forceinline__ uint32_t load_one(__amdgpu_buffer_rsrc_t r, int off) {
-    return __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0);
-  }
-  static __device__ __forceinline__ void store_one(uint32_t b, __amdgpu_buffer_rsrc_t r, int off) {
-    __builtin_amdgcn_raw_buffer_store_b16((unsigned short)b, r, off, 0, kAuxStoreNT);
-  }
-};
-template <> struct Pack16<TagF32> {
-  static constexpr int EPV = 4, LOG2_EPV = 2;
-  static constexpr uint32_t SGN2 = 0x80000000u, SGN1 = 0x80000000u;
-  static __device__ __forceinline__ void unpack(const u32x4& u, float (&x)[4]) {
-    x[0] = __uint_as_float(u.x); x[1] = __uint_as_float(u.y);
-    x[2] = __uint_as_float(u.z); x[3] = __uint_as_float(u.w);
-  }
-  static __device__ __forceinline__ u32x4 pack(const float (&d)[4]) {
-    u32x4 o;
-    o.x = __float_as_uint(d[0]); o.y = __float_as_uint(d[1]);
-    o.z = __float_as_uint(d[2]); o.w = __float_as_uint(d[3]);
-    return o;
-  }
-  static __device__ __forceinline__ float one(uint32_t b) { return __uint_as_float(b); }
-  static __device__ __forceinline__ uint32_t pack_one(float d) { return __float_as_uint(d); }
-  static __device__ __forceinline__ uint32_t load_one(__amdgpu_buffer_rsrc_t r, int off) {
-    return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
-  }
-  static __device__ __forceinline__ void store_one(uint32_t b, __amdgpu_buffer_rsrc_t r, int off) {
-    __builtin_amdgcn_raw_buffer_store_b32(b, r, off, 0, kAuxStoreNT);
-  }
-};
-
-// A row as the resident kernels hold it: `head` single elements up to the
-// first 128-byte boundary, `nbody` 16-byte vectors (the register slabs), then
-// `tail` single elements.  The body starts on a 128-byte boundary so that
-// each wave's 1 KB run of vector stores covers whole cache lines: runs that
-// share a partly written line with the next wave's run cost up to 10% of the
-// write rate.  head < 128 / element size (at most 63) and tail <= EPV - 1,
-// so lanes 0-63 carry the head and lanes 64-71 the tail in one extra
-// register.  Without EXTRAS every row is 16-byte aligned with V % EPV == 0:
-// head = tail = 0 and nbody is the same for every row.
-constexpr uint32_t kBodyAlign = 128;
-constexpr int kHeadLanes = 64;
-
-struct RowGeo {
-  uint32_t head, nbody, tail;
-};
-
-template <class Tag, bool EXTRAS>
-__device__ __forceinline__ RowGeo row_geo(const void* row, uint32_t V, int32_t nvec) {
-  constexpr uint32_t EPV = Pack16<Tag>::EPV, ESZ = 16 / EPV;
-  RowGeo g;
-  if constexpr (EXTRAS) {
-    const uint32_t mis = (uint32_t)(reinterpret_cast<uintptr_t>(row) & (kBodyAlign - 1u));
-    uint32_t h = mis ? (kBodyAlign - mis) / ESZ : 0u;
-    h = h < V ? h : V;
-    const uint32_t rem = V - h;
-    g.head = h;
-    g.nbody = rem / EPV;
-    g.tail = rem - g.nbody * EPV;
-  } else {
-    g.head = 0;
-    g.nbody = (uint32_t)nvec;
-    g.tail = 0;
-  }
-  return g;
-}
-
-// Vocabulary index of the extra element lane `tid` carries, or -1.
-template <class Tag>
-__device__ __forceinline__ int32_t extra_index(const RowGeo& g, int tid) {
-  constexpr int EPV = Pack16<Tag>::EPV;
-  if (tid < kHeadLanes) return tid < (int)g.head ? tid : -1;
-  if (tid < kHeadLanes + EPV)
-    return tid - kHeadLanes < (int)g.tail ? (int)(g.head + g.nbody * EPV) + tid - kHeadLanes : -1;
-  return -1;
-}
 
 // Per-token records for the resident kernel (TokenRecord): the views' dtype
 // and stride handling happens here, once per token, so that the row loop reads
@@ -204,29 +72,6 @@ __device__ __forceinline__ TokenRecord load_record(const void* base, uint32_t r)
   rec.adv = __uint_as_float(q.z);
   rec.wcoef = __uint_as_float(q.w);
   return rec;
-}
-
-// s * exp(m - M) for the combine: exact s when m == M (also for M = -inf or
-// +inf, where m - M is NaN), 0 for m = -inf below a finite M.
-__device__ __forceinline__ float rescale(float s, float m, float M) {
-  return m == M ? s : s * exp2_hw((m - M) * kLog2e);
-}
-
-// Balanced max / sum of the EPV values of one vector.
-template <int N>
-__device__ __forceinline__ float vmax(const float (&v)[N]) {
-  if constexpr (N == 8)
-    return fmaxf(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])),
-                 fmaxf(fmaxf(v[4], v[5]), fmaxf(v[6], v[7])));
-  else
-    return fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
-}
-template <int N>
-__device__ __forceinline__ float vsum(const float (&e)[N]) {
-  if constexpr (N == 8)
-    return ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
-  else
-    return (e[0] + e[1]) + (e[2] + e[3]);
 }
 
 // exp2 exponent of -g * exp(x - lse) without the sign: x*log2e + (log2|g| -
@@ -333,53 +178,17 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
     const int ti = bt & (EPV - 1);
     const bool ex_tgt = EXTRAS && tgt_ok && ei == tgt;
 
-    // Sweep 1: per-lane online (max, sum exp) over the slabs.  The running max
-    // starts at -inf; `mg` (the max as an exponent offset) is kept finite so
-    // that slabs of -inf contribute exp(-inf) = 0 rather than
-    // exp(-inf + inf) = NaN, while NaN and +inf still poison the row as in
-    // log_softmax.  The target column is left out of the sum in the one lane
-    // and slab that hold it.
-    float m = -__builtin_huge_valf(), s = 0.0f;
-    auto fold = [&](int k) {
-      if (lane < (int)g.nbody - k * NT) {
-        float v[EPV];
-        P::unpack(x[k], v);
-        const float mn = fmaxf(m, vmax(v));
-        const float mg = fmaxf(mn, -__FLT_MAX__);
-        float e[EPV];
-#pragma unroll
-        for (int i = 0; i < EPV; ++i) e[i] = exp2_hw((v[i] - mg) * kLog2e);
-        float se = vsum(e);
-        if (rel == k * NT) {
-          float xv = v[0], so = 0.0f;
-#pragma unroll
-          for (int i = 0; i < EPV; ++i) {
-            xv = (i == ti) ? v[i] : xv;
-            so += (i == ti) ? 0.0f : e[i];
-          }
-          se = so;
-          sh_xt[buf] = xv;
-        }
-        s = __builtin_fmaf(s, exp2_hw((m - mg) * kLog2e), se);
-        m = mn;
-      }
-    };
-    float xt = 0.0f;
+    // Sweep 1: per-lane online (max, sum exp) over the slabs; the target
+    // column is left out of the sum in the one lane and slab that hold it.
+    LaneLse acc{-__builtin_huge_valf(), 0.0f};
+    float m = -__builtin_huge_valf(), s = 0.0f, xt = 0.0f;
     if (!skip) {  // uniform over the workgroup
 #pragma unroll
-      for (int k = 0; k < SL; ++k) fold(k);
+      for (int k = 0; k < SL; ++k)
+        if (lane < (int)g.nbody - k * NT)
+          fold_vector<Tag>(acc, x[k], rel == k * NT, ti, &sh_xt[buf]);
       if constexpr (EXTRAS) {
-        // As in a slab: the element joins the max, and the sum unless it is
-        // the target.
-        if (ei >= 0) {
-          const float v = P::one(xe);
-          const float mn = fmaxf(m, v);
-          const float mg = fmaxf(mn, -__FLT_MAX__);
-          const float ev = ex_tgt ? 0.0f : exp2_hw((v - mg) * kLog2e);
-          if (ex_tgt) sh_xt[buf] = v;
-          s = __builtin_fmaf(s, exp2_hw((m - mg) * kLog2e), ev);
-          m = mn;
-        }
+        if (ei >= 0) fold_one(acc, P::one(xe), ex_tgt, &sh_xt[buf]);
       }
       // No valid target: xt = -inf keeps the row's log-sum-exp finite (the
       // log-prob is set to NaN below).
@@ -387,8 +196,8 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
       // Workgroup combine, kept short: the next row's loads are not issued
       // until it ends.  Wave max, then the rescaled sum (one exponential per
       // lane), then the wave pairs through LDS with one barrier.
-      const float Mw = wave_max_dpp(m);
-      const float Sw = wave_sum_dpp(rescale(s, m, Mw));
+      const float Mw = wave_max_dpp(acc.m);
+      const float Sw = wave_sum_dpp(rescale(acc.s, acc.m, Mw));
       if ((tid & 63) == 0) {
         sh_m[buf][tid >> 6] = Mw;
         sh_s[buf][tid >> 6] = Sw;

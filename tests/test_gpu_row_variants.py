@@ -108,3 +108,33 @@ def test_odd_rows(device, dtype, V):
 
     print(f"[row-variants] {dtype} odd V={V}", flush=True)
     _run(*_rows(V, 2300, V, dtype, device))
+
+
+@pytest.mark.parametrize("dtype,V", [(torch.float32, v) for v in (81924, 81925, 151936, 163853)]
+                         + [(torch.bfloat16, v) for v in (163848, 163853, 256000)])
+@pytest.mark.parametrize("rows", [3, 300])
+def test_rows_past_the_registers(device, dtype, V, rows):
+    print(f"[row-variants] {dtype} V={V} rows={rows}", flush=True)
+    _run(*_rows(V + rows, rows, V, dtype, device))
+
+
+@pytest.mark.parametrize("nvec", [511, 512, 513, 768, 769, 3072, 3073])
+@pytest.mark.parametrize("rows", [255, 256])
+def test_forward_lengths(device, nvec, rows):
+    """The streaming forward's lane counts and depth remainders (four slabs of
+    128 to 1024 lanes), log-probs of a masked-out row 0."""
+
+    V = 8 * nvec + (nvec % 3)
+    print(f"[row-variants] forward V={V} rows={rows}", flush=True)
+    x, t, _ = _rows(nvec, rows, V, torch.float16, device)
+    x[0, 1, V // 2] = -float("inf")
+    lp, _ = _want(x, t, torch.ones_like(t, dtype=torch.float32))
+    got = R.gather_token_logprobs(x, t)
+    assert torch.allclose(got.double(), lp, rtol=1e-5, atol=1e-6)
+    live = torch.rand(1, rows, device=device) < 0.5
+    old, adv = lp.float() + 0.01, torch.ones_like(got)
+    live[0, :2] = True
+    a = R.fused_policy_loss(x, t, old, adv[:, 0], live, objective="gspo", clip_low=0.2)
+    b = R.fused_policy_loss(x, t, old, adv[:, 0], live, objective="gspo", clip_low=0.2,
+                            skip_masked_rows=True)
+    assert torch.equal(a.loss, b.loss)
