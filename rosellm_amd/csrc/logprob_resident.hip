@@ -268,10 +268,7 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
     // Every element goes through the same arithmetic, also for a zero-weight
     // row: there log2|g| = -inf and exp2(-inf) = 0 for every finite or -inf
     // logit (a +inf or NaN logit makes lse non-finite and the row NaN, as in
-    // log_softmax).  A uniform branch around the arithmetic with
-    // zero-initialised registers was tried with the store-then-load order
-    // below: on gfx950 it stored the zero initialiser instead of the computed
-    // first dword of odd slabs in waves 4-15, so it is not used.
+    // log_softmax), so zero-weight rows take no branch.
 #pragma unroll
     for (int k = 0; k < SL; ++k) {
       float d[EPV];
@@ -285,8 +282,7 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
       }
       u32x4 o = P::pack(d);
       o.x ^= sgn; o.y ^= sgn; o.z ^= sgn; o.w ^= sgn;
-      __builtin_amdgcn_raw_buffer_store_b128(o, dst, voff, k * NT * 16, kAuxStoreNT);
-      __builtin_amdgcn_sched_barrier(0);
+      store_b128_nt(o, dst, voff, k * NT * 16);
     }
     if constexpr (EXTRAS) {
       const float dv = ex_tgt ? tgt_pre : exp2_hw(exp_arg<Tag>(P::one(xe), q));
@@ -438,8 +434,7 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_bwd_kernel(RowArgs
       // rows went through the arithmetic below.
 #pragma unroll
       for (int k = 0; k < SL; ++k) {
-        __builtin_amdgcn_raw_buffer_store_b128(zv, dst, voff, k * NT * 16, kAuxStoreNT);
-        __builtin_amdgcn_sched_barrier(0);
+        store_b128_nt(zv, dst, voff, k * NT * 16);
       }
       if constexpr (EXTRAS) {
         P::store_one(zv.x, row_rsrc(drow, V32 * ESZ), extra_off(g));
@@ -459,8 +454,7 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_bwd_kernel(RowArgs
         }
         u32x4 o = P::pack(d);
         o.x ^= sgn; o.y ^= sgn; o.z ^= sgn; o.w ^= sgn;
-        __builtin_amdgcn_raw_buffer_store_b128(o, dst, voff, k * NT * 16, kAuxStoreNT);
-        __builtin_amdgcn_sched_barrier(0);
+        store_b128_nt(o, dst, voff, k * NT * 16);
       }
       if constexpr (EXTRAS) {
         const float dv =

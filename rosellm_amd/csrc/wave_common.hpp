@@ -33,6 +33,20 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const void* base, uin
 constexpr int kAuxLoad = 2;
 constexpr int kAuxStoreNT = 2;
 
+// Non-temporal 16-byte store at byte offset voff + soff.  The data registers
+// are read after the instruction issues: on gfx950 a VALU write to them needs
+// two wait states in between.  The compiler keeps that distance only where the
+// scalar offset is a constant, so the wait is written here (without it, the
+// first dword of some waves' vectors came out as the next instruction's
+// result: an LDS address computed into the register just stored).
+__device__ __forceinline__ void store_b128_nt(const u32x4& o, __amdgpu_buffer_rsrc_t dst, int voff,
+                                              int soff) {
+  __builtin_amdgcn_raw_buffer_store_b128(o, dst, voff, soff, kAuxStoreNT);
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_nop 1");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 // Butterfly steps inside a row of 16 lanes: DPP quad_perm [1,0,3,2] and
 // [2,3,0,1] exchange with lanes i^1 and i^2; once quads agree, the half-row
 // and row mirrors pair each half with the other (i^4, i^8 for a reduction).

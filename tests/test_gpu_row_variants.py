@@ -51,6 +51,12 @@ def _check(x, t, up, got_lp, got_dl):
     lp, dl = _want(x, t, up)
     assert torch.allclose(got_lp.double(), lp, rtol=1e-5, atol=1e-6)
     # every row's gradient carries |up| at its target at least once
+    if x.dtype == torch.float16:
+        # 11 significant bits, and below 2^-14 half a subnormal step (2^-25)
+        # per element whatever its size
+        d = (got_dl.double() - dl).abs()
+        assert bool((d <= dl.abs() * (2.0 ** -11 + 1e-5) + 2.0 ** -25).all())
+        return
     bar = 2.0 ** -8 + 1e-5 if x.dtype == torch.bfloat16 else 1e-5
     assert _row_err(got_dl, dl) <= bar
 
@@ -99,6 +105,15 @@ def test_long_rows(device, dtype, nvec, rows):
     V = nvec * (8 if dtype == torch.bfloat16 else 4)
     print(f"[row-variants] {dtype} V={V} rows={rows}", flush=True)
     _run(*_rows(nvec + rows, rows, V, dtype, device))
+
+
+@pytest.mark.parametrize("nvec", [512, 1024, 3072, 4096, 16032, 18992])
+def test_float16_every_element(device, nvec):
+    """Every element of float16 rows (their kernels write a store's registers
+    soonest after it)."""
+
+    print(f"[row-variants] f16 V={8 * nvec}", flush=True)
+    _run(*_rows(nvec, 2100 if nvec < 8000 else 530, 8 * nvec, torch.float16, device))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
