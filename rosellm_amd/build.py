@@ -25,6 +25,7 @@ SOURCES = [
     "rrl_host.hip",
     "logprob.hip",
     "logprob_fwd.hip",
+    "logprob_long.hip",
     "logprob_resident.hip",
     "objectives.hip",
     "estimators.hip",

@@ -27,10 +27,14 @@
 // dropped by the hardware range check.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "policy_math.hpp"
 #include "slab_common.hpp"
 
 namespace rrl {
+
+int launch_long_fused(const RowArgs& a, int logits_dtype, hipStream_t stream);
 
 namespace {
 
@@ -57,21 +61,6 @@ __global__ __launch_bounds__(256) void pack_records_kernel(RowArgs a) {
     r.wcoef = weight_coef(mask_weight<float>(c, a.mask, b, t), coef[b]);
     rec[i] = r;
   }
-}
-
-// The records are read-only for the resident kernel, so they can come through
-// the scalar data cache: a uniform load from the constant address space is a
-// single s_load_dwordx4, waited on with lgkmcnt and never behind the
-// vector-memory queue of slab loads and stores.
-__device__ __forceinline__ TokenRecord load_record(const void* base, uint32_t r) {
-  typedef __attribute__((address_space(4))) const u32x4 ConstWords;
-  const u32x4 q = reinterpret_cast<ConstWords*>(reinterpret_cast<uintptr_t>(base))[r];
-  TokenRecord rec;
-  rec.target = (int32_t)q.x;
-  rec.old = __uint_as_float(q.y);
-  rec.adv = __uint_as_float(q.z);
-  rec.wcoef = __uint_as_float(q.w);
-  return rec;
 }
 
 // exp2 exponent of -g * exp(x - lse) without the sign: x*log2e + (log2|g| -
@@ -343,14 +332,19 @@ __device__ __forceinline__ bool bwd_zero_row(const BwdRow& q) {
 // lane (plus the head and tail elements with EXTRAS), is written back as one
 // burst of stores and the registers are refilled with the workgroup's next
 // row as one burst of loads.  The waves never synchronise.
-template <class Tag, int NT, int SL, bool EXTRAS>
-__global__ __launch_bounds__(NT, kWavesPerSimd) void resident_bwd_kernel(RowArgs a, int32_t nvec) {
+//
+// PIECES: a row longer than one set of slabs goes through as `pieces` runs of
+// SL * NT vectors (there is nothing to reduce, so a piece is a row of its
+// own); the head belongs to the first run and the tail to the last.
+template <class Tag, int NT, int SL, bool EXTRAS, bool PIECES>
+__global__ __launch_bounds__(NT, kWavesPerSimd) void resident_bwd_kernel(RowArgs a, int32_t nvec,
+                                                                         uint32_t pieces) {
   using P = Pack16<Tag>;
   using S = typename Tag::S;
   constexpr int EPV = P::EPV;
   constexpr int ESZ = (int)sizeof(S);
   const int tid = threadIdx.x;
-  const uint32_t rows32 = (uint32_t)(a.B * a.T);
+  const uint32_t rows32 = (uint32_t)(a.B * a.T) * (PIECES ? pieces : 1u);
   const uint32_t T32 = (uint32_t)a.T;
   const uint32_t V32 = (uint32_t)a.V;
   const int voff = tid * 16;
@@ -359,29 +353,49 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_bwd_kernel(RowArgs
   uint32_t r = blockIdx.x;
   if (r >= rows32) return;
 
+  // Work item rr: row rr, or piece rr % pieces of row rr / pieces.
+  auto row_of = [&](uint32_t rr) { return PIECES ? rr / pieces : rr; };
+  auto piece_of = [&](uint32_t rr) { return PIECES ? rr - (rr / pieces) * pieces : 0u; };
   auto row_ptr = [&](uint32_t rr) {
-    const uint32_t bb = rr / T32, tt = rr - bb * T32;
+    const uint32_t row = row_of(rr);
+    const uint32_t bb = row / T32, tt = row - bb * T32;
     return logits + (int64_t)bb * a.ls_b + (int64_t)tt * a.ls_t;
   };
-  auto extra_off = [&](const RowGeo& g) {
-    const int32_t ei = extra_index<Tag>(g, tid);
+  // The item's first body vector and their number.
+  auto body_of = [&](const RowGeo& g, uint32_t rr, uint32_t& count) {
+    const uint32_t first = PIECES ? piece_of(rr) * (uint32_t)(SL * NT) : 0u;
+    const uint32_t left = g.nbody > first ? g.nbody - first : 0u;
+    count = PIECES && left > (uint32_t)(SL * NT) ? (uint32_t)(SL * NT) : left;
+    return first;
+  };
+  auto extra_of = [&](const RowGeo& g, uint32_t rr) {
+    if (PIECES && piece_of(rr) != (tid < kHeadLanes ? 0u : pieces - 1)) return -1;
+    return extra_index<Tag>(g, tid);
+  };
+  auto extra_off = [&](const RowGeo& g, uint32_t rr) {
+    const int32_t ei = extra_of(g, rr);
     return ei >= 0 ? ei * ESZ : (int)(V32 * ESZ);
   };
-  BwdRow next = load_bwd_row(a, r, T32);
+  auto body_rsrc = [&](const S* row, const RowGeo& g, uint32_t rr) {
+    uint32_t count;
+    const uint32_t first = body_of(g, rr, count);
+    return row_rsrc(row + g.head + first * EPV, count * 16);
+  };
+  BwdRow next = load_bwd_row(a, row_of(r), T32);
   u32x4 x[SL];
   uint32_t xe = 0;
   {
     const bool z0 = bwd_zero_row(next);
     const S* p0 = row_ptr(r);
     const RowGeo g0 = row_geo<Tag, EXTRAS>(p0, V32, nvec);
-    const __amdgpu_buffer_rsrc_t src = z0 ? row_rsrc(logits, 0u) : row_rsrc(p0 + g0.head, g0.nbody * 16);
+    const __amdgpu_buffer_rsrc_t src = z0 ? row_rsrc(logits, 0u) : body_rsrc(p0, g0, r);
 #pragma unroll
     for (int k = 0; k < SL; ++k) {
       x[k] = __builtin_amdgcn_raw_buffer_load_b128(src, voff, k * NT * 16, kAuxLoad);
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (EXTRAS)
-      xe = P::load_one(z0 ? row_rsrc(logits, 0u) : row_rsrc(p0, V32 * ESZ), extra_off(g0));
+      xe = P::load_one(z0 ? row_rsrc(logits, 0u) : row_rsrc(p0, V32 * ESZ), extra_off(g0, r));
   }
 
   // The zero rows' store data: a register quad of its own, opaque so that it
@@ -392,21 +406,24 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_bwd_kernel(RowArgs
   asm volatile("" : "+v"(zv));
 
   for (; r < rows32; r += gridDim.x) {
-    const uint32_t b = r / T32, t = r - b * T32;
+    const uint32_t row = row_of(r);
+    const uint32_t b = row / T32, t = row - b * T32;
     int lane = tid;
     asm volatile("" : "+v"(lane));
     const RowGeo g = row_geo<Tag, EXTRAS>(row_ptr(r), V32, nvec);
-    const int32_t ei = EXTRAS ? extra_index<Tag>(g, tid) : -1;
+    const int32_t ei = EXTRAS ? extra_of(g, r) : -1;
+    uint32_t count;
+    const uint32_t first = body_of(g, r, count);
     const BwdRow cur = next;
     const uint32_t rn = r + gridDim.x;
     const bool has_next = rn < rows32;
-    if (has_next) next = load_bwd_row(a, rn, T32);
+    if (has_next) next = load_bwd_row(a, row_of(rn), T32);
     // A target outside [0, V) has no column: every element takes the
     // exp(x - lse) term, as in the generic kernel.
     const bool tgt_ok = cur.target >= 0 && cur.target < a.V;
     const int32_t tgt = tgt_ok ? (int32_t)cur.target : 0;
-    const int32_t bt = tgt - (int32_t)g.head;
-    const bool in_body = tgt_ok && (!EXTRAS || (bt >= 0 && bt < (int32_t)(g.nbody * EPV)));
+    const int32_t bt = tgt - (int32_t)(g.head + first * EPV);
+    const bool in_body = tgt_ok && ((!EXTRAS && !PIECES) || (bt >= 0 && bt < (int32_t)(count * EPV)));
     const int rel = in_body ? (bt >> P::LOG2_EPV) - lane : -1;
     const int ti = bt & (EPV - 1);
     const bool ex_tgt = EXTRAS && tgt_ok && ei == tgt;
@@ -423,9 +440,9 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_bwd_kernel(RowArgs
     const S* pn = row_ptr(load_next ? rn : r);
     const RowGeo gn = row_geo<Tag, EXTRAS>(pn, V32, nvec);
     const __amdgpu_buffer_rsrc_t src =
-        load_next ? row_rsrc(pn + gn.head, gn.nbody * 16) : row_rsrc(logits, 0u);
+        load_next ? body_rsrc(pn, gn, rn) : row_rsrc(logits, 0u);
     const S* drow = dl + (int64_t)b * a.ds_b + (int64_t)t * a.ds_t;
-    const __amdgpu_buffer_rsrc_t dst = row_rsrc(drow + g.head, g.nbody * 16);
+    const __amdgpu_buffer_rsrc_t dst = row_rsrc(drow + g.head + first * EPV, count * 16);
     if (zero) {  // uniform over the workgroup
       // Stores only, with no dependence on the (never read) slabs: a run of
       // zero rows (a clipped GSPO sequence, masked prompt tokens) streams its
@@ -437,7 +454,7 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_bwd_kernel(RowArgs
         store_b128_nt(zv, dst, voff, k * NT * 16);
       }
       if constexpr (EXTRAS) {
-        P::store_one(zv.x, row_rsrc(drow, V32 * ESZ), extra_off(g));
+        P::store_one(zv.x, row_rsrc(drow, V32 * ESZ), extra_off(g, r));
         __builtin_amdgcn_sched_barrier(0);
       }
     } else {
@@ -460,7 +477,7 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_bwd_kernel(RowArgs
         const float dv =
             ex_tgt ? tgt_pre : exp2_hw(__builtin_fmaf(P::one(xe) - lse, kLog2e, lg));
         P::store_one(P::pack_one(dv) ^ (flip ? P::SGN1 : 0u), row_rsrc(drow, V32 * ESZ),
-                     extra_off(g));
+                     extra_off(g, r));
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -470,8 +487,17 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_bwd_kernel(RowArgs
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (EXTRAS)
-      xe = P::load_one(load_next ? row_rsrc(pn, V32 * ESZ) : row_rsrc(logits, 0u), extra_off(gn));
+      xe = P::load_one(load_next ? row_rsrc(pn, V32 * ESZ) : row_rsrc(logits, 0u), extra_off(gn, rn));
   }
+}
+
+}  // namespace
+
+int launch_pack_records(const RowArgs& a, hipStream_t stream) {
+  const int64_t rows = a.B * a.T;
+  const unsigned grid = (unsigned)((rows + 255) / 256 < 65536 ? (rows + 255) / 256 : 65536);
+  hipLaunchKernelGGL(pack_records_kernel, dim3(grid), dim3(256), 0, stream, a);
+  return check_launch("pack_records_kernel");
 }
 
 int cu_count_of_current_device(int* n_out) {
@@ -489,6 +515,8 @@ int cu_count_of_current_device(int* n_out) {
   return RRL_OK;
 }
 
+namespace {
+
 // Workgroups per CU by slab count: the waves per SIMD that the kernels'
 // registers allow (4 SL of slabs and about 45 more), in NT-lane workgroups.
 template <int NT, int SL>
@@ -504,8 +532,8 @@ int launch_resident(int mode, const RowArgs& a, int32_t nvec, int cus, hipStream
   const int64_t wgs = (int64_t)cus * wgs_per_cu<NT, SL>();
   const unsigned grid = (unsigned)(rows < wgs ? rows : wgs);
   if (mode == 1) {
-    hipLaunchKernelGGL((resident_bwd_kernel<Tag, NT, SL, EXTRAS>), dim3(grid), dim3(NT), 0, stream,
-                       a, nvec);
+    hipLaunchKernelGGL((resident_bwd_kernel<Tag, NT, SL, EXTRAS, false>), dim3(grid), dim3(NT), 0,
+                       stream, a, nvec, 1u);
     return check_launch("resident_bwd_kernel");
   }
   hipLaunchKernelGGL((resident_fused_kernel<Tag, NT, SL, EXTRAS>), dim3(grid), dim3(NT), 0, stream,
@@ -539,9 +567,7 @@ int launch_variant(int mode, const RowArgs& a, int32_t nvec, hipStream_t stream)
   if (int rc = cu_count_of_current_device(&cus)) return rc;
   const int64_t rows = a.B * a.T;
   if (mode == 2) {
-    const unsigned pgrid = (unsigned)((rows + 255) / 256 < 65536 ? (rows + 255) / 256 : 65536);
-    hipLaunchKernelGGL(pack_records_kernel, dim3(pgrid), dim3(256), 0, stream, a);
-    if (int rc = check_launch("pack_records_kernel")) return rc;
+    if (int rc = launch_pack_records(a, stream)) return rc;
   }
   const bool many = rows >= 2048;
 #define RRL_RESIDENT_CASE(NTV, SLV) \
@@ -593,13 +619,41 @@ int launch_variant(int mode, const RowArgs& a, int32_t nvec, hipStream_t stream)
   return RRL_EINVAL;
 }
 
+constexpr int64_t kMaxResidentVec = kMaxSlabs * 1024;  // SL = 20 fits 128 VGPRs without spills
+
+// rrl_logprob_bwd of longer rows, in the fewest pieces and the fewest slabs
+// that cover them.
+template <class Tag, bool EXTRAS>
+int launch_pieces(const RowArgs& a, int32_t nvec, hipStream_t stream) {
+  int cus = 0;
+  if (int rc = cu_count_of_current_device(&cus)) return rc;
+  const int64_t pieces = (nvec + kMaxResidentVec - 1) / kMaxResidentVec;
+  const int64_t items = a.B * a.T * pieces;
+  const unsigned grid = (unsigned)(items < cus ? items : cus);
+#define RRL_PIECES_CASE(SLV)                                                                   \
+  if (nvec <= pieces * SLV * 1024) {                                                           \
+    hipLaunchKernelGGL((resident_bwd_kernel<Tag, 1024, SLV, EXTRAS, true>), dim3(grid),        \
+                       dim3(1024), 0, stream, a, nvec, (uint32_t)pieces);                      \
+    return check_launch("resident_bwd_kernel");                                                \
+  }
+  RRL_PIECES_CASE(12)
+  RRL_PIECES_CASE(14)
+  RRL_PIECES_CASE(16)
+  RRL_PIECES_CASE(18)
+  RRL_PIECES_CASE(19)
+  RRL_PIECES_CASE(20)
+#undef RRL_PIECES_CASE
+  set_error("resident_bwd_kernel: row too long");
+  return RRL_EINVAL;
+}
+
 template <class Tag>
 int dispatch_resident(int mode, bool extras, const RowArgs& a, int32_t nvec, hipStream_t st) {
+  if (nvec > kMaxResidentVec)
+    return extras ? launch_pieces<Tag, true>(a, nvec, st) : launch_pieces<Tag, false>(a, nvec, st);
   return extras ? launch_variant<Tag, true>(mode, a, nvec, st)
                 : launch_variant<Tag, false>(mode, a, nvec, st);
 }
-
-constexpr int64_t kMaxResidentVec = kMaxSlabs * 1024;  // SL = 20 fits 128 VGPRs without spills
 
 }  // namespace
 
@@ -623,8 +677,11 @@ int maybe_launch_resident(const RowArgs& a, int mode, int logits_dtype, hipStrea
   if (a.dl_dt != logits_dtype || a.accumulate) return RRL_OK;
   const int64_t esz = logits_dtype == RRL_F32 ? 4 : 2;
   const int64_t epv = 16 / esz;
-  if (a.B * a.T == 0 || a.V / epv > kMaxResidentVec) return RRL_OK;
-  if (a.B * a.T >= ((int64_t)1 << 31) || a.T >= ((int64_t)1 << 31)) return RRL_OK;
+  const int64_t lim = (int64_t)1 << 31;
+  if (a.B * a.T == 0 || a.V * esz >= lim - (1 << 24)) return RRL_OK;
+  // Work items (rows, or pieces of long rows) are counted in 32 bits.
+  const int64_t pieces = (a.V / epv + kMaxResidentVec - 1) / kMaxResidentVec;
+  if (a.B * a.T * std::max<int64_t>(pieces, 1) >= lim || a.T >= lim) return RRL_OK;
   const auto al = [&](int64_t elems, int64_t n) { return ((elems * esz) % n) == 0; };
   const auto rows_aligned = [&](int64_t n) {
     return a.V % epv == 0 && (uintptr_t)a.logits % n == 0 && (uintptr_t)a.dl % n == 0 &&
@@ -647,6 +704,15 @@ int maybe_launch_resident(const RowArgs& a, int mode, int logits_dtype, hipStrea
     if ((uintptr_t)a.records % 16) return RRL_OK;
   }
   *launched = true;
+  // The long kernel's rows may start anywhere on both sides as long as the
+  // offsets agree; 16-byte aligned rows at other offsets stay generic.
+  if (mode == 2 && nvec > kMaxResidentVec) {
+    if (!same_offset) {
+      *launched = false;
+      return RRL_OK;
+    }
+    return launch_long_fused(a, logits_dtype, stream);
+  }
   switch (logits_dtype) {
     case RRL_BF16: return dispatch_resident<TagBF16>(mode, !aligned, a, nvec, stream);
     case RRL_F16: return dispatch_resident<TagF16>(mode, !aligned, a, nvec, stream);

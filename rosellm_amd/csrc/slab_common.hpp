@@ -211,5 +211,20 @@ __device__ __forceinline__ void fold_one(LaneLse& q, float v, bool is_target, fl
   q.m = mn;
 }
 
+// The records are read-only for the resident kernel, so they can come through
+// the scalar data cache: a uniform load from the constant address space is a
+// single s_load_dwordx4, waited on with lgkmcnt and never behind the
+// vector-memory queue of slab loads and stores.
+__device__ __forceinline__ TokenRecord load_record(const void* base, uint32_t r) {
+  typedef __attribute__((address_space(4))) const u32x4 ConstWords;
+  const u32x4 q = reinterpret_cast<ConstWords*>(reinterpret_cast<uintptr_t>(base))[r];
+  TokenRecord rec;
+  rec.target = (int32_t)q.x;
+  rec.old = __uint_as_float(q.y);
+  rec.adv = __uint_as_float(q.z);
+  rec.wcoef = __uint_as_float(q.w);
+  return rec;
+}
+
 }  // namespace
 }  // namespace rrl
