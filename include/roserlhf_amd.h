@@ -71,10 +71,9 @@ enum rrl_flag {
   RRL_FLAG_TARGET_RANGE = 4,     /* target id outside [0, V)              (gather, losses.py:36) */
   RRL_FLAG_INVALID_TURN = 8,     /* unmasked token with invalid turn id   (advantages.py:284-286) */
   RRL_FLAG_FAST_RANGE = 16,      /* rrl_fused_logprob_policy's 16-bit register-resident kernel met a
-                                    row with finite |log-sum-exp| > 2e38, outside its exponent range;
-                                    that call's outputs are undefined: rerun it with
-                                    RRL_POLICY_GENERIC set, or queue a rerun with
-                                    RRL_POLICY_RERUN_FAST_RANGE (no reference counterpart) */
+                                    row with finite |log-sum-exp| > 2e38.  Its outputs are the exact
+                                    ones; callers that refuse such logits read it (no reference
+                                    counterpart) */
   RRL_FLAG_BAD_PROBS = 32,       /* rrl_sample_logprobs: a row holds NaN or +inf logits (torch.multinomial
                                     rejects such probabilities, roseinfer/engine.py:1155,1169) */
   RRL_FLAG_LM_RANGE = 64         /* rrl_lm_head_fwd without mref_in: a token's logits rose more than 64
@@ -92,12 +91,14 @@ enum rrl_policy_flag {
                                  lse as 0 (equal to the reference for finite logits, where such a
                                  row contributes exactly 0; no reference counterpart) */
   RRL_POLICY_SUM = 4,         /* RRL_OBJ_NLL: reduction "sum" instead of "mean" */
-  RRL_POLICY_RERUN_FAST_RANGE = 8 /* rrl_fused_logprob_policy: launch the generic row kernel as a
+  RRL_POLICY_RERUN_FAST_RANGE = 8, /* rrl_fused_logprob_policy: launch the generic row kernel as a
                                  conditional rerun of the call just made with the same arguments
                                  on the same stream and status word (status required): its
                                  workgroups return at once unless the status word holds
                                  RRL_FLAG_FAST_RANGE, so a caller need not read the status between
                                  the two launches (no reference counterpart) */
+  RRL_POLICY_RECORDS_READY = 16 /* rrl_fused_logprob_policy: rrl_policy_prepare has packed the
+                                 records (no reference counterpart) */
 };
 
 /* Policy objectives (losses.py). */
@@ -216,6 +217,27 @@ RRL_API int rrl_policy_bwd(const rrl_policy_params* params, int64_t B, int64_t T
                    const void* workspace, const void* grad_scalars, const void* grad_seq,
                    void* grad_cur, void* stream);
 
+/* Destinations (rrl_policy_forward) or upstream gradients (rrl_policy_backward)
+ * of the four scalars above and of the loss (slot 4, minus slot 0): one element
+ * each, of dtype[k]; a null ptr means not wanted, or no gradient. */
+typedef struct rrl_scalars {
+  void* ptr[5];
+  int32_t dtype[5];
+} rrl_scalars;
+
+/* rrl_policy_fwd with every scalar written to a destination of its own (one
+ * launch for the caller's copies, conversions and negation), and
+ * rrl_policy_bwd reading its upstream gradients where autograd left them.
+ * status: as rrl_policy_prepare's below, or NULL. */
+RRL_API int rrl_policy_forward(const rrl_policy_params* params, int64_t B, int64_t T, rrl_view cur,
+                       rrl_view old, rrl_view adv, rrl_view mask, int32_t acc_dtype,
+                       void* workspace, const rrl_scalars* out, void* seq_out,
+                       uint8_t* trusted_out, int32_t* status, void* stream);
+RRL_API int rrl_policy_backward(const rrl_policy_params* params, int64_t B, int64_t T,
+                       rrl_view cur, rrl_view old, rrl_view adv, rrl_view mask,
+                       int32_t acc_dtype, const void* workspace, const rrl_scalars* grads,
+                       const void* grad_seq, void* grad_cur, void* stream);
+
 /* ---- single pass: log-prob + token-local objective gradient --------------
  * For PPO, SAO, SAPO and NLL, d loss / d logp is token-local once the mask
  * denominators are known, so one sweep over each logits row produces logp,
@@ -226,8 +248,7 @@ RRL_API int rrl_policy_bwd(const rrl_policy_params* params, int64_t B, int64_t T
  * records: caller workspace of rrl_fused_records_bytes(B, T) bytes, where the
  * register-resident path (16-bit and float32 logits, V <= 163840 16-bit or
  * 81920 float32 entries) packs each token's target, old log-prob, advantage
- * and mask weight * row_coef (16 bytes per token) for one scalar load per
- * row. */
+ * and mask weight (16 bytes per token) for one scalar load per row. */
 RRL_API int rrl_policy_row_coef(const rrl_policy_params* params, int64_t B, int64_t T,
                         rrl_view mask, int32_t acc_dtype, void* row_coef,
                         void* workspace, int32_t* status, void* stream);
@@ -243,6 +264,26 @@ RRL_API size_t rrl_fused_records_bytes(int64_t B, int64_t T);
  * replaces no reference function of its own. */
 RRL_API int rrl_check_targets(const rrl_policy_params* params, int64_t B, int64_t T, int64_t V,
                       rrl_view target, int32_t* status, void* stream);
+
+/* rrl_policy_row_coef, rrl_check_targets and the packing of the records in two
+ * launches.  The data errors (EMPTY_MASK, EMPTY_ROW, TARGET_RANGE) are stored,
+ * not or-ed, into *status by the last launch, so the word needs no clearing and
+ * may be host memory that the GPU can write (hipHostMalloc): the caller records
+ * an event behind this call, queues the sweep and everything after it, and
+ * reads the word once the event has passed.  For GSPO and GSPO-token, which
+ * have no row coefficients, row_coef and records are NULL and the call is the
+ * check alone.  records may be NULL (float64 logits); with records, pass RRL_POLICY_RECORDS_READY in the sweep's
+ * params->flags.  workspace: rrl_policy_workspace_bytes. */
+RRL_API int rrl_policy_prepare(const rrl_policy_params* params, int64_t B, int64_t T, int64_t V,
+                       rrl_view target, rrl_view old, rrl_view adv, rrl_view mask,
+                       int32_t acc_dtype, void* row_coef, void* records, void* workspace,
+                       int32_t* status, void* stream);
+
+/* rrl_check_targets with the result stored into *status as above.  workspace:
+ * rrl_targets_workspace_bytes() bytes. */
+RRL_API size_t rrl_targets_workspace_bytes(void);
+RRL_API int rrl_targets_status(const rrl_policy_params* params, int64_t B, int64_t T, int64_t V,
+                       rrl_view target, void* workspace, int32_t* status, void* stream);
 
 RRL_API int rrl_fused_logprob_policy(const rrl_policy_params* params, const void* logits,
                              int32_t logits_dtype, int64_t B, int64_t T, int64_t V,

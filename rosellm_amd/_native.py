@@ -47,6 +47,7 @@ POLICY_GENERIC = 1
 POLICY_SKIP_MASKED = 2
 POLICY_SUM = 4
 POLICY_RERUN_FAST_RANGE = 8
+POLICY_RECORDS_READY = 16
 
 # rrl_objective
 OBJ_PPO, OBJ_SAO, OBJ_GSPO, OBJ_GSPO_TOKEN, OBJ_SAPO, OBJ_NLL = range(6)
@@ -77,12 +78,17 @@ class RrlPolicyParams(ctypes.Structure):
     ]
 
 
+class RrlScalars(ctypes.Structure):
+    _fields_ = [("ptr", ctypes.c_void_p * 5), ("dtype", ctypes.c_int32 * 5)]
+
+
 _P = ctypes.c_void_p
 _I32 = ctypes.c_int32
 _I64 = ctypes.c_int64
 _D = ctypes.c_double
 _V = RrlView
 _PP = ctypes.POINTER(RrlPolicyParams)
+_PS = ctypes.POINTER(RrlScalars)
 
 # name -> (restype, argtypes); mirrors include/roserlhf_amd.h
 SIGNATURES = {
@@ -95,6 +101,11 @@ SIGNATURES = {
     "rrl_policy_workspace_bytes": (ctypes.c_size_t, [_I64, _I32]),
     "rrl_policy_fwd": (ctypes.c_int, [_PP, _I64, _I64, _V, _V, _V, _V, _I32, _P, _P, _P, _P, _P, _P]),
     "rrl_policy_bwd": (ctypes.c_int, [_PP, _I64, _I64, _V, _V, _V, _V, _I32, _P, _P, _P, _P, _P]),
+    "rrl_policy_forward": (ctypes.c_int, [_PP, _I64, _I64, _V, _V, _V, _V, _I32, _P, _PS, _P, _P, _P, _P]),
+    "rrl_policy_backward": (ctypes.c_int, [_PP, _I64, _I64, _V, _V, _V, _V, _I32, _P, _PS, _P, _P, _P]),
+    "rrl_policy_prepare": (ctypes.c_int, [_PP, _I64, _I64, _I64, _V, _V, _V, _V, _I32, _P, _P, _P, _P, _P]),
+    "rrl_targets_workspace_bytes": (ctypes.c_size_t, []),
+    "rrl_targets_status": (ctypes.c_int, [_PP, _I64, _I64, _I64, _V, _P, _P, _P]),
     "rrl_policy_row_coef": (ctypes.c_int, [_PP, _I64, _I64, _V, _I32, _P, _P, _P, _P]),
     "rrl_fused_records_bytes": (ctypes.c_size_t, [_I64, _I64]),
     "rrl_check_targets": (ctypes.c_int, [_PP, _I64, _I64, _I64, _V, _P, _P]),
@@ -349,3 +360,48 @@ def new_status(device: torch.device) -> torch.Tensor:
 
 def read_status(status: torch.Tensor) -> int:
     return int(status.item())
+
+
+class HostStatus:
+    """A status word in host memory that a kernel stores (rrl_policy_prepare,
+    rrl_targets_status, rrl_policy_forward) and the host reads without waiting
+    for anything queued behind that kernel: ``record()`` marks the place on the
+    current stream, ``read()`` waits for the mark alone.  As a context manager
+    it waits on the way out, so the word outlives its writer on every path."""
+
+    __slots__ = ("_word", "_event")
+
+    def __init__(self):
+        self._word = torch.empty(1, dtype=torch.int32, pin_memory=True)
+        self._event = None
+
+    @property
+    def ptr(self) -> int:
+        return self._word.data_ptr()
+
+    def record(self, device: torch.device) -> None:
+        self._event = torch.cuda.Event()
+        self._event.record(torch.cuda.current_stream(device))
+
+    def read(self) -> int:
+        self._event.synchronize()
+        return self._word.item()
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        if self._event is not None:
+            self._event.synchronize()
+        return False
+
+
+def scalars(tensors: Sequence[Optional[torch.Tensor]]) -> RrlScalars:
+    """The five one-element operands of rrl_policy_forward / _backward."""
+
+    sc = RrlScalars()
+    for k, t in enumerate(tensors):
+        if t is not None:
+            sc.ptr[k] = t.data_ptr()
+            sc.dtype[k] = dtype_code(t.dtype)
+    return sc

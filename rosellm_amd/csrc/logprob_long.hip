@@ -20,7 +20,6 @@
 // wrote itself, so the one barrier is the reduction's.
 #include <hip/hip_runtime.h>
 
-#include "policy_math.hpp"
 #include "slab_common.hpp"
 
 namespace rrl {
@@ -94,11 +93,11 @@ __global__ __launch_bounds__(NT, 2) void long_fused_kernel(RowArgs a) {
     const int32_t ei = extra_index<Tag>(g, tid);
     return ei >= 0 ? ei * ESZ : (int)(V32 * ESZ);
   };
-  TokenRecord rec_next = load_record(a.records, r);
+  RowRecord rec_next = load_record(a, r, T32);
   u32x4 x[kRegs];
   uint32_t xe;
   {
-    const bool skip0 = skip_masked && rec_next.wcoef == 0.0f;
+    const bool skip0 = skip_masked && rec_next.wcoef() == 0.0f;
     const S* p0 = row_ptr(r);
     const RowGeo g0 = row_geo<Tag, true>(p0, V32, 0);
     const __amdgpu_buffer_rsrc_t src =
@@ -118,11 +117,11 @@ __global__ __launch_bounds__(NT, 2) void long_fused_kernel(RowArgs a) {
     const S* row = row_ptr(r);
     const RowGeo g = row_geo<Tag, true>(row, V32, 0);
     const int32_t ei = extra_index<Tag>(g, tid);
-    const TokenRecord rec = rec_next;
-    const bool skip = skip_masked && rec.wcoef == 0.0f;
+    const RowRecord rec = rec_next;
+    const bool skip = skip_masked && rec.wcoef() == 0.0f;
     const uint32_t rn = r + gridDim.x;
     const bool has_next = rn < rows32;
-    if (has_next) rec_next = load_record(a.records, rn);
+    if (has_next) rec_next = load_record(a, rn, T32);
     const int32_t tgt = rec.target;
     const bool tgt_ok = tgt >= 0;
     const int32_t bt = tgt - (int32_t)g.head;
@@ -191,7 +190,7 @@ __global__ __launch_bounds__(NT, 2) void long_fused_kernel(RowArgs a) {
     q.lse = skip ? 0.0f : fr.lse;
     const float logp = skip ? 0.0f : (tgt_ok ? fr.logp : __builtin_nanf(""));
     const float gr =
-        skip ? 0.0f : -(rec.wcoef * token_local_grad<float>(c, logp, rec.old, rec.adv));
+        skip ? 0.0f : -(rec.wcoef() * token_local_grad<float>(c, logp, rec.old, rec.adv));
     const float tgt_d = target_grad<float>(gr, logp, true, xt, q.lse);
     if (tid == 0) {
       store_as<float>(a.logp, a.logp_dt, r, logp);
@@ -250,7 +249,7 @@ __global__ __launch_bounds__(NT, 2) void long_fused_kernel(RowArgs a) {
         }
       }
     }
-    const bool load_next = has_next && !(skip_masked && rec_next.wcoef == 0.0f);
+    const bool load_next = has_next && !(skip_masked && rec_next.wcoef() == 0.0f);
     const S* pn = row_ptr(load_next ? rn : r);
     const RowGeo gn = row_geo<Tag, true>(pn, V32, 0);
     const __amdgpu_buffer_rsrc_t src =

@@ -29,7 +29,6 @@
 
 #include <algorithm>
 
-#include "policy_math.hpp"
 #include "slab_common.hpp"
 
 namespace rrl {
@@ -47,7 +46,6 @@ constexpr int kWavesPerSimd = 4;
 __global__ __launch_bounds__(256) void pack_records_kernel(RowArgs a) {
   const PolicyConsts<float> c = PolicyConsts<float>::make(a.pp);
   TokenRecord* rec = static_cast<TokenRecord*>(a.records);
-  const float* coef = static_cast<const float*>(a.row_coef);
   const int64_t n = a.B * a.T;
   for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
     const int64_t b = i / a.T, t = i - (i / a.T) * a.T;
@@ -58,24 +56,9 @@ __global__ __launch_bounds__(256) void pack_records_kernel(RowArgs a) {
     r.target = ok ? (int32_t)tgt : -1;
     r.old = a.old.get<float>(b, t);
     r.adv = a.adv.get<float>(b, t);
-    r.wcoef = weight_coef(mask_weight<float>(c, a.mask, b, t), coef[b]);
+    r.weight = mask_weight<float>(c, a.mask, b, t);
     rec[i] = r;
   }
-}
-
-// exp2 exponent of -g * exp(x - lse) without the sign: x*log2e + (log2|g| -
-// lse*log2e) for 16-bit logits (one FMA per element; |lse| > 2e38 is flagged
-// and rerun by the host), (x - lse)*log2e + log2|g| for float32 logits (a
-// subtract more, and exact for every finite lse).
-struct ExpArg {
-  float cg, lg, lse;
-};
-template <class Tag>
-__device__ __forceinline__ float exp_arg(float x, const ExpArg& q) {
-  if constexpr (Pack16<Tag>::EPV == 4)
-    return __builtin_fmaf(x - q.lse, kLog2e, q.lg);
-  else
-    return __builtin_fmaf(x, kLog2e, q.cg);
 }
 
 template <class Tag, int NT, int SL, bool EXTRAS>
@@ -120,11 +103,11 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
   // (their loads use a 0-byte descriptor: no memory traffic) and get zero
   // dlogits and log-prob 0.
   const bool skip_masked = (a.pp.flags & RRL_POLICY_SKIP_MASKED) != 0;
-  TokenRecord rec_next = load_record(a.records, r);
+  RowRecord rec_next = load_record(a, r, T32);
   u32x4 x[SL];
   uint32_t xe = 0;  // EXTRAS: the lane's head or tail element, as stored
   {
-    const bool skip0 = skip_masked && rec_next.wcoef == 0.0f;
+    const bool skip0 = skip_masked && rec_next.wcoef() == 0.0f;
     const S* p0 = row_ptr(r);
     const RowGeo g0 = row_geo<Tag, EXTRAS>(p0, V32, nvec);
     const __amdgpu_buffer_rsrc_t src = skip0 ? row_rsrc(logits, 0u) : row_rsrc(p0 + g0.head, g0.nbody * 16);
@@ -152,11 +135,11 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
     const RowGeo g = row_geo<Tag, EXTRAS>(row_ptr(r), V32, nvec);
     const int32_t ei = EXTRAS ? extra_index<Tag>(g, tid) : -1;
     // Per-row scalars: one scalar-cache load, issued a row ahead.
-    const TokenRecord rec = rec_next;
-    const bool skip = skip_masked && rec.wcoef == 0.0f;
+    const RowRecord rec = rec_next;
+    const bool skip = skip_masked && rec.wcoef() == 0.0f;
     const uint32_t rn = r + gridDim.x;
     const bool has_next = rn < rows32;
-    if (has_next) rec_next = load_record(a.records, rn);
+    if (has_next) rec_next = load_record(a, rn, T32);
     const int32_t tgt = rec.target;
     const bool tgt_ok = tgt >= 0;
     // Slab k of this lane holds the target iff rel == k * NT; a target in
@@ -211,7 +194,7 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
     }
     // Past the last row (or for a skipped next row) the descriptor covers 0
     // bytes: the refills return zeros without touching memory.
-    const bool skip_next = skip_masked && rec_next.wcoef == 0.0f;
+    const bool skip_next = skip_masked && rec_next.wcoef() == 0.0f;
     const bool load_next = has_next && !skip_next;
     const S* pn = row_ptr(load_next ? rn : r);
     const RowGeo gn = row_geo<Tag, EXTRAS>(pn, V32, nvec);
@@ -228,7 +211,7 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
     const float lse = skip ? 0.0f : fr.lse;
     const float logp = skip ? 0.0f : (tgt_ok ? fr.logp : __builtin_nanf(""));
     const float gr =
-        skip ? 0.0f : -(rec.wcoef * token_local_grad<float>(c, logp, rec.old, rec.adv));
+        skip ? 0.0f : -(rec.wcoef() * token_local_grad<float>(c, logp, rec.old, rec.adv));
     const float tgt_d = target_grad<float>(gr, logp, true, xt, lse);
     if (tid == 0) {
       store_as<float>(a.logp, a.logp_dt, r, logp);
@@ -238,19 +221,20 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
     // Sweep 2: dlogits, then refill the register slabs with the next row.
     const S* drow = dl + (int64_t)b * a.ds_b + (int64_t)t * a.ds_t;
     const __amdgpu_buffer_rsrc_t dst = row_rsrc(drow + g.head, g.nbody * 16);
-    // lse * log2e overflows for finite |lse| > 2.3e38 (logits near the 16-bit
-    // maximum): such a row is flagged and the host reruns the call on the
-    // generic kernel.  Non-finite lse needs no care: NaN propagates as in
-    // log_softmax.  Float32 logits use the x - lse form, which has no limit.
     if (EPV == 8 && tid == 0 && fabsf(lse) > 2e38f && fabsf(lse) != __builtin_huge_valf())
       raise_flag(a.status, RRL_FLAG_FAST_RANGE);
-    // -g * exp(x - lse) = -sign(g) * exp2(x*log2e + (log2|g| - lse*log2e)):
-    // one FMA and one v_exp_f32 per element; the sign is applied to the packed
-    // words with one XOR per dword.
-    ExpArg q;
-    q.lg = __log2f(fabsf(gr));
-    q.cg = q.lg - lse * kLog2e;
-    q.lse = lse;
+    // -g * exp(x - lse) = -sign(g) * exp2(x * log2e + (log2|g| - lse * log2e)):
+    // one FMA per 16-bit element (forming x - lse first costs 1-2% of the
+    // 151936-entry sweep), the difference first for float32, whose 1e-7 it
+    // keeps.  lse * log2e overflows past 2.3e38; logits there lie 1e36 apart,
+    // so e^(x - lse) is 1 or 0 and half the scale gives the same.  The sign is
+    // applied to the packed words with one XOR per dword.
+    const float lg = __log2f(fabsf(gr));
+    const float sc = EPV == 8 && fabsf(lse) > 2e38f ? 0.5f * kLog2e : kLog2e;
+    const float cg = lg - lse * sc;
+    auto expo = [&](float xv) {
+      return EPV == 8 ? __builtin_fmaf(xv, sc, cg) : __builtin_fmaf(xv - lse, kLog2e, lg);
+    };
     const bool flip = gr > 0.0f;
     const uint32_t sgn = flip ? P::SGN2 : 0u;
     const float tgt_pre = flip ? -tgt_d : tgt_d;  // the XOR restores tgt_d
@@ -264,7 +248,7 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
       float v[EPV];
       P::unpack(x[k], v);
 #pragma unroll
-      for (int i = 0; i < EPV; ++i) d[i] = exp2_hw(exp_arg<Tag>(v[i], q));
+      for (int i = 0; i < EPV; ++i) d[i] = exp2_hw(expo(v[i]));
       if (rel == k * NT) {
 #pragma unroll
         for (int i = 0; i < EPV; ++i) d[i] = (i == ti) ? tgt_pre : d[i];
@@ -274,7 +258,7 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
       store_b128_nt(o, dst, voff, k * NT * 16);
     }
     if constexpr (EXTRAS) {
-      const float dv = ex_tgt ? tgt_pre : exp2_hw(exp_arg<Tag>(P::one(xe), q));
+      const float dv = ex_tgt ? tgt_pre : exp2_hw(expo(P::one(xe)));
       P::store_one(P::pack_one(dv) ^ (flip ? P::SGN1 : 0u), row_rsrc(drow, V32 * ESZ),
                    extra_off(g));
       __builtin_amdgcn_sched_barrier(0);
@@ -494,6 +478,7 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_bwd_kernel(RowArgs
 }  // namespace
 
 int launch_pack_records(const RowArgs& a, hipStream_t stream) {
+  if (a.pp.flags & RRL_POLICY_RECORDS_READY) return RRL_OK;
   const int64_t rows = a.B * a.T;
   const unsigned grid = (unsigned)((rows + 255) / 256 < 65536 ? (rows + 255) / 256 : 65536);
   hipLaunchKernelGGL(pack_records_kernel, dim3(grid), dim3(256), 0, stream, a);

@@ -33,12 +33,12 @@ struct RowArgs {
 
 // One token's inputs to the single-pass kernel, packed for a single 16-byte
 // scalar load per row: target id (-1 when outside [0, V)), old log-prob,
-// advantage and mask weight * row coefficient.
+// advantage and mask weight.
 struct TokenRecord {
   int32_t target;
   float old;
   float adv;
-  float wcoef;
+  float weight;
 };
 
 __device__ __forceinline__ int dtype_size_dev(int dt) {

@@ -4,6 +4,7 @@
 // (logprob_resident.hip) and the streaming forward (logprob_fwd.hip).
 #pragma once
 
+#include "policy_math.hpp"
 #include "row_common.hpp"
 #include "wave_common.hpp"
 
@@ -211,18 +212,28 @@ __device__ __forceinline__ void fold_one(LaneLse& q, float v, bool is_target, fl
   q.m = mn;
 }
 
-// The records are read-only for the resident kernel, so they can come through
+// The records and row coefficients are read-only for the sweep, so they come through
 // the scalar data cache: a uniform load from the constant address space is a
 // single s_load_dwordx4, waited on with lgkmcnt and never behind the
 // vector-memory queue of slab loads and stores.
-__device__ __forceinline__ TokenRecord load_record(const void* base, uint32_t r) {
+struct RowRecord {
+  int32_t target;
+  float old, adv;
+  float weight, coef;
+  // Mask weight * row coefficient, formed where it is used: forming it where
+  // the record is requested would wait for the loads at the top of every row.
+  __device__ __forceinline__ float wcoef() const { return weight_coef(weight, coef); }
+};
+__device__ __forceinline__ RowRecord load_record(const RowArgs& a, uint32_t r, uint32_t T32) {
   typedef __attribute__((address_space(4))) const u32x4 ConstWords;
-  const u32x4 q = reinterpret_cast<ConstWords*>(reinterpret_cast<uintptr_t>(base))[r];
-  TokenRecord rec;
+  typedef __attribute__((address_space(4))) const float ConstFloat;
+  const u32x4 q = reinterpret_cast<ConstWords*>(reinterpret_cast<uintptr_t>(a.records))[r];
+  RowRecord rec;
   rec.target = (int32_t)q.x;
   rec.old = __uint_as_float(q.y);
   rec.adv = __uint_as_float(q.z);
-  rec.wcoef = __uint_as_float(q.w);
+  rec.weight = __uint_as_float(q.w);
+  rec.coef = reinterpret_cast<ConstFloat*>(reinterpret_cast<uintptr_t>(a.row_coef))[r / T32];
   return rec;
 }
 

@@ -38,6 +38,7 @@ log-probs are an ordinary differentiable tensor.
 
 from __future__ import annotations
 
+import ctypes
 from typing import Optional, Tuple
 
 import torch
@@ -449,28 +450,25 @@ class _ChunkedLinearPolicy(torch.autograd.Function):
             if not skip_masked:
                 _logprob_rows(h2, w, tflat, torch.nonzero(~live).reshape(-1), lse, logp, status,
                               row_block)
-        scal = torch.empty(nat.NSCALARS, dtype=acc, device=dev)
         trusted = torch.empty(N if kind == nat.OBJ_SAO else 0, dtype=torch.bool, device=dev)
+        outs = L._scalar_outputs(L._scalar_dtypes(kind, logp, old, adv), dev)
         lview = nat.RrlView(logp.data_ptr(), acc_code, T, 1)
-        nat.call("rrl_policy_fwd", pref, B, T, lview, ov, av, mv, acc_code, ws.data_ptr(),
-                 scal.data_ptr(), None, nat.ptr(trusted) if trusted.numel() else None,
-                 status.data_ptr(), stream)
-        L._raise_flags(nat.read_status(status) & ~nat.FLAG_FAST_RANGE, kind)
+        nat.call("rrl_policy_forward", pref, B, T, lview, ov, av, mv, acc_code, ws.data_ptr(),
+                 ctypes.byref(nat.scalars(outs)), None,
+                 nat.ptr(trusted) if trusted.numel() else None, None, stream)
 
         ctx.params = params
         ctx.grads = grads
         ctx.meta = (B, T, acc, hidden.shape, row_block)
         ctx.save_for_backward(h2, w, tflat, ok, ak, mk, lse, logp, ws)
         ctx.set_materialize_grads(False)
-        dts = L._scalar_dtypes(kind, logp, old, adv)
-        outs = [scal[k].to(dts[k], copy=True) for k in range(4)]
         logp_out = logp.view(hidden.shape[:-1])
         trusted_out = trusted.view(hidden.shape[:-1]) if kind == nat.OBJ_SAO else trusted
         if kind in (nat.OBJ_PPO, nat.OBJ_SAO):
             ctx.mark_non_differentiable(outs[2], logp_out, trusted_out)
         else:
             ctx.mark_non_differentiable(logp_out, trusted_out)
-        return outs[0], outs[1], outs[2], outs[3], logp_out, trusted_out
+        return (*outs, logp_out, trusted_out)
 
     @staticmethod
     def _sweep(params, h2, w, tflat, ok, ak, mk, coef, act, T, lse, logp, need_h, need_w,
@@ -516,7 +514,7 @@ class _ChunkedLinearPolicy(torch.autograd.Function):
         return grads.finish()
 
     @staticmethod
-    def backward(ctx, g0, g1, g2, g3, _glogp, _gtrusted):
+    def backward(ctx, g0, g1, g2, g3, gloss, _glogp, _gtrusted):
         need_h, need_w = ctx.needs_input_grad[3], ctx.needs_input_grad[4]
         nones = (None, None, None)
         if not (need_h or need_w):
@@ -531,8 +529,7 @@ class _ChunkedLinearPolicy(torch.autograd.Function):
             params.kind == nat.OBJ_SAPO and g2 is not None)
         if grads is not None and not extra:
             # the stored gradients are those of d(-objective) = d loss
-            scale = (-g0).reshape(1).to(acc) if g0 is not None else torch.zeros(
-                1, dtype=acc, device=dev)
+            scale = L._loss_scale(g0, gloss, acc, dev)
             dh, dw = grads
             out = []
             for t in (dh, dw):
@@ -547,17 +544,14 @@ class _ChunkedLinearPolicy(torch.autograd.Function):
                     dw if need_w else None, None, None, None, None)
         # General case: d loss / d logp from every differentiated output, then
         # the chunked backward over the rows it reaches.
-        gs = torch.zeros(nat.NSCALARS, dtype=acc, device=dev)
-        for k, g in enumerate((g0, g1, g2, g3)):
-            if g is not None:
-                gs[k] = g.to(acc)
         lview = nat.RrlView(logp.data_ptr(), nat.dtype_code(acc), T, 1)
         ov, _ = nat.rows_view(ok, B, T)
         av, _ = nat.rows_view(ak, B, T)
         mv, _ = nat.rows_view(mk, B, T)
         g = torch.empty(B * T, dtype=acc, device=dev)
-        nat.call("rrl_policy_bwd", L.ctypes_ref(params), B, T, lview, ov, av, mv,
-                 nat.dtype_code(acc), ws.data_ptr(), gs.data_ptr(), None, g.data_ptr(), stream)
+        nat.call("rrl_policy_backward", L.ctypes_ref(params), B, T, lview, ov, av, mv,
+                 nat.dtype_code(acc), ws.data_ptr(),
+                 ctypes.byref(nat.scalars((g0, g1, g2, g3, gloss))), None, g.data_ptr(), stream)
         ctx.grads = None
         dh, dw = _chunked_backward(h2, w, tflat, lse, logp, g, need_h, need_w, row_block)
         return (*nones, (dh.view(shape) if dh is not None else None), dw, None, None, None, None)
@@ -822,15 +816,15 @@ def fused_linear_policy_loss(
     if path == "tiles":
         logp = _LinearLogprobs.apply(ppo, hidden, weight, target_ids, mask,
                                      bool(skip_masked_rows))
-        obj, d1, d2, d3, _seq, trusted = L._objective(p, logp, old_logprobs, advantages, mask)
-        out = L._token_local_output(kind, obj, d1, d2, d3, trusted)
+        obj, d1, d2, d3, loss, _seq, trusted = L._objective(p, logp, old_logprobs, advantages, mask)
+        out = L._token_local_output(kind, obj, d1, d2, d3, loss, trusted)
         return (out, _cfg.as_reference_dtype(logp.detach(), hidden)) if return_logprobs else out
     prefix = hidden.shape[:-1]
     old_d = L._on_device(old_logprobs, hidden)
     adv_d = L._on_device(advantages, hidden)
-    obj, d1, d2, d3, logp, trusted = _ChunkedLinearPolicy.apply(
+    obj, d1, d2, d3, loss, logp, trusted = _ChunkedLinearPolicy.apply(
         p, (bool(skip_masked_rows), torch.is_grad_enabled()), int(row_block), hidden, weight,
         target_ids,
         old_d.expand(prefix), adv_d.expand(prefix), mask.expand(prefix))
-    out = L._token_local_output(kind, obj, d1, d2, d3, trusted)
+    out = L._token_local_output(kind, obj, d1, d2, d3, loss, trusted)
     return (out, _cfg.as_reference_dtype(logp, hidden)) if return_logprobs else out

@@ -108,42 +108,67 @@ def _raise_target_range() -> None:
     raise RuntimeError("index out of bounds: every target id must lie in [0, vocabulary)")
 
 
+# torch.gather's target rule: every id lies in [0, vocabulary)
+_GATHER = nat.RrlPolicyParams()
+_GSPO_CHECK = nat.RrlPolicyParams(kind=nat.OBJ_GSPO)
+
+
 class _TokenLogprobs(torch.autograd.Function):
     """log_softmax(logits)[target] per row; backward writes dlogits in one sweep.
 
     With ``skip_mask`` (same shape as the targets) a row whose mask is exactly
     0 is not read: its log-prob and log-sum-exp are 0 (for objectives that
     weight such a token's log-prob by its zero mask; its d loss / d logp is
-    then 0 and the backward writes its dlogits row as zeros unread)."""
+    then 0 and the backward writes its dlogits row as zeros unread).
+
+    ``rows_mask`` ([B, T] action mask of a GSPO objective that follows): its
+    rule, an action token in every row, is checked with the targets."""
 
     @staticmethod
-    def forward(ctx, logits: Tensor, target_ids: Tensor,
-                skip_mask: Optional[Tensor] = None) -> Tensor:
+    def forward(ctx, logits: Tensor, target_ids: Tensor, skip_mask: Optional[Tensor] = None,
+                rows_mask: Optional[Tensor] = None) -> Tensor:
         dev = nat.require_device(logits, target_ids)
         x, B, T, V, s_b, s_t = nat.logits_rows(logits)
         tview, tkeep = nat.rows_view(target_ids, B, T)
         acc = nat.acc_dtype(logits.dtype)
         logp = torch.empty(B * T, dtype=acc, device=dev)
         lse = torch.empty(B * T, dtype=acc, device=dev)
-        status = nat.new_status(dev)
-        if skip_mask is None:
-            nat.call(
-                "rrl_logprob_fwd", x.data_ptr(), nat.dtype_code(x.dtype), B, T, V, s_b, s_t,
-                tview, logp.data_ptr(), nat.dtype_code(acc), lse.data_ptr(), status.data_ptr(),
-                nat.stream_ptr(dev),
-            )
-        else:
-            mview, _mkeep = nat.rows_view(skip_mask, B, T)
-            nat.call(
-                "rrl_logprob_fwd_masked", x.data_ptr(), nat.dtype_code(x.dtype), B, T, V, s_b,
-                s_t, tview, mview, logp.data_ptr(), nat.dtype_code(acc), lse.data_ptr(),
-                status.data_ptr(), nat.stream_ptr(dev),
-            )
-        if B * T and nat.read_status(status) & nat.FLAG_TARGET_RANGE:
-            _raise_target_range()
-        # The backward forms the target column from logp (-g * expm1(logp)); a
-        # private copy keeps it independent of in-place edits to the output.
-        ctx.save_for_backward(x, tkeep, lse, logp.clone())
+        stream = nat.stream_ptr(dev)
+        with nat.HostStatus() as status:
+            # The data errors are found ahead of the sweep, so that the wait
+            # below is over before the sweep is.
+            if rows_mask is not None:
+                ws = torch.empty(nat.lib().rrl_policy_workspace_bytes(B, nat.F32),
+                                 dtype=torch.uint8, device=dev)
+                mv, _mk = nat.rows_view(rows_mask, B, T)
+                nat.call("rrl_policy_prepare", ctypes_ref(_GSPO_CHECK), B, T, V, tview,
+                         nat.NONE_VIEW, nat.NONE_VIEW, mv, nat.F32, None, None, ws.data_ptr(),
+                         status.ptr, stream)
+                status.record(dev)
+            elif B * T:
+                part = torch.empty(nat.lib().rrl_targets_workspace_bytes(), dtype=torch.uint8,
+                                   device=dev)
+                nat.call("rrl_targets_status", ctypes_ref(_GATHER), B, T, V, tview,
+                         part.data_ptr(), status.ptr, stream)
+                status.record(dev)
+            if skip_mask is None:
+                nat.call(
+                    "rrl_logprob_fwd", x.data_ptr(), nat.dtype_code(x.dtype), B, T, V, s_b, s_t,
+                    tview, logp.data_ptr(), nat.dtype_code(acc), lse.data_ptr(), None, stream,
+                )
+            else:
+                mview, _mkeep = nat.rows_view(skip_mask, B, T)
+                nat.call(
+                    "rrl_logprob_fwd_masked", x.data_ptr(), nat.dtype_code(x.dtype), B, T, V, s_b,
+                    s_t, tview, mview, logp.data_ptr(), nat.dtype_code(acc), lse.data_ptr(),
+                    None, stream,
+                )
+            if rows_mask is not None or B * T:
+                _raise_flags(status.read(), nat.OBJ_GSPO)
+        if ctx.needs_input_grad[0]:
+            # The backward forms the target column from logp (-g * expm1(logp)); a
+            # private copy keeps it independent of in-place edits to the output.
+            ctx.save_for_backward(x, tkeep, lse, logp.clone())
         ctx.meta = (B, T, V, s_b, s_t, tuple(logits.shape), logits.dtype)
         ctx.set_materialize_grads(False)
         return logp.view(logits.shape[:-1])
@@ -151,7 +176,7 @@ class _TokenLogprobs(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad: Optional[Tensor]):
         if grad is None or not ctx.needs_input_grad[0]:
-            return None, None, None
+            return None, None, None, None
         x, tkeep, lse, logp = ctx.saved_tensors
         B, T, V, s_b, s_t, shape, dtype = ctx.meta
         g = grad.reshape(-1).to(lse.dtype).contiguous()
@@ -162,7 +187,7 @@ class _TokenLogprobs(torch.autograd.Function):
             lse.data_ptr(), logp.data_ptr(), g.data_ptr(), dl.data_ptr(), nat.dtype_code(dtype),
             T * V, V, 0, nat.stream_ptr(x.device),
         )
-        return dl, None, None
+        return dl, None, None, None
 
 
 def gather_token_logprobs(logits: Tensor, target_ids: Tensor) -> Tensor:
@@ -270,41 +295,19 @@ def _raise_flags(flags: int, kind: int) -> None:
         raise ValueError("cannot reduce an empty mask")
 
 
-def _check_before_sweep(logits: Tensor, inplace: bool) -> bool:
-    """Whether the single-pass call reads its status before the sweep.
-
-    Every data error is known before the sweep runs: the row coefficients
-    flag empty masks and rrl_check_targets the targets.  The one host
-    synchronisation then waits for those small kernels only, and the host
-    runs ahead of the sweep.  A log-sum-exp beyond 2e38, which only
-    bfloat16's range allows (float16 stops at 65504), makes the
-    register-resident kernel flag FAST_RANGE instead; a conditional generic
-    launch queued behind it (_rerun_on_device) redoes the call on the GPU in
-    that case.  In place the logits are gone by then, so bfloat16 in place
-    reads the status after the sweep and raises.
-    """
-
-    return logits.dtype != torch.bfloat16 or not inplace
-
-
-def _rerun_on_device(logits: Tensor, inplace: bool) -> bool:
-    """Whether the single-pass call queues RRL_POLICY_RERUN_FAST_RANGE."""
-
-    return logits.dtype == torch.bfloat16 and not inplace
-
-
-def _rerun_params(params):
-    p = nat.RrlPolicyParams.from_buffer_copy(params)
-    p.flags |= nat.POLICY_RERUN_FAST_RANGE
-    return p
-
-
 def _scalar_dtypes(kind: int, cur: Tensor, old: Tensor, adv: Tensor) -> Tuple[torch.dtype, ...]:
     ratio = torch.promote_types(cur.dtype, old.dtype)
     obj = torch.promote_types(ratio, adv.dtype)
     if kind == nat.OBJ_SAPO:
         return obj, ratio, ratio, obj
     return obj, ratio, ratio, ratio
+
+
+def _scalar_outputs(dtypes: Tuple[torch.dtype, ...], dev: torch.device) -> Tuple[Tensor, ...]:
+    """The objective, its three diagnostics and the loss (minus the objective),
+    each a tensor of its own for rrl_policy_forward to write."""
+
+    return tuple(torch.empty((), dtype=d, device=dev) for d in (*dtypes, dtypes[0]))
 
 
 def _views(kind: int, cur: Tensor, old: Tensor, adv: Tensor, mask: Tensor):
@@ -324,74 +327,73 @@ class _PolicyObjective(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, params: nat.RrlPolicyParams, cur: Tensor, old: Tensor, adv: Tensor,
-                mask: Tensor):
+                mask: Tensor, checked: bool = False):
         kind = params.kind
         dev = nat.require_device(cur, old, adv, mask)
         B, T, views, keep = _views(kind, cur, old, adv, mask)
         acc = nat.acc_dtype(cur.dtype, old.dtype, adv.dtype)
         ws = torch.empty(nat.lib().rrl_policy_workspace_bytes(B, nat.dtype_code(acc)),
                          dtype=torch.uint8, device=dev)
-        scal = torch.empty(nat.NSCALARS, dtype=acc, device=dev)
+        outs = _scalar_outputs(_scalar_dtypes(kind, cur, old, adv), dev)
         seq = torch.empty(B if kind in (nat.OBJ_GSPO, nat.OBJ_GSPO_TOKEN) else 0, dtype=acc,
                           device=dev)
         trusted = torch.empty(B * T if kind == nat.OBJ_SAO else 0, dtype=torch.bool, device=dev)
-        status = nat.new_status(dev)
-        nat.call(
-            "rrl_policy_fwd", ctypes_ref(params), B, T, *views, nat.dtype_code(acc), ws.data_ptr(),
-            scal.data_ptr(), nat.ptr(seq) if seq.numel() else None,
-            nat.ptr(trusted) if trusted.numel() else None, status.data_ptr(), nat.stream_ptr(dev),
-        )
-        _raise_flags(nat.read_status(status), kind)
+        with nat.HostStatus() as status:
+            nat.call(
+                "rrl_policy_forward", ctypes_ref(params), B, T, *views, nat.dtype_code(acc),
+                ws.data_ptr(), ctypes.byref(nat.scalars(outs)), nat.ptr(seq) if seq.numel() else None,
+                nat.ptr(trusted) if trusted.numel() else None, None if checked else status.ptr,
+                nat.stream_ptr(dev),
+            )
+            if not checked:
+                status.record(dev)
+                _raise_flags(status.read(), kind)
         ctx.save_for_backward(*keep, ws)
         ctx.params = params
         ctx.meta = (B, T, acc, tuple(cur.shape), cur.dtype)
         ctx.set_materialize_grads(False)
-        dts = _scalar_dtypes(kind, cur, old, adv)
-        outs = [scal[k].to(dts[k], copy=True) for k in range(4)]
-        ratio_dt = torch.promote_types(cur.dtype, old.dtype)
-        seq_out = seq.to(ratio_dt, copy=True)
+        seq_out = seq.to(torch.promote_types(cur.dtype, old.dtype))
         trusted_out = trusted.view(cur.shape) if kind == nat.OBJ_SAO else trusted
         # clip / rejected fractions count tokens and carry no gradient
-        if kind in (nat.OBJ_PPO, nat.OBJ_SAO):
-            ctx.mark_non_differentiable(outs[2], trusted_out)
-        elif kind in (nat.OBJ_GSPO, nat.OBJ_GSPO_TOKEN):
-            ctx.mark_non_differentiable(outs[2], trusted_out)
-        else:
+        if kind == nat.OBJ_SAPO:
             ctx.mark_non_differentiable(trusted_out)
-        return outs[0], outs[1], outs[2], outs[3], seq_out, trusted_out
+        else:
+            ctx.mark_non_differentiable(outs[2], trusted_out)
+        return (*outs, seq_out, trusted_out)
 
     @staticmethod
-    def backward(ctx, g0, g1, g2, g3, gseq, _gtrusted):
+    def backward(ctx, g0, g1, g2, g3, gloss, gseq, _gtrusted):
         if not ctx.needs_input_grad[1]:
-            return None, None, None, None, None
+            return None, None, None, None, None, None
         ck, ok, ak, mk, ws = ctx.saved_tensors
         B, T, acc, shape, dtype = ctx.meta
         params = ctx.params
         kind = params.kind
         dev = ws.device
-        gs = torch.zeros(nat.NSCALARS, dtype=acc, device=dev)
-        for k, g in enumerate((g0, g1, g2, g3)):
-            if g is not None:
-                gs[k] = g.to(acc)
         gseq_t = None
         if gseq is not None and gseq.numel():
             gseq_t = gseq.reshape(-1).to(acc).contiguous()
         _, _, views, _ = _views(kind, ck, ok, ak, mk)
         grad = torch.empty(B * T, dtype=acc, device=dev)
         nat.call(
-            "rrl_policy_bwd", ctypes_ref(params), B, T, *views, nat.dtype_code(acc), ws.data_ptr(),
-            gs.data_ptr(), nat.ptr(gseq_t), grad.data_ptr(), nat.stream_ptr(dev),
+            "rrl_policy_backward", ctypes_ref(params), B, T, *views, nat.dtype_code(acc),
+            ws.data_ptr(), ctypes.byref(nat.scalars((g0, g1, g2, g3, gloss))), nat.ptr(gseq_t),
+            grad.data_ptr(), nat.stream_ptr(dev),
         )
-        return None, grad.view(shape).to(dtype), None, None, None
+        return None, grad.view(shape).to(dtype), None, None, None, None
 
 
 def ctypes_ref(params: nat.RrlPolicyParams):
     return ctypes.byref(params)
 
 
-def _objective(params: nat.RrlPolicyParams, cur: Tensor, old: Tensor, adv: Tensor, mask: Tensor):
+def _objective(params: nat.RrlPolicyParams, cur: Tensor, old: Tensor, adv: Tensor, mask: Tensor,
+               checked: bool = False):
+    """``checked``: the mask's rule has been checked already; the call then
+    makes no host synchronisation."""
+
     mask = _on_device(mask, cur)
-    return _PolicyObjective.apply(params, cur, old, adv, mask)
+    return _PolicyObjective.apply(params, cur, old, adv, mask, checked)
 
 
 def direct_double_sided_mask(ratios: Tensor, *, clip_low: float, clip_high: float) -> Tensor:
@@ -452,11 +454,11 @@ def sao_policy_loss(
 
     p = _params(nat.OBJ_SAO, clip_low=clip_low, clip_high=clip_high, max_log_ratio=max_log_ratio,
                 detach_ratio=detach_ratio, mask_is_weight=False)
-    obj, kl, rejected, ratio, _, trusted = _objective(
+    obj, kl, rejected, ratio, loss, _, trusted = _objective(
         p, current_logprobs, rollout_logprobs, advantages, action_mask
     )
     return SaoPolicyLossOutput(
-        loss=-obj,
+        loss=loss,
         objective=obj,
         approximate_kl=kl,
         rejected_fraction=rejected,
@@ -487,6 +489,20 @@ def _check_clip_range(clip_low: float, clip_high: float, max_log_ratio: float) -
         raise ValueError("max_log_ratio must exceed both clip-boundary log ratios")
 
 
+def _gspo_arguments_valid(kind, target_ids, old, adv, mask, clip) -> bool:
+    """Whether a GSPO call on log-probs of the targets' shape passes every check
+    that precedes its kernels."""
+
+    try:
+        _check_rank2("GSPO", target_ids)
+        _check_float(old, adv)
+        _check_clip_range(*clip)
+    except (ValueError, TypeError):
+        return False
+    want = target_ids.shape if kind == nat.OBJ_GSPO_TOKEN else target_ids.shape[:-1]
+    return old.shape == target_ids.shape == mask.shape and adv.shape == want
+
+
 def gspo_policy_loss(
     current_logprobs: Tensor,
     rollout_logprobs: Tensor,
@@ -500,6 +516,12 @@ def gspo_policy_loss(
     """GSPO sequence objective (losses.py:206-273): geometric-mean sequence
     ratios, clipped once per response, responses weighted equally."""
 
+    return _gspo(current_logprobs, rollout_logprobs, sequence_advantages, action_mask,
+                 clip_low, clip_high, max_log_ratio)
+
+
+def _gspo(current_logprobs, rollout_logprobs, sequence_advantages, action_mask, clip_low, clip_high,
+          max_log_ratio, checked=False) -> GspoPolicyLossOutput:
     _check_rank2("GSPO", current_logprobs)
     if not (current_logprobs.shape == rollout_logprobs.shape == action_mask.shape):
         raise ValueError("log-probability tensors and action_mask must match")
@@ -510,11 +532,11 @@ def gspo_policy_loss(
 
     p = _params(nat.OBJ_GSPO, clip_low=clip_low, clip_high=clip_high,
                 max_log_ratio=max_log_ratio, mask_is_weight=False)
-    obj, div, frac, mean_ratio, seq, _ = _objective(
-        p, current_logprobs, rollout_logprobs, sequence_advantages, action_mask
+    obj, div, frac, mean_ratio, loss, seq, _ = _objective(
+        p, current_logprobs, rollout_logprobs, sequence_advantages, action_mask, checked
     )
     return GspoPolicyLossOutput(
-        loss=-obj,
+        loss=loss,
         objective=obj,
         sequence_ratio_divergence=div,
         sequence_clip_fraction=frac,
@@ -537,6 +559,12 @@ def gspo_token_policy_loss(
     sequence ratio numerically while its gradient flows through that token's
     own log-prob."""
 
+    return _gspo_token(current_logprobs, rollout_logprobs, token_advantages, action_mask,
+                 clip_low, clip_high, max_log_ratio)
+
+
+def _gspo_token(current_logprobs, rollout_logprobs, token_advantages, action_mask, clip_low, clip_high,
+          max_log_ratio, checked=False) -> GspoPolicyLossOutput:
     _check_rank2("GSPO-token", current_logprobs)
     if not (
         current_logprobs.shape
@@ -550,11 +578,11 @@ def gspo_token_policy_loss(
 
     p = _params(nat.OBJ_GSPO_TOKEN, clip_low=clip_low, clip_high=clip_high,
                 max_log_ratio=max_log_ratio, mask_is_weight=False)
-    obj, div, frac, mean_ratio, seq, _ = _objective(
-        p, current_logprobs, rollout_logprobs, token_advantages, action_mask
+    obj, div, frac, mean_ratio, loss, seq, _ = _objective(
+        p, current_logprobs, rollout_logprobs, token_advantages, action_mask, checked
     )
     return GspoPolicyLossOutput(
-        loss=-obj,
+        loss=loss,
         objective=obj,
         sequence_ratio_divergence=div,
         sequence_clip_fraction=frac,
@@ -597,11 +625,11 @@ def sapo_policy_loss(
                 tau_positive, tau_negative, max_log_ratio)
     p = _params(nat.OBJ_SAPO, max_log_ratio=max_log_ratio, tau_positive=tau_positive,
                 tau_negative=tau_negative, mask_is_weight=False)
-    obj, kl, ratio, gate, _, _ = _objective(
+    obj, kl, ratio, gate, loss, _, _ = _objective(
         p, current_logprobs, rollout_logprobs, token_advantages, action_mask
     )
     return SapoPolicyLossOutput(
-        loss=-obj,
+        loss=loss,
         objective=obj,
         approximate_kl=kl,
         mean_ratio=ratio,
@@ -650,10 +678,10 @@ def clipped_policy_loss(
                                clip_high, max_log_ratio)
     p = _params(nat.OBJ_PPO, clip_low=clip_low, clip_high=clip_high,
                 max_log_ratio=max_log_ratio, mask_is_weight=True)
-    obj, kl, frac, ratio, _, _ = _objective(p, current_logprobs, old_logprobs, advantages,
-                                            action_mask)
+    obj, kl, frac, ratio, loss, _, _ = _objective(p, current_logprobs, old_logprobs, advantages,
+                                                  action_mask)
     return PolicyLossOutput(
-        loss=-obj,
+        loss=loss,
         objective=obj,
         approximate_kl=kl,
         clip_fraction=frac,
@@ -775,18 +803,91 @@ def _token_local_params(kind: int, prefix, old_logprobs: Tensor, advantages: Ten
     return p
 
 
-def _token_local_output(kind: int, obj: Tensor, d1: Tensor, d2: Tensor, d3: Tensor,
+def _token_local_output(kind: int, obj: Tensor, d1: Tensor, d2: Tensor, d3: Tensor, loss: Tensor,
                         trusted: Tensor):
     """The output record of the token-local objective ``kind``."""
 
     if kind == nat.OBJ_PPO:
-        return PolicyLossOutput(loss=-obj, objective=obj, approximate_kl=d1, clip_fraction=d2,
+        return PolicyLossOutput(loss=loss, objective=obj, approximate_kl=d1, clip_fraction=d2,
                                 mean_ratio=d3)
     if kind == nat.OBJ_SAO:
-        return SaoPolicyLossOutput(loss=-obj, objective=obj, approximate_kl=d1,
+        return SaoPolicyLossOutput(loss=loss, objective=obj, approximate_kl=d1,
                                    rejected_fraction=d2, mean_ratio=d3, trusted_mask=trusted)
-    return SapoPolicyLossOutput(loss=-obj, objective=obj, approximate_kl=d1, mean_ratio=d2,
+    return SapoPolicyLossOutput(loss=loss, objective=obj, approximate_kl=d1, mean_ratio=d2,
                                 mean_gradient_gate=d3)
+
+
+class _Sweep:
+    """One single-pass call over logits rows (rrl_fused_logprob_policy) with the
+    launches around it: rrl_policy_prepare (row coefficients, records, every
+    data error), the sweep, rrl_policy_forward (the scalars).
+
+    The host waits for the errors once.  Out of place it waits behind
+    everything queued: the wait ends when the prepare kernels do, and the sweep
+    is already next in line.  In place the errors are read before the sweep
+    overwrites the logits, except for bfloat16, whose log-sum-exp range
+    (FAST_RANGE) is known after it."""
+
+    def __init__(self, params, x, geom, tview, ov, av, mv, dev):
+        self.params, self.x, self.dev = params, x, dev
+        self.tview, self.ov, self.av, self.mv = tview, ov, av, mv
+        B, T, V, self.s_b, self.s_t = geom
+        self.B, self.T, self.V = B, T, V
+        self.acc = nat.acc_dtype(x.dtype)
+        self.acc_code = nat.dtype_code(self.acc)
+        lib = nat.lib()
+        # workspace | row coefficients | records, each part 256-byte aligned
+        sizes = [(n + 255) // 256 * 256 for n in (
+            lib.rrl_policy_workspace_bytes(B, self.acc_code), B * 8,
+            lib.rrl_fused_records_bytes(B, T))]
+        self.scratch = torch.empty(sum(sizes), dtype=torch.uint8, device=dev)
+        self.ws_ptr = self.scratch.data_ptr()
+        self.coef_ptr = self.ws_ptr + sizes[0]
+        self.rec_ptr = self.coef_ptr + sizes[1]
+        self.logp = torch.empty(B * T, dtype=self.acc, device=dev)
+        self.lse = torch.empty(B * T, dtype=self.acc, device=dev)
+
+    def run(self, dl_ptr: int, d_b: int, d_t: int, inplace: bool, outs, trusted, inplace_error):
+        """Launch everything; raises the call's data errors."""
+
+        B, T, V = self.B, self.T, self.V
+        stream = nat.stream_ptr(self.dev)
+        code = nat.dtype_code(self.x.dtype)
+        p = nat.RrlPolicyParams.from_buffer_copy(self.params)
+        p.flags |= nat.POLICY_RECORDS_READY
+        pref = ctypes_ref(p)
+        late = inplace and self.x.dtype == torch.bfloat16
+        sweep_status = nat.new_status(self.dev) if late else None
+        with nat.HostStatus() as status:
+            nat.call("rrl_policy_prepare", pref, B, T, V, self.tview, self.ov, self.av, self.mv,
+                     self.acc_code, self.coef_ptr, self.rec_ptr, self.ws_ptr, status.ptr, stream)
+            status.record(self.dev)
+            if inplace and not late:
+                _raise_flags(status.read(), p.kind)
+            nat.call("rrl_fused_logprob_policy", pref, self.x.data_ptr(), code, B, T, V, self.s_b,
+                     self.s_t, self.tview, self.ov, self.av, self.mv, self.coef_ptr,
+                     self.rec_ptr, self.logp.data_ptr(), self.lse.data_ptr(), dl_ptr, code, d_b,
+                     d_t, nat.ptr(sweep_status), stream)
+            lview = nat.RrlView(self.logp.data_ptr(), self.acc_code, T, 1)
+            nat.call("rrl_policy_forward", pref, B, T, lview, self.ov, self.av, self.mv,
+                     self.acc_code, self.ws_ptr, ctypes.byref(nat.scalars(outs)), None,
+                     nat.ptr(trusted), None, stream)
+            if late and nat.read_status(sweep_status) & nat.FLAG_FAST_RANGE:
+                raise RuntimeError(inplace_error)
+            if late or not inplace:
+                _raise_flags(status.read(), p.kind)
+
+
+def _loss_scale(g0: Optional[Tensor], gloss: Optional[Tensor], acc: torch.dtype,
+                dev: torch.device) -> Tensor:
+    """The upstream factor of gradients stored for d loss = 1, from the
+    gradients of the objective and of the loss."""
+
+    if g0 is None:
+        scale = gloss if gloss is not None else torch.zeros((), dtype=acc, device=dev)
+    else:
+        scale = -g0 if gloss is None else gloss - g0
+    return scale.reshape(1).to(acc)
 
 
 class _FusedPolicy(torch.autograd.Function):
@@ -809,61 +910,19 @@ class _FusedPolicy(torch.autograd.Function):
         ov, ok = nat.rows_view(old, B, T)
         av, ak = nat.rows_view(adv, B, T)
         mv, mk = nat.rows_view(mask, B, T)
-        acc = nat.acc_dtype(logits.dtype)
-        acc_code = nat.dtype_code(acc)
-        stream = nat.stream_ptr(dev)
-        ws = torch.empty(nat.lib().rrl_policy_workspace_bytes(B, acc_code), dtype=torch.uint8,
-                         device=dev)
-        coef = torch.empty(B, dtype=acc, device=dev)
-        records = torch.empty(nat.lib().rrl_fused_records_bytes(B, T), dtype=torch.uint8,
-                              device=dev)
-        logp = torch.empty(B * T, dtype=acc, device=dev)
-        lse = torch.empty(B * T, dtype=acc, device=dev)
+        sweep = _Sweep(params, x, (B, T, V, s_b, s_t), tview, ov, av, mv, dev)
+        acc = sweep.acc
         if inplace:
             dl, d_b, d_t = x, s_b, s_t
         else:
             dl = torch.empty((B, T, V), dtype=logits.dtype, device=dev)
             d_b, d_t = T * V, V
-        scal = torch.empty(nat.NSCALARS, dtype=acc, device=dev)
         trusted = torch.empty(B * T if kind == nat.OBJ_SAO else 0, dtype=torch.bool, device=dev)
-        lview = nat.RrlView(logp.data_ptr(), acc_code, T, 1)
-
-        early = _check_before_sweep(logits, inplace)
-        rerun = _rerun_on_device(logits, inplace)
-
-        def run(p):
-            status = nat.new_status(dev)
-            pref = ctypes_ref(p)
-            nat.call("rrl_policy_row_coef", pref, B, T, mv, acc_code, coef.data_ptr(),
-                     ws.data_ptr(), status.data_ptr(), stream)
-            if early:
-                nat.call("rrl_check_targets", pref, B, T, V, tview, status.data_ptr(), stream)
-                _raise_flags(nat.read_status(status), kind)
-            for q in (pref, ctypes_ref(_rerun_params(p))) if rerun else (pref,):
-                nat.call("rrl_fused_logprob_policy", q, x.data_ptr(), nat.dtype_code(x.dtype),
-                         B, T, V, s_b, s_t, tview, ov, av, mv, coef.data_ptr(),
-                         records.data_ptr(), logp.data_ptr(), lse.data_ptr(), dl.data_ptr(),
-                         nat.dtype_code(logits.dtype), d_b, d_t, status.data_ptr(), stream,
-                         timed=q is pref)
-            nat.call("rrl_policy_fwd", pref, B, T, lview, ov, av, mv, acc_code, ws.data_ptr(),
-                     scal.data_ptr(), None, nat.ptr(trusted) if trusted.numel() else None,
-                     status.data_ptr(), stream)
-            return 0 if early else nat.read_status(status)
-
-        flags = run(params)
-        if flags & nat.FLAG_FAST_RANGE:
-            # A row's log-sum-exp lies beyond the register-resident 16-bit kernel's exponent
-            # range (logits near the format's maximum): redo the call on the
-            # generic row kernel.
-            if inplace:
-                raise RuntimeError(
-                    "fused_policy_loss(inplace=True): logits beyond +-2e38 need the generic "
-                    "kernel, which cannot rerun over overwritten logits; call with inplace=False"
-                )
-            generic = nat.RrlPolicyParams.from_buffer_copy(params)
-            generic.flags |= nat.POLICY_GENERIC
-            flags = run(generic)
-        _raise_flags(flags, kind)
+        logp, lse, ws = sweep.logp, sweep.lse, sweep.scratch
+        outs = _scalar_outputs(_scalar_dtypes(kind, logp, old, adv), dev)
+        sweep.run(dl.data_ptr(), d_b, d_t, inplace, outs, trusted if trusted.numel() else None,
+                  "fused_policy_loss(inplace=True): logits beyond +-2e38 need the generic "
+                  "kernel, which cannot rerun over overwritten logits; call with inplace=False")
 
         ctx.params = params
         ctx.inplace = inplace
@@ -871,18 +930,16 @@ class _FusedPolicy(torch.autograd.Function):
         ctx.meta = (B, T, V, s_b, s_t, d_b, d_t, acc, tuple(logits.shape), logits.dtype)
         ctx.save_for_backward(x if not inplace else lse, tkeep, ok, ak, mk, lse, logp, ws)
         ctx.set_materialize_grads(False)
-        dts = _scalar_dtypes(kind, logp, old, adv)
-        outs = [scal[k].to(dts[k], copy=True) for k in range(4)]
         logp_out = logp.view(logits.shape[:-1])
         trusted_out = trusted.view(logits.shape[:-1]) if kind == nat.OBJ_SAO else trusted
         if kind in (nat.OBJ_PPO, nat.OBJ_SAO):
             ctx.mark_non_differentiable(outs[2], logp_out, trusted_out)
         else:
             ctx.mark_non_differentiable(logp_out, trusted_out)
-        return outs[0], outs[1], outs[2], outs[3], logp_out, trusted_out
+        return (*outs, logp_out, trusted_out)
 
     @staticmethod
-    def backward(ctx, g0, g1, g2, g3, _glogp, _gtrusted):
+    def backward(ctx, g0, g1, g2, g3, gloss, _glogp, _gtrusted):
         nones = (None, None)
         if not ctx.needs_input_grad[2]:
             return (*nones, None, None, None, None, None)
@@ -897,8 +954,7 @@ class _FusedPolicy(torch.autograd.Function):
             params.kind == nat.OBJ_SAPO and g2 is not None
         )
         if dl is not None and not extra:
-            scale = (-g0).reshape(1).to(acc) if g0 is not None else torch.zeros(1, dtype=acc,
-                                                                                 device=dev)
+            scale = _loss_scale(g0, gloss, acc, dev)
             nat.call("rrl_scale_rows", dl.data_ptr(), nat.dtype_code(dtype), B, T, V, d_b, d_t,
                      scale.data_ptr(), nat.dtype_code(acc), 1.0, stream)
             ctx.dl = None
@@ -910,18 +966,15 @@ class _FusedPolicy(torch.autograd.Function):
             )
         # General case: full d/d logp from every differentiated output, then
         # one backward sweep over the logits.
-        gs = torch.zeros(nat.NSCALARS, dtype=acc, device=dev)
-        for k, g in enumerate((g0, g1, g2, g3)):
-            if g is not None:
-                gs[k] = g.to(acc)
         lview = nat.RrlView(logp.data_ptr(), nat.dtype_code(acc), T, 1)
         ov, _ = nat.rows_view(ok, B, T)
         av, _ = nat.rows_view(ak, B, T)
         mv, _ = nat.rows_view(mk, B, T)
         g = torch.empty(B * T, dtype=acc, device=dev)
         pref = ctypes_ref(params)
-        nat.call("rrl_policy_bwd", pref, B, T, lview, ov, av, mv, nat.dtype_code(acc),
-                 ws.data_ptr(), gs.data_ptr(), None, g.data_ptr(), stream)
+        nat.call("rrl_policy_backward", pref, B, T, lview, ov, av, mv, nat.dtype_code(acc),
+                 ws.data_ptr(), ctypes.byref(nat.scalars((g0, g1, g2, g3, gloss))), None,
+                 g.data_ptr(), stream)
         out = dl if dl is not None else torch.empty((B, T, V), dtype=dtype, device=dev)
         tview, _ = nat.rows_view(tkeep, B, T)
         nat.call("rrl_logprob_bwd", x.data_ptr(), nat.dtype_code(x.dtype), B, T, V, s_b, s_t,
@@ -996,17 +1049,20 @@ def fused_policy_loss(
         # forward's log-sum-exp and writes rows with a zero gradient unread.
         # With skip_masked_rows the forward does not read tokens whose mask
         # is 0: they enter the sequence log-ratio only times their zero mask.
+        mask_dev = _on_device(action_mask, logits)
+        clip = (clip_low, clip_low if clip_high is None else clip_high, max_log_ratio)
+        # A valid call's mask is checked ahead of the forward sweep, and the
+        # objective then queues up behind it without a wait; any other call
+        # goes the objective's own way, with its errors in its order.
+        checked = _gspo_arguments_valid(kind, target_ids, old_logprobs, advantages, mask_dev, clip)
+        skip_mask = None
         if skip_masked_rows:
-            mask_dev = _on_device(action_mask, logits)
-            if mask_dev.shape != target_ids.shape:
-                mask_dev = mask_dev.expand(target_ids.shape)
-            logp = _TokenLogprobs.apply(logits, target_ids, mask_dev)
-        else:
-            logp = gather_token_logprobs(logits, target_ids)
-        fn = gspo_policy_loss if kind == nat.OBJ_GSPO else gspo_token_policy_loss
-        out = fn(logp, old_logprobs, advantages, action_mask, clip_low=clip_low,
-                 clip_high=clip_low if clip_high is None else clip_high,
-                 max_log_ratio=max_log_ratio)
+            skip_mask = mask_dev.expand(target_ids.shape)
+        logp = _TokenLogprobs.apply(logits, target_ids, skip_mask, mask_dev if checked else None)
+        if not skip_masked_rows:
+            logp = _cfg.as_reference_dtype(logp, logits)
+        fn = _gspo if kind == nat.OBJ_GSPO else _gspo_token
+        out = fn(logp, old_logprobs, advantages, mask_dev, *clip, checked)
         return (out, _cfg.as_reference_dtype(logp.detach(), logits)) if return_logprobs else out
 
     p = _token_local_params(kind, logits.shape[:-1], old_logprobs, advantages, action_mask,
@@ -1016,8 +1072,8 @@ def fused_policy_loss(
     if skip_masked_rows:
         p.flags |= nat.POLICY_SKIP_MASKED
     mask = _on_device(action_mask, logits)
-    obj, d1, d2, d3, logp, trusted = _FusedPolicy.apply(p, bool(inplace), logits, target_ids,
-                                                        old_logprobs, advantages, mask)
-    out = _token_local_output(kind, obj, d1, d2, d3, trusted)
+    obj, d1, d2, d3, loss, logp, trusted = _FusedPolicy.apply(
+        p, bool(inplace), logits, target_ids, old_logprobs, advantages, mask)
+    out = _token_local_output(kind, obj, d1, d2, d3, loss, trusted)
     return (out, _cfg.as_reference_dtype(logp, logits)) if return_logprobs else out
 

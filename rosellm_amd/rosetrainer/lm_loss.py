@@ -13,8 +13,8 @@ logits.  Here the same loss is the objective kind NLL of the single-pass row
 kernel (``rrl_fused_logprob_policy``): every logits row is read once, in place
 through the shifted view, and its gradient row written once, with
 d loss / d logp = -1/n for the n non-ignored tokens known before the sweep
-(``rrl_policy_row_coef`` counts them).  The loss itself is the reduction of the
-per-token log-probs (``rrl_policy_fwd``).
+(``rrl_policy_prepare`` counts them).  The loss itself is the reduction of the
+per-token log-probs (``rrl_policy_forward``).
 
 Semantics follow ``torch.nn.functional.cross_entropy`` with ``weight=None``
 and ``label_smoothing=0`` (the reference's call): ``ignore_index`` tokens carry
@@ -25,8 +25,6 @@ logits dtype); arithmetic is float32 (float64 for float64 logits).
 """
 
 from __future__ import annotations
-
-from typing import Tuple
 
 import torch
 from torch import Tensor
@@ -65,14 +63,6 @@ def _check_labels(labels: Tensor) -> None:
         raise RuntimeError(f"expected scalar type Long but found {str(labels.dtype)[6:].capitalize()}")
 
 
-def _unused_operand(dev: torch.device, acc: torch.dtype) -> Tuple[nat.RrlView, Tensor]:
-    """The old-log-prob / advantage operands NLL does not read: one zero
-    broadcast to every token."""
-
-    z = torch.zeros(1, dtype=acc, device=dev)
-    return nat.RrlView(z.data_ptr(), nat.dtype_code(acc), 0, 0), z
-
-
 class _CrossEntropyRows(torch.autograd.Function):
     """-mean/sum of log_softmax(rows)[label] over non-ignored labels, with the
     gradient of every logits row written during the forward.
@@ -92,18 +82,10 @@ class _CrossEntropyRows(torch.autograd.Function):
         if inplace and (x.data_ptr() != src.data_ptr() or logits.stride(-1) != 1):
             raise RuntimeError("inplace=True needs logits whose rows can be addressed in place")
         tview, tkeep = nat.rows_view(lab, B, T)
-        acc = nat.acc_dtype(logits.dtype)
-        acc_code = nat.dtype_code(acc)
-        stream = nat.stream_ptr(dev)
-        unused, keep0 = _unused_operand(dev, acc)
-        ws = torch.empty(nat.lib().rrl_policy_workspace_bytes(B, acc_code), dtype=torch.uint8,
-                         device=dev)
-        coef = torch.empty(B, dtype=acc, device=dev)
-        records = torch.empty(nat.lib().rrl_fused_records_bytes(B, T), dtype=torch.uint8,
-                              device=dev)
-        logp = torch.empty(B * T, dtype=acc, device=dev)
-        lse = torch.empty(B * T, dtype=acc, device=dev)
-        scal = torch.empty(nat.NSCALARS, dtype=acc, device=dev)
+        # NLL reads neither old log-probs nor advantages; the operands must name
+        # some float memory, and the labels' own addresses will do.
+        unused = nat.RrlView(tview.ptr, nat.F32, 0, 0)
+        sweep = _losses._Sweep(params, x, (B, T, V, s_b, s_t), tview, unused, unused, tview, dev)
         if inplace:
             dl = logits
             d_b, d_t = s_b, s_t
@@ -115,44 +97,13 @@ class _CrossEntropyRows(torch.autograd.Function):
             else:
                 d_b, d_t = T * V, V
             dptr = dl.data_ptr()
-        lview = nat.RrlView(logp.data_ptr(), acc_code, T, 1)
-
-        early = _losses._check_before_sweep(logits, inplace)
-        rerun = _losses._rerun_on_device(logits, inplace)
-
-        def run(p):
-            status = nat.new_status(dev)
-            pref = _losses.ctypes_ref(p)
-            nat.call("rrl_policy_row_coef", pref, B, T, tview, acc_code, coef.data_ptr(),
-                     ws.data_ptr(), status.data_ptr(), stream)
-            if early:
-                nat.call("rrl_check_targets", pref, B, T, V, tview, status.data_ptr(), stream)
-                _losses._raise_flags(nat.read_status(status), nat.OBJ_NLL)
-            for q in (pref, _losses.ctypes_ref(_losses._rerun_params(p))) if rerun else (pref,):
-                nat.call("rrl_fused_logprob_policy", q, x.data_ptr(), nat.dtype_code(x.dtype), B,
-                         T, V, s_b, s_t, tview, unused, unused, tview, coef.data_ptr(),
-                         records.data_ptr(), logp.data_ptr(), lse.data_ptr(), dptr,
-                         nat.dtype_code(logits.dtype), d_b, d_t, status.data_ptr(), stream,
-                         timed=q is pref)
-            nat.call("rrl_policy_fwd", pref, B, T, lview, unused, unused, tview, acc_code,
-                     ws.data_ptr(), scal.data_ptr(), None, None, status.data_ptr(), stream)
-            return 0 if early else nat.read_status(status)
-
-        flags = run(params)
-        if flags & nat.FLAG_FAST_RANGE:
-            # A row's log-sum-exp lies beyond the register-resident 16-bit kernel's exponent
-            # range: redo the call on the generic row kernel.
-            if inplace:
-                raise RuntimeError(
-                    "cross-entropy with inplace=True: logits beyond +-2e38 need the generic "
-                    "kernel, which cannot rerun over overwritten logits; call with inplace=False")
-            generic = nat.RrlPolicyParams.from_buffer_copy(params)
-            generic.flags |= nat.POLICY_GENERIC
-            flags = run(generic)
-        _losses._raise_flags(flags, nat.OBJ_NLL)
+        loss = torch.empty((), dtype=sweep.acc, device=dev)
+        sweep.run(dptr, d_b, d_t, inplace, (None, None, None, None, loss), None,
+                  "cross-entropy with inplace=True: logits beyond +-2e38 need the generic "
+                  "kernel, which cannot rerun over overwritten logits; call with inplace=False")
         if shift and logits.shape[1] > 0:
             dl[:, -1].zero_()  # the last position predicts nothing
-        del keep0, tkeep
+        del tkeep
         # Row geometry of the whole gradient tensor for the backward's rescale:
         # in place it is the caller's logits, which may be a strided view (a
         # padded-vocabulary slice, a [:, :-1] shift) whose rows are not V apart.
@@ -162,7 +113,7 @@ class _CrossEntropyRows(torch.autograd.Function):
         ctx.dl = dl
         ctx.geom = (gB, gT, gV, gs_b, gs_t)
         ctx.set_materialize_grads(False)
-        return -scal[0]
+        return loss
 
     @staticmethod
     def backward(ctx, g):
@@ -248,8 +199,8 @@ def fused_linear_cross_entropy(hidden: Tensor, weight: Tensor, target: Tensor, *
     logp = _linear.linear_label_logprobs(hidden, weight, target, ignore_index,
                                          row_block=row_block, impl=impl)
     unused = torch.zeros((), dtype=torch.float32, device=dev).expand(target.shape)
-    obj = _losses._objective(p, logp, unused, unused, target)[0]
-    return _cfg.as_reference_dtype(-obj, hidden)
+    loss = _losses._objective(p, logp, unused, unused, target)[4]
+    return _cfg.as_reference_dtype(loss, hidden)
 
 
 def linear_causal_lm_loss(hidden: Tensor, weight: Tensor, labels: Tensor, *,
