@@ -371,8 +371,12 @@ class HostStatus:
 
     __slots__ = ("_word", "_event")
 
-    def __init__(self):
+    def __init__(self, zero: bool = False):
+        """``zero``: cleared first, for kernels that only set bits."""
+
         self._word = torch.empty(1, dtype=torch.int32, pin_memory=True)
+        if zero:
+            self._word.zero_()
         self._event = None
 
     @property

@@ -3,21 +3,28 @@
 //
 // The reverse recurrences (discounted returns, GAE, skip-observation GAE) are
 // affine maps on a small carried state, with padding acting as the identity.
-// One workgroup owns one sequence; each lane owns a contiguous chunk of time
-// steps:
-//   1. every lane composes the affine map of its chunk (reverse time);
-//   2. a log-depth suffix scan of the chunk maps over the lanes (8 steps
-//      through LDS for 256 lanes) gives each lane the composition of every
-//      later chunk, hence its chunk's incoming state;
-//   3. every lane replays its chunk with the reference's step arithmetic from
-//      its incoming state and writes the outputs.
+// One workgroup owns one sequence; each lane owns a few consecutive time steps:
+//   1. every lane composes the affine map of its steps (reverse time);
+//   2. a suffix scan of the lanes' maps (shuffles in a wave, then the waves'
+//      maps through LDS) gives each lane its incoming state;
+//   3. every lane replays its steps with the reference's step arithmetic from
+//      that state and writes the outputs.
 #include "rrl_common.hpp"
 
 namespace rrl {
 
 namespace {
 
-constexpr int SCAN_NT = 256;
+// Sets a bit of the caller's cleared status word without an atomic, so that
+// the word may be host memory: every writer in one of these launches sets the
+// same single bit.
+__device__ __forceinline__ void or_flag(int32_t* status, int32_t bit) {
+  if (status) {
+    volatile int32_t* p = status;
+    *p = *p | bit;
+    __threadfence_system();
+  }
+}
 
 struct ScanArgs {
   int64_t B, T;
@@ -30,170 +37,293 @@ struct ScanArgs {
   int odt;
 };
 
-// Affine map on a D-dimensional state: S' = Mx * S + c (row-major Mx).
-template <typename Acc, int D>
-struct Aff {
-  Acc m[D * D];
-  Acc c[D];
-  __device__ __forceinline__ static Aff identity() {
-    Aff a;
-#pragma unroll
-    for (int i = 0; i < D * D; ++i) a.m[i] = Acc(0);
-#pragma unroll
-    for (int i = 0; i < D; ++i) { a.m[i * D + i] = Acc(1); a.c[i] = Acc(0); }
-    return a;
+// Per-estimator recurrences.  KIND 0: discounted returns (state: the return).
+// KIND 1: GAE (state: next value, next advantage).  KIND 2: skip-observation
+// GAE (state: next advantage).
+template <int KIND> struct StateDim { static constexpr int D = KIND == 1 ? 2 : 1; };
+
+// A run of steps as a map on the carried state, S' = m S + c.  Padding is the
+// identity.
+template <typename Acc, int KIND>
+struct Run {
+  Acc m = Acc(1), c = Acc(0);
+  // This run preceded in time by one step with S' = sm S + sc.
+  __device__ __forceinline__ void step(Acc sm, Acc sc) {
+    c = sc + sm * c;
+    m = sm * m;
   }
-  // this <- step o this  (apply `this` first, then step)
-  __device__ __forceinline__ void prepend(const Aff& s) {
-    Aff r;
-#pragma unroll
-    for (int i = 0; i < D; ++i) {
-#pragma unroll
-      for (int j = 0; j < D; ++j) {
-        Acc acc = Acc(0);
-#pragma unroll
-        for (int k = 0; k < D; ++k) acc += s.m[i * D + k] * m[k * D + j];
-        r.m[i * D + j] = acc;
-      }
-      Acc acc = s.c[i];
-#pragma unroll
-      for (int k = 0; k < D; ++k) acc += s.m[i * D + k] * c[k];
-      r.c[i] = acc;
-    }
-    *this = r;
+  // This run applied after `later`.
+  __device__ __forceinline__ void after(const Run& later) {
+    c = c + m * later.c;
+    m = m * later.m;
   }
-  __device__ __forceinline__ void apply(Acc (&S)[D]) const {
-    Acc o[D];
-#pragma unroll
-    for (int i = 0; i < D; ++i) {
-      Acc acc = c[i];
-#pragma unroll
-      for (int k = 0; k < D; ++k) acc += m[i * D + k] * S[k];
-      o[i] = acc;
+  __device__ __forceinline__ void apply(Acc (&S)[1]) const { S[0] = c + m * S[0]; }
+  template <class F>
+  __device__ __forceinline__ Run moved(F f) const {
+    Run r;
+    r.m = f(m);
+    r.c = f(c);
+    return r;
+  }
+};
+// GAE: a run with a valid step leaves the value of its first one and an
+// advantage affine in the state; the value is carried as such (a product with
+// zero would turn an infinite value further on into NaN).
+template <typename Acc>
+struct Run<Acc, 1> {
+  int any = 0;
+  Acc v = Acc(0), c = Acc(0), mv = Acc(0), ma = Acc(1);
+  // One valid step: delta = rv + gn V', A = delta + gln A', V = sv.
+  __device__ __forceinline__ void step(Acc sv, Acc rv, Acc gn, Acc gln) {
+    c = any ? (rv + gn * v) + gln * c : rv;
+    mv = any ? gln * mv : gn;
+    ma = any ? gln * ma : gln;
+    v = sv;
+    any = 1;
+  }
+  __device__ __forceinline__ void after(const Run& later) {
+    if (!any) {
+      *this = later;
+    } else if (later.any) {
+      c = (c + mv * later.v) + ma * later.c;
+      mv = ma * later.mv;
+      ma = ma * later.ma;
     }
-#pragma unroll
-    for (int i = 0; i < D; ++i) S[i] = o[i];
+  }
+  __device__ __forceinline__ void apply(Acc (&S)[2]) const {
+    if (any) {
+      S[1] = (c + mv * S[0]) + ma * S[1];
+      S[0] = v;
+    }
+  }
+  template <class F>
+  __device__ __forceinline__ Run moved(F f) const {
+    Run r;
+    r.any = f(any);
+    r.v = f(v);
+    r.c = f(c);
+    r.mv = f(mv);
+    r.ma = f(ma);
+    return r;
   }
 };
 
-// Per-estimator step definitions.  KIND 0: discounted returns (state R).
-// KIND 1: GAE (state next_value, next_advantage).  KIND 2: skip-observation
-// GAE (state next_advantage).
-template <int KIND> struct StateDim { static constexpr int D = KIND == 1 ? 2 : 1; };
+// The runs of the wave's later lanes composed (`later`), and the whole wave's.
+template <class R>
+__device__ __forceinline__ void wave_suffix(const R& f, R& later, R& whole) {
+  const int lane = threadIdx.x & 63;
+  R p = f;  // this lane's run after those of the lanes behind it
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const R o = p.moved([&](auto x) { return __shfl_down(x, d, 64); });
+    if (lane + d < 64) p.after(o);
+  }
+  later = p.moved([&](auto x) { return __shfl_down(x, 1, 64); });
+  whole = p.moved([&](auto x) { return __shfl(x, 0, 64); });
+  if (lane == 63) later = R{};
+}
 
-template <typename Acc, int KIND>
-__device__ __forceinline__ Aff<Acc, StateDim<KIND>::D> step_map(const ScanArgs& a, int64_t b,
-                                                              int64_t t, Acc g, Acc gl) {
-  constexpr int D = StateDim<KIND>::D;
-  Aff<Acc, D> f = Aff<Acc, D>::identity();
-  const bool valid = a.valid.present() ? a.valid.truth(b, t) : true;
-  if (!valid) return f;
-  const Acc nt = (a.term.present() && a.term.truth(b, t)) ? Acc(0) : Acc(1);
-  if (KIND == 0) {
-    f.m[0] = g * nt;
-    f.c[0] = a.r.get<Acc>(b, t);
-  } else if (KIND == 1) {
-    const Acc V = a.v.get<Acc>(b, t);
-    f.m[0] = Acc(0); f.m[1] = Acc(0);
-    f.m[2] = g * nt; f.m[3] = gl * nt;
-    f.c[0] = V;
-    f.c[1] = a.r.get<Acc>(b, t) - V;
+// Four consecutive steps of an operand: one 16-byte load of contiguous aligned
+// float32 (VEC), or element by element.
+template <typename Acc, bool VEC>
+__device__ __forceinline__ void load_steps(const View& v, int64_t b, int64_t t, int64_t T,
+                                           Acc (&x)[4]) {
+  if constexpr (VEC) {
+    const float4 u = *reinterpret_cast<const float4*>(static_cast<const float*>(v.ptr) + b * v.sr + t);
+    x[0] = u.x; x[1] = u.y; x[2] = u.z; x[3] = u.w;
   } else {
-    f.m[0] = gl * nt;
-    f.c[0] = (a.r.get<Acc>(b, t) + (g * nt) * a.nv.get<Acc>(b, t)) - a.v.get<Acc>(b, t);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = t + i < T ? v.get<Acc>(b, t + i) : Acc(0);
+  }
+}
+template <bool VEC>
+__device__ __forceinline__ uint32_t load_flags(const View& v, int64_t b, int64_t t, int64_t T,
+                                               bool absent) {
+  if (!v.present()) return absent ? 0xFu : 0u;
+  uint32_t f = 0;
+  if constexpr (VEC) {
+    const uint32_t u =
+        *reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(v.ptr) + b * v.sr + t);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f |= (u >> (8 * i) & 0xFFu) ? 1u << i : 0u;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f |= t + i < T && v.truth(b, t + i) ? 1u << i : 0u;
   }
   return f;
 }
 
-// Reference step (advantages.py:75-79, :129-139, :196-210): update the state
-// in place and return the outputs for time t.
+// One step (the kind's reference: advantages.py:75-79, :129-139, :196-210)
+// as an addition to a run and in the
+// reference's own arithmetic.
 template <typename Acc, int KIND>
-__device__ __forceinline__ void ref_step(const ScanArgs& a, int64_t b, int64_t t, Acc g, Acc gl,
-                                         Acc (&S)[StateDim<KIND>::D], Acc& o0, Acc& o1) {
-  const bool valid = a.valid.present() ? a.valid.truth(b, t) : true;
-  const Acc nt = (a.term.present() && a.term.truth(b, t)) ? Acc(0) : Acc(1);
-  if (KIND == 0) {
-    const Acc cand = a.r.get<Acc>(b, t) + (g * nt) * S[0];
-    if (valid) S[0] = cand;
-    o0 = valid ? S[0] : Acc(0);
-    o1 = Acc(0);
-  } else if (KIND == 1) {
-    const Acc V = a.v.get<Acc>(b, t);
-    const Acc delta = (a.r.get<Acc>(b, t) + (g * nt) * S[0]) - V;
-    const Acc cand = delta + (gl * nt) * S[1];
-    const Acc adv = valid ? cand : Acc(0);
-    o0 = adv;
-    o1 = valid ? adv + V : Acc(0);
-    if (valid) { S[0] = V; S[1] = adv; }
-  } else {
-    const Acc V = a.v.get<Acc>(b, t);
-    const Acc delta = (a.r.get<Acc>(b, t) + (g * nt) * a.nv.get<Acc>(b, t)) - V;
-    const Acc cand = delta + (gl * nt) * S[0];
-    const Acc adv = valid ? cand : Acc(0);
-    o0 = adv;
-    o1 = valid ? adv + V : Acc(0);
-    if (valid) S[0] = adv;
+struct Step {
+  static constexpr int D = StateDim<KIND>::D;
+  Acc r, v, nv;
+  bool valid, term;
+  __device__ __forceinline__ void add_to(Run<Acc, KIND>& f, Acc g, Acc gl) const {
+    if (!valid) return;
+    const Acc nt = term ? Acc(0) : Acc(1);
+    if constexpr (KIND == 0) f.step(g * nt, r);
+    if constexpr (KIND == 1) f.step(v, r - v, g * nt, gl * nt);
+    if constexpr (KIND == 2) f.step(gl * nt, (r + (g * nt) * nv) - v);
   }
-}
+  __device__ __forceinline__ void replay(Acc g, Acc gl, Acc (&S)[D], Acc& o0, Acc& o1) const {
+    const Acc nt = term ? Acc(0) : Acc(1);
+    if (KIND == 0) {
+      const Acc cand = r + (g * nt) * S[0];
+      if (valid) S[0] = cand;
+      o0 = valid ? S[0] : Acc(0);
+      o1 = Acc(0);
+    } else if (KIND == 1) {
+      const Acc delta = (r + (g * nt) * S[0]) - v;
+      const Acc cand = delta + (gl * nt) * S[1];
+      const Acc adv = valid ? cand : Acc(0);
+      o0 = adv;
+      o1 = valid ? adv + v : Acc(0);
+      if (valid) { S[0] = v; S[1] = adv; }
+    } else {
+      const Acc delta = (r + (g * nt) * nv) - v;
+      const Acc cand = delta + (gl * nt) * S[0];
+      const Acc adv = valid ? cand : Acc(0);
+      o0 = adv;
+      o1 = valid ? adv + v : Acc(0);
+      if (valid) S[0] = adv;
+    }
+  }
+};
 
-template <typename Acc, int KIND>
-__global__ __launch_bounds__(SCAN_NT) void reverse_scan_kernel(ScanArgs a) {
+// Latency bounds the scan: 64 sequences of 8192 steps are 9 MB, but a sequence
+// is one dependent chain.  A lane holds E = 4 or 8 consecutive steps in
+// registers (read once, 16 bytes at a time where the layout allows), a wave
+// scans its lanes' runs with shuffles, and each wave carries the incoming
+// state through the later waves' runs (up to 15 of them), so a
+// tile of NT * E steps costs one barrier; longer sequences go tile by tile
+// from the end.  rrl_gae at 64 x 8192: 57.7 us before (32-step chunks read
+// twice, 16 barriers), 9.2 us here.
+template <typename Acc, int KIND, int NT, int E, bool VEC>
+__global__ __launch_bounds__(NT) void reverse_scan_kernel(ScanArgs a) {
   constexpr int D = StateDim<KIND>::D;
-  __shared__ Aff<Acc, D> sh_map[SCAN_NT];
+  constexpr int NW = NT / 64;
+  // Raw storage: the runs have initialisers, which LDS cannot.
+  __shared__ __align__(16) char sh_raw[2 * NW * sizeof(Run<Acc, KIND>)];
+  auto* sh_wave = reinterpret_cast<Run<Acc, KIND>*>(sh_raw);
   // gamma and gamma*lambda as the reference forms them: python float products
   // rounded to the tensor dtype.
   const Acc g = (Acc)a.gamma;
   const Acc gl = (Acc)(a.gamma * a.lam);
-  const int64_t C = (a.T + SCAN_NT - 1) / SCAN_NT;
+  const int wave = threadIdx.x >> 6;
+  const int64_t tile = (int64_t)NT * E;
   for (int64_t b = blockIdx.x; b < a.B; b += gridDim.x) {
-    const int64_t t0 = threadIdx.x * C;
-    const int64_t t1 = (t0 + C < a.T) ? t0 + C : a.T;
-    Aff<Acc, D> f = Aff<Acc, D>::identity();
-    for (int64_t t = t1 - 1; t >= t0; --t) f.prepend(step_map<Acc, KIND>(a, b, t, g, gl));
-    // Log-depth inclusive suffix scan of the chunk maps (Kogge-Stone over
-    // the lanes, through LDS): after the step of distance d, lane j holds
-    // P_j = f_j o f_(j+1) o ... o f_(j+2d-1) (the later chunks applied first),
-    // and after the last step P_j runs through every chunk from the
-    // sequence's end down to chunk j.
-    sh_map[threadIdx.x] = f;
-    __syncthreads();
-    for (int d = 1; d < SCAN_NT; d <<= 1) {
-      const bool has = threadIdx.x + d < SCAN_NT;
-      Aff<Acc, D> later;
-      if (has) later = sh_map[threadIdx.x + d];
-      __syncthreads();
-      if (has) {
-        later.prepend(f);  // `later` first, then this lane's map
-        f = later;
+    // The state behind the tile: at first the bootstrap value.
+    Acc C[D];
+    C[0] = KIND != 2 && a.boot.present() ? a.boot.get<Acc>(b, 0) : Acc(0);
+    if (D == 2) C[D - 1] = Acc(0);
+    int buf = 0;
+    for (int64_t base = (a.T - 1) / tile * tile; base >= 0; base -= tile, buf ^= 1) {
+      const int64_t t0 = base + (int64_t)threadIdx.x * E;
+      Step<Acc, KIND> st[E];
+#pragma unroll
+      for (int e = 0; e < E; e += 4) {
+        const int64_t t = t0 + e;
+        Acc r[4] = {}, v[4] = {}, nv[4] = {};
+        uint32_t ok = 0, term = 0;
+        if (t < a.T) {
+          load_steps<Acc, VEC>(a.r, b, t, a.T, r);
+          if (KIND != 0) load_steps<Acc, VEC>(a.v, b, t, a.T, v);
+          if (KIND == 2) load_steps<Acc, VEC>(a.nv, b, t, a.T, nv);
+          ok = load_flags<VEC>(a.valid, b, t, a.T, true);
+          term = load_flags<VEC>(a.term, b, t, a.T, false);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          st[e + i] = {r[i], v[i], nv[i], (ok >> i & 1u) && t + i < a.T, (term >> i & 1u) != 0};
       }
-      sh_map[threadIdx.x] = f;
+      Run<Acc, KIND> f, later, whole;
+#pragma unroll
+      for (int e = E - 1; e >= 0; --e) st[e].add_to(f, g, gl);
+      wave_suffix(f, later, whole);
+      if ((threadIdx.x & 63) == 0) sh_wave[buf * NW + wave] = whole;
       __syncthreads();
+      // Every wave carries the tile's incoming state down to its own end, and
+      // on through the rest for the next tile's.
+      Acc S[D];
+#pragma unroll
+      for (int i = 0; i < D; ++i) S[i] = C[i];
+#pragma unroll
+      for (int w = NW - 1; w >= 0; --w) {
+        if (w == wave) {
+#pragma unroll
+          for (int i = 0; i < D; ++i) S[i] = C[i];
+        }
+        sh_wave[buf * NW + w].apply(C);
+      }
+      later.apply(S);
+      Acc o0[E], o1[E];
+#pragma unroll
+      for (int e = E - 1; e >= 0; --e) st[e].replay(g, gl, S, o0[e], o1[e]);
+#pragma unroll
+      for (int e = 0; e < E; e += 4) {
+        const int64_t t = t0 + e;
+        if constexpr (VEC) {
+          if (t < a.T) {
+            float* p = static_cast<float*>(a.out0) + b * a.T + t;
+            *reinterpret_cast<float4*>(p) =
+                make_float4((float)o0[e], (float)o0[e + 1], (float)o0[e + 2], (float)o0[e + 3]);
+            if (KIND != 0) {
+              float* q = static_cast<float*>(a.out1) + b * a.T + t;
+              *reinterpret_cast<float4*>(q) =
+                  make_float4((float)o1[e], (float)o1[e + 1], (float)o1[e + 2], (float)o1[e + 3]);
+            }
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            if (t + i >= a.T) continue;
+            store_as<Acc>(a.out0, a.odt, b * a.T + t + i, o0[e + i]);
+            if (KIND != 0) store_as<Acc>(a.out1, a.odt, b * a.T + t + i, o1[e + i]);
+          }
+        }
+      }
     }
-    // Chunk j's incoming state: the initial state through P_(j+1).
-    Acc S[D];
-    if (KIND == 0) S[0] = a.boot.present() ? a.boot.get<Acc>(b, 0) : Acc(0);
-    if (KIND == 1) { S[0] = a.boot.present() ? a.boot.get<Acc>(b, 0) : Acc(0); S[1] = Acc(0); }
-    if (KIND == 2) S[0] = Acc(0);
-    if (threadIdx.x + 1 < SCAN_NT) sh_map[threadIdx.x + 1].apply(S);
-    for (int64_t t = t1 - 1; t >= t0; --t) {
-      Acc o0, o1;
-      ref_step<Acc, KIND>(a, b, t, g, gl, S, o0, o1);
-      store_as<Acc>(a.out0, a.odt, b * a.T + t, o0);
-      if (KIND != 0) store_as<Acc>(a.out1, a.odt, b * a.T + t, o1);
-    }
-    __syncthreads();
+    __syncthreads();  // the next sequence writes sh_wave again
   }
+}
+
+// Contiguous float32 steps at 16-byte aligned rows.
+bool vec_steps(const View& v, bool used) {
+  return !used || (v.dt == RRL_F32 && v.sc == 1 && v.sr % 4 == 0 && (uintptr_t)v.ptr % 16 == 0);
+}
+// Contiguous one-byte flags at 4-byte aligned rows, or none.
+bool vec_flags(const View& v) {
+  return !v.present() || ((v.dt == RRL_BOOL || v.dt == RRL_U8 || v.dt == RRL_I8) && v.sc == 1 &&
+                          v.sr % 4 == 0 && (uintptr_t)v.ptr % 4 == 0);
+}
+
+template <typename Acc, int KIND, bool VEC>
+int launch_scan_as(const ScanArgs& a, hipStream_t st) {
+  const unsigned grid = (unsigned)(a.B < 65536 ? a.B : 65536);
+  // One wave for short sequences: no other wave's map to carry the state through.
+  if (a.T <= 256)
+    hipLaunchKernelGGL((reverse_scan_kernel<Acc, KIND, 64, 4, VEC>), dim3(grid), dim3(64), 0, st, a);
+  else if (a.T <= 1024)
+    hipLaunchKernelGGL((reverse_scan_kernel<Acc, KIND, 256, 4, VEC>), dim3(grid), dim3(256), 0, st,
+                       a);
+  else
+    hipLaunchKernelGGL((reverse_scan_kernel<Acc, KIND, 1024, 8, VEC>), dim3(grid), dim3(1024), 0,
+                       st, a);
+  return check_launch("reverse_scan_kernel");
 }
 
 template <int KIND>
 int launch_scan(const ScanArgs& a, bool f64, hipStream_t st) {
   if (a.B * a.T == 0) return RRL_OK;
-  const unsigned grid = (unsigned)(a.B < 65536 ? a.B : 65536);
-  if (f64)
-    hipLaunchKernelGGL((reverse_scan_kernel<double, KIND>), dim3(grid), dim3(SCAN_NT), 0, st, a);
-  else
-    hipLaunchKernelGGL((reverse_scan_kernel<float, KIND>), dim3(grid), dim3(SCAN_NT), 0, st, a);
-  return check_launch("reverse_scan_kernel");
+  if (f64) return launch_scan_as<double, KIND, false>(a, st);
+  const bool vec = a.T % 4 == 0 && vec_steps(a.r, true) && vec_steps(a.v, KIND != 0) &&
+                   vec_steps(a.nv, KIND == 2) && vec_flags(a.term) && vec_flags(a.valid) &&
+                   a.odt == RRL_F32 && (uintptr_t)a.out0 % 16 == 0 &&
+                   (KIND == 0 || (uintptr_t)a.out1 % 16 == 0);
+  return vec ? launch_scan_as<float, KIND, true>(a, st) : launch_scan_as<float, KIND, false>(a, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -255,7 +385,7 @@ __global__ void broadcast_turn_kernel(int64_t B, int64_t K, int64_t T, View adv,
     Acc v = Acc(0);
     if (m) {
       if (id < 0 || id >= K) {
-        raise_flag(status, RRL_FLAG_INVALID_TURN);
+        or_flag(status, RRL_FLAG_INVALID_TURN);
       } else {
         v = adv.get<Acc>(b, id);
       }
@@ -274,7 +404,6 @@ constexpr int RED_MAXB = 1024;
 struct RedArgs {
   int64_t B, T;
   View x, mask;
-  bool weight;     // mask cast to the value dtype (masked_mean) vs mask != 0
   void* part;      // Acc[RED_MAXB][4]
   double eps;
   int shift;
@@ -291,12 +420,7 @@ inline unsigned red_grid(int64_t n) {
   return (unsigned)g;
 }
 
-template <typename Acc>
-__device__ __forceinline__ Acc red_weight(const RedArgs& a, int64_t b, int64_t t) {
-  return a.weight ? a.mask.get<Acc>(b, t) : (a.mask.truth(b, t) ? Acc(1) : Acc(0));
-}
-
-// Sum of the first two partial columns over all blocks, in block order.
+// Sum of a partial column over all blocks, in block order.
 template <typename Acc>
 __device__ void sum_partials(const Acc* part, int nb, int col, Acc& out, Acc* sh) {
   Acc v[1] = {Acc(0)};
@@ -305,45 +429,24 @@ __device__ void sum_partials(const Acc* part, int nb, int col, Acc& out, Acc* sh
   out = v[0];
 }
 
-// pass 0: part = (sum w*x, sum w); pass 1: part[.,2] = sum w*(x - mean)^2.
-template <typename Acc, int PASS>
+// masked_mean: part = (sum w*x, sum w).
+template <typename Acc>
 __global__ __launch_bounds__(RED_NT) void masked_partials_kernel(RedArgs a) {
   __shared__ Acc sh[(RED_NT / 64) * 2];
   Acc* part = static_cast<Acc*>(a.part);
-  Acc mean = Acc(0);
-  if (PASS == 1) {
-    Acc s0, s1;
-    sum_partials<Acc>(part, gridDim.x, 0, s0, sh);
-    sum_partials<Acc>(part, gridDim.x, 1, s1, sh);
-    mean = s0 / s1;
-  }
   Acc v[2] = {Acc(0), Acc(0)};
   const int64_t n = a.B * a.T;
   for (int64_t i = blockIdx.x * (int64_t)RED_NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * RED_NT) {
     const int64_t b = i / a.T, t = i - (i / a.T) * a.T;
-    const Acc w = red_weight<Acc>(a, b, t);
+    const Acc w = a.mask.get<Acc>(b, t);
     const Acc x = a.x.get<Acc>(b, t);
-    if (PASS == 0) {
-      if (a.weight) {
-        v[0] += x * w;
-        v[1] += w;
-      } else if (w != Acc(0)) {
-        v[0] += x;
-        v[1] += Acc(1);
-      }
-    } else if (w != Acc(0)) {
-      const Acc d = x - mean;
-      v[0] += d * d * w;
-    }
+    v[0] += x * w;
+    v[1] += w;
   }
   block_sum<RED_NT, 2, Acc>(v, sh);
   if (threadIdx.x == 0) {
-    if (PASS == 0) {
-      part[blockIdx.x * 4 + 0] = v[0];
-      part[blockIdx.x * 4 + 1] = v[1];
-    } else {
-      part[blockIdx.x * 4 + 2] = v[0];
-    }
+    part[blockIdx.x * 4 + 0] = v[0];
+    part[blockIdx.x * 4 + 1] = v[1];
   }
 }
 
@@ -355,7 +458,7 @@ __global__ __launch_bounds__(RED_NT) void masked_mean_final_kernel(RedArgs a, in
   sum_partials<Acc>(static_cast<const Acc*>(a.part), nb, 0, s0, sh);
   sum_partials<Acc>(static_cast<const Acc*>(a.part), nb, 1, s1, sh);
   if (threadIdx.x == 0) {
-    if (s1 == Acc(0)) raise_flag(a.status, RRL_FLAG_EMPTY_MASK);
+    if (s1 == Acc(0)) or_flag(a.status, RRL_FLAG_EMPTY_MASK);
     static_cast<Acc*>(a.out)[0] = s0 / s1;
     static_cast<Acc*>(a.part)[RED_MAXB * 4] = s1;  // denominator for the backward
   }
@@ -368,30 +471,133 @@ __global__ __launch_bounds__(RED_NT) void masked_mean_bwd_kernel(RedArgs a) {
   const int64_t n = a.B * a.T;
   for (int64_t i = blockIdx.x * (int64_t)RED_NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * RED_NT) {
     const int64_t b = i / a.T, t = i - (i / a.T) * a.T;
-    static_cast<Acc*>(a.out)[i] = (G / den) * red_weight<Acc>(a, b, t);
+    static_cast<Acc*>(a.out)[i] = (G / den) * a.mask.get<Acc>(b, t);
   }
 }
 
+// Masked whitening in two launches.  The first forms each tile's count, mean
+// and sum of squared deviations from the tile's own mean (the tile sits in
+// registers, so that is a two-pass sum without a second read) and merges a
+// workgroup's tiles; the second merges the workgroups' and writes.  Bytes are
+// few (64 x 8192: 4.7 MB); launches and the 64-bit division per element that
+// strided operands need bounded it: three launches took 24 us, these 15.7.
+constexpr int WH_E = 8;  // elements per lane and tile
+
+// (count, mean, M2) <- merged with another group's.
 template <typename Acc>
+struct Moments {
+  Acc n, mean, m2;
+  __device__ __forceinline__ void merge(Acc n2, Acc mean2, Acc m22) {
+    if (n2 == Acc(0)) return;
+    const Acc nt = n + n2, d = mean2 - mean, f = n2 / nt;
+    mean += d * f;
+    m2 += m22 + d * d * n * f;
+    n = nt;
+  }
+};
+
+// Element offsets of flat index i: FLAT operands are contiguous as a whole.
+template <bool FLAT>
+__device__ __forceinline__ void split_index(const RedArgs& a, int64_t i, int64_t& b, int64_t& t) {
+  if constexpr (FLAT) {
+    b = 0;
+    t = i;
+  } else {
+    b = i / a.T;
+    t = i - b * a.T;
+  }
+}
+
+template <typename Acc, bool FLAT>
+__global__ __launch_bounds__(RED_NT) void whiten_moments_kernel(RedArgs a) {
+  __shared__ Acc sh[(RED_NT / 64) * 2];
+  Acc* part = static_cast<Acc*>(a.part);
+  const int64_t n = a.B * a.T;
+  constexpr int64_t kTile = (int64_t)RED_NT * WH_E;
+  Moments<Acc> q{Acc(0), Acc(0), Acc(0)};
+  for (int64_t i0 = blockIdx.x * kTile; i0 < n; i0 += (int64_t)gridDim.x * kTile) {
+    Acc x[WH_E];
+    bool m[WH_E];
+    Acc v[2] = {Acc(0), Acc(0)};
+#pragma unroll
+    for (int e = 0; e < WH_E; ++e) {
+      const int64_t i = i0 + e * RED_NT + threadIdx.x;
+      m[e] = false;
+      x[e] = Acc(0);
+      if (i < n) {
+        int64_t b, t;
+        split_index<FLAT>(a, i, b, t);
+        m[e] = a.mask.truth(b, t);
+        x[e] = a.x.get<Acc>(b, t);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < WH_E; ++e)
+      if (m[e]) {
+        v[0] += x[e];
+        v[1] += Acc(1);
+      }
+    block_sum<RED_NT, 2, Acc>(v, sh);
+    const Acc mean = v[1] != Acc(0) ? v[0] / v[1] : Acc(0);
+    Acc s[1] = {Acc(0)};
+#pragma unroll
+    for (int e = 0; e < WH_E; ++e) {
+      const Acc d = x[e] - mean;
+      if (m[e]) s[0] += d * d;
+    }
+    block_sum<RED_NT, 1, Acc>(s, sh);
+    q.merge(v[1], mean, s[0]);
+  }
+  if (threadIdx.x == 0) {
+    part[blockIdx.x * 4 + 0] = q.n * q.mean;
+    part[blockIdx.x * 4 + 1] = q.n;
+    part[blockIdx.x * 4 + 2] = q.m2;
+  }
+}
+
+template <typename Acc, bool FLAT>
 __global__ __launch_bounds__(RED_NT) void whiten_write_kernel(RedArgs a, int nb) {
-  __shared__ Acc sh[RED_NT / 64];
+  __shared__ Acc sh[(RED_NT / 64) * 2];
   const Acc* part = static_cast<const Acc*>(a.part);
-  Acc s0, s1, s2;
-  sum_partials<Acc>(part, nb, 0, s0, sh);
-  sum_partials<Acc>(part, nb, 1, s1, sh);
-  sum_partials<Acc>(part, nb, 2, s2, sh);
-  if (blockIdx.x == 0 && threadIdx.x == 0 && s1 == Acc(0)) raise_flag(a.status, RRL_FLAG_EMPTY_MASK);
-  const Acc mean = s0 / s1;
-  const Acc sd = M<Acc>::sqrt(s2 / s1);
+  Acc v[2] = {Acc(0), Acc(0)};
+  for (int i = threadIdx.x; i < nb; i += RED_NT) {
+    v[0] += part[i * 4 + 0];
+    v[1] += part[i * 4 + 1];
+  }
+  block_sum<RED_NT, 2, Acc>(v, sh);
+  if (blockIdx.x == 0 && threadIdx.x == 0 && v[1] == Acc(0)) or_flag(a.status, RRL_FLAG_EMPTY_MASK);
+  const Acc mean = v[0] / v[1];
+  Acc s2[1] = {Acc(0)};
+  for (int i = threadIdx.x; i < nb; i += RED_NT) {
+    const Acc ni = part[i * 4 + 1];
+    const Acc d = ni != Acc(0) ? part[i * 4 + 0] / ni - mean : Acc(0);
+    s2[0] += part[i * 4 + 2] + ni * d * d;
+  }
+  block_sum<RED_NT, 1, Acc>(s2, sh);
+  const Acc sd = M<Acc>::sqrt(s2[0] / v[1]);
   const Acc den = sd + (Acc)a.eps;
   const int64_t n = a.B * a.T;
   for (int64_t i = blockIdx.x * (int64_t)RED_NT + threadIdx.x; i < n; i += (int64_t)gridDim.x * RED_NT) {
-    const int64_t b = i / a.T, t = i - (i / a.T) * a.T;
+    int64_t b, t;
+    split_index<FLAT>(a, i, b, t);
     const bool m = a.mask.truth(b, t);
     const Acc x = a.x.get<Acc>(b, t);
     const Acc y = a.shift ? (x - mean) / den : x / den;
     store_as<Acc>(a.out, a.odt, i, m ? y : Acc(0));
   }
+}
+
+template <typename Acc>
+int launch_whiten(const RedArgs& a, unsigned nb, hipStream_t st) {
+  const auto flat = [&](const View& v) { return v.sc == 1 && (v.sr == a.T || a.B == 1); };
+  if (flat(a.x) && flat(a.mask)) {
+    hipLaunchKernelGGL((whiten_moments_kernel<Acc, true>), dim3(nb), dim3(RED_NT), 0, st, a);
+    hipLaunchKernelGGL((whiten_write_kernel<Acc, true>), dim3(nb), dim3(RED_NT), 0, st, a, (int)nb);
+  } else {
+    hipLaunchKernelGGL((whiten_moments_kernel<Acc, false>), dim3(nb), dim3(RED_NT), 0, st, a);
+    hipLaunchKernelGGL((whiten_write_kernel<Acc, false>), dim3(nb), dim3(RED_NT), 0, st, a, (int)nb);
+  }
+  return check_launch("masked_whiten");
 }
 
 // sequence_log_ratio: one workgroup per row.
@@ -410,7 +616,7 @@ __global__ __launch_bounds__(RED_NT) void seq_log_ratio_kernel(int64_t B, int64_
     }
     block_sum<RED_NT, 2, Acc>(v, sh);
     if (threadIdx.x == 0) {
-      if (v[1] == Acc(0)) raise_flag(status, RRL_FLAG_EMPTY_ROW);
+      if (v[1] == Acc(0)) or_flag(status, RRL_FLAG_EMPTY_ROW);
       out[b] = norm ? v[0] / v[1] : v[0];
       counts[b] = v[1];
     }
@@ -584,16 +790,16 @@ extern "C" int rrl_masked_mean_fwd(int64_t B, int64_t T, rrl_view values, rrl_vi
   RRL_REQUIRE(is_float_dtype(values.dtype) && is_known_dtype(mask.dtype), RRL_EDTYPE,
               "unsupported dtype");
   RedArgs a{};
-  a.B = B; a.T = T; a.x = to_view(values); a.mask = to_view(mask); a.weight = true;
+  a.B = B; a.T = T; a.x = to_view(values); a.mask = to_view(mask);
   a.part = workspace; a.out = out; a.status = status;
   const unsigned nb = red_grid(B * T);
   hipStream_t st = as_stream(stream);
   if (acc_dtype == RRL_F64) {
-    hipLaunchKernelGGL((masked_partials_kernel<double, 0>), dim3(nb), dim3(RED_NT), 0, st, a);
+    hipLaunchKernelGGL((masked_partials_kernel<double>), dim3(nb), dim3(RED_NT), 0, st, a);
     if (int rc = check_launch("masked_partials_kernel")) return rc;
     hipLaunchKernelGGL((masked_mean_final_kernel<double>), dim3(1), dim3(RED_NT), 0, st, a, (int)nb);
   } else {
-    hipLaunchKernelGGL((masked_partials_kernel<float, 0>), dim3(nb), dim3(RED_NT), 0, st, a);
+    hipLaunchKernelGGL((masked_partials_kernel<float>), dim3(nb), dim3(RED_NT), 0, st, a);
     if (int rc = check_launch("masked_partials_kernel")) return rc;
     hipLaunchKernelGGL((masked_mean_final_kernel<float>), dim3(1), dim3(RED_NT), 0, st, a, (int)nb);
   }
@@ -607,7 +813,7 @@ extern "C" int rrl_masked_mean_bwd(int64_t B, int64_t T, rrl_view mask, int32_t 
   RRL_REQUIRE(workspace && grad && (B * T == 0 || grad_values), RRL_EINVAL, "null pointer argument");
   if (B * T == 0) return RRL_OK;
   RedArgs a{};
-  a.B = B; a.T = T; a.mask = to_view(mask); a.weight = true;
+  a.B = B; a.T = T; a.mask = to_view(mask);
   a.part = const_cast<void*>(workspace); a.grad = grad; a.out = grad_values;
   hipStream_t st = as_stream(stream);
   const unsigned grid = flat_grid(B * T, RED_NT);
@@ -628,21 +834,12 @@ extern "C" int rrl_masked_whiten(int64_t B, int64_t T, rrl_view x, rrl_view mask
   RRL_REQUIRE(is_float_dtype(x.dtype) && is_known_dtype(mask.dtype) && is_float_dtype(out_dtype),
               RRL_EDTYPE, "unsupported dtype");
   RedArgs a{};
-  a.B = B; a.T = T; a.x = to_view(x); a.mask = to_view(mask); a.weight = false;
+  a.B = B; a.T = T; a.x = to_view(x); a.mask = to_view(mask);
   a.part = workspace; a.eps = eps; a.shift = shift_mean; a.out = out; a.odt = out_dtype;
   a.status = status;
   const unsigned nb = red_grid(B * T);
   hipStream_t st = as_stream(stream);
-  if (acc_dtype == RRL_F64) {
-    hipLaunchKernelGGL((masked_partials_kernel<double, 0>), dim3(nb), dim3(RED_NT), 0, st, a);
-    hipLaunchKernelGGL((masked_partials_kernel<double, 1>), dim3(nb), dim3(RED_NT), 0, st, a);
-    hipLaunchKernelGGL((whiten_write_kernel<double>), dim3(nb), dim3(RED_NT), 0, st, a, (int)nb);
-  } else {
-    hipLaunchKernelGGL((masked_partials_kernel<float, 0>), dim3(nb), dim3(RED_NT), 0, st, a);
-    hipLaunchKernelGGL((masked_partials_kernel<float, 1>), dim3(nb), dim3(RED_NT), 0, st, a);
-    hipLaunchKernelGGL((whiten_write_kernel<float>), dim3(nb), dim3(RED_NT), 0, st, a, (int)nb);
-  }
-  return check_launch("masked_whiten");
+  return acc_dtype == RRL_F64 ? launch_whiten<double>(a, nb, st) : launch_whiten<float>(a, nb, st);
 }
 
 extern "C" int rrl_sequence_log_ratio_fwd(int64_t B, int64_t T, rrl_view cur, rrl_view old,

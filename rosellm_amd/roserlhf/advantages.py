@@ -256,11 +256,12 @@ def broadcast_turn_advantages(
     mv, _mk = nat.rows_view(mask, B, T)
     acc = nat.acc_dtype(turn_advantages.dtype)
     out = torch.empty((B, T), dtype=acc, device=dev)
-    status = nat.new_status(dev)
-    nat.call("rrl_broadcast_turn", B, K, T, av, iv, mv, out.data_ptr(), nat.dtype_code(acc),
-             status.data_ptr(), nat.stream_ptr(dev))
-    if B * T and nat.read_status(status) & nat.FLAG_INVALID_TURN:
-        raise ValueError("an unmasked policy token has an invalid turn ID")
+    with nat.HostStatus(zero=True) as status:
+        nat.call("rrl_broadcast_turn", B, K, T, av, iv, mv, out.data_ptr(), nat.dtype_code(acc),
+                 status.ptr, nat.stream_ptr(dev))
+        status.record(dev)
+        if status.read() & nat.FLAG_INVALID_TURN:
+            raise ValueError("an unmasked policy token has an invalid turn ID")
     return out.to(turn_advantages.dtype)
 
 
@@ -293,10 +294,11 @@ def masked_whiten(
     acc = nat.acc_dtype(values.dtype)
     ws = torch.empty(nat.lib().rrl_reduce_workspace_bytes(B * T), dtype=torch.uint8, device=dev)
     out = torch.empty(values.shape, dtype=acc, device=dev)
-    status = nat.new_status(dev)
-    nat.call("rrl_masked_whiten", B, T, xv, mv, float(eps), int(bool(shift_mean)),
-             nat.dtype_code(acc), ws.data_ptr(), out.data_ptr(), nat.dtype_code(acc),
-             status.data_ptr(), nat.stream_ptr(dev))
-    if nat.read_status(status) & nat.FLAG_EMPTY_MASK:
-        raise ValueError("cannot reduce an empty mask")
+    with nat.HostStatus(zero=True) as status:
+        nat.call("rrl_masked_whiten", B, T, xv, mv, float(eps), int(bool(shift_mean)),
+                 nat.dtype_code(acc), ws.data_ptr(), out.data_ptr(), nat.dtype_code(acc),
+                 status.ptr, nat.stream_ptr(dev))
+        status.record(dev)
+        if status.read() & nat.FLAG_EMPTY_MASK:
+            raise ValueError("cannot reduce an empty mask")
     return out.to(values.dtype)

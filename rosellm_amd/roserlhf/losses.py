@@ -228,11 +228,12 @@ class _MaskedMean(torch.autograd.Function):
         acc = nat.acc_dtype(values.dtype)
         ws = torch.empty(nat.lib().rrl_reduce_workspace_bytes(B * T), dtype=torch.uint8, device=dev)
         out = torch.empty(1, dtype=acc, device=dev)
-        status = nat.new_status(dev)
-        nat.call("rrl_masked_mean_fwd", B, T, vview, mview, nat.dtype_code(acc), ws.data_ptr(),
-                 out.data_ptr(), status.data_ptr(), nat.stream_ptr(dev))
-        if nat.read_status(status) & nat.FLAG_EMPTY_MASK:
-            raise ValueError("cannot reduce an empty mask")
+        with nat.HostStatus(zero=True) as status:
+            nat.call("rrl_masked_mean_fwd", B, T, vview, mview, nat.dtype_code(acc),
+                     ws.data_ptr(), out.data_ptr(), status.ptr, nat.stream_ptr(dev))
+            status.record(dev)
+            if status.read() & nat.FLAG_EMPTY_MASK:
+                raise ValueError("cannot reduce an empty mask")
         ctx.save_for_backward(mkeep, ws)
         ctx.meta = (B, T, acc, tuple(values.shape), values.dtype)
         ctx.set_materialize_grads(False)
@@ -705,12 +706,13 @@ class _SequenceLogRatio(torch.autograd.Function):
         acc = nat.acc_dtype(cur.dtype, old.dtype)
         out = torch.empty(B, dtype=acc, device=dev)
         counts = torch.empty(B, dtype=acc, device=dev)
-        status = nat.new_status(dev)
-        nat.call("rrl_sequence_log_ratio_fwd", B, T, cv, ov, mv, int(normalize),
-                 nat.dtype_code(acc), out.data_ptr(), counts.data_ptr(), status.data_ptr(),
-                 nat.stream_ptr(dev))
-        if B and nat.read_status(status) & nat.FLAG_EMPTY_ROW:
-            raise ValueError("every sequence needs at least one action token")
+        with nat.HostStatus(zero=True) as status:
+            nat.call("rrl_sequence_log_ratio_fwd", B, T, cv, ov, mv, int(normalize),
+                     nat.dtype_code(acc), out.data_ptr(), counts.data_ptr(), status.ptr,
+                     nat.stream_ptr(dev))
+            status.record(dev)
+            if status.read() & nat.FLAG_EMPTY_ROW:
+                raise ValueError("every sequence needs at least one action token")
         ctx.save_for_backward(mk, counts)
         ctx.meta = (B, T, acc, normalize, cur.dtype)
         ctx.set_materialize_grads(False)

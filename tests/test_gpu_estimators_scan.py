@@ -1,0 +1,118 @@
+"""The reverse scans and the masked whitening at the edges of their tiles
+(MI355X), against a plain walk through time in float64.
+
+Sequence lengths sit on, and one past, one wave (256 steps), one 256-lane
+tile (1024) and one and two 1024-lane tiles (8192, 16384); lengths that are
+not multiples of four and strided operands take the element-wise loads.  Bars:
+the carried state is a sum of at most T terms in float32 (1e-5 of the largest
+term); whitening 1e-5 relative.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from rosellm_amd import roserlhf as R
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [1, 3, 4, 255, 256, 257, 260, 1023, 1024, 1025, 1028, 8191, 8192, 8196, 16384, 16388]
+
+
+def _inputs(B, T, device):
+    g = torch.Generator(device=device).manual_seed(T)
+    r = torch.randn(B, T, device=device, generator=g)
+    v = torch.randn(B, T, device=device, generator=g)
+    nv = torch.randn(B, T, device=device, generator=g)
+    valid = torch.rand(B, T, device=device, generator=g) < 0.8
+    term = torch.rand(B, T, device=device, generator=g) < 0.01
+    valid[0, -1] = False
+    if B > 2:
+        valid[2] = False  # nothing but padding
+    boot = torch.randn(B, device=device, generator=g)
+    return r, v, nv, valid, term, boot
+
+
+def _walk(r, v, nv, valid, term, boot, gamma, lam):
+    r, v, nv, boot = (x.double().cpu() for x in (r, v, nv, boot))
+    ok, nt = valid.cpu(), (~term.cpu()).double()
+    B, T = r.shape
+    ret, gae, tgt, skip = (torch.zeros(B, T, dtype=torch.float64) for _ in range(4))
+    R0, V1, A1, A2 = boot.clone(), boot.clone(), torch.zeros(B).double(), torch.zeros(B).double()
+    for t in range(T - 1, -1, -1):
+        m = ok[:, t]
+        R0 = torch.where(m, r[:, t] + gamma * nt[:, t] * R0, R0)
+        ret[:, t] = torch.where(m, R0, 0.0)
+        a = r[:, t] + gamma * nt[:, t] * V1 - v[:, t] + gamma * lam * nt[:, t] * A1
+        A1, V1 = torch.where(m, a, A1), torch.where(m, v[:, t], V1)
+        gae[:, t] = torch.where(m, a, 0.0)
+        tgt[:, t] = torch.where(m, a + v[:, t], 0.0)
+        a = r[:, t] + gamma * nt[:, t] * nv[:, t] - v[:, t] + gamma * lam * nt[:, t] * A2
+        A2 = torch.where(m, a, A2)
+        skip[:, t] = torch.where(m, a, 0.0)
+    return ret, gae, tgt, skip
+
+
+def _near(got, want):
+    scale = max(1.0, want.abs().max().item())
+    assert (got.double().cpu() - want).abs().max().item() <= 1e-5 * scale
+
+
+@pytest.mark.parametrize("T", LENGTHS)
+@pytest.mark.parametrize("strided", [False, True])
+def test_scans(device, T, strided):
+    print(f"[scan] T={T} strided={strided}", flush=True)
+    ins = _inputs(3, T, device)
+    if strided:  # every second element of a wider tensor
+        wide = lambda x: torch.stack([x, torch.zeros_like(x)], -1).reshape(3, -1)[:, ::2]  # noqa: E731
+        ins = tuple(wide(x) if x.ndim == 2 else x for x in ins)
+    r, v, nv, valid, term, boot = ins
+    ret, gae, tgt, skip = _walk(*ins, 0.99, 0.95)
+    kw = dict(terminated=term, valid_mask=valid)
+    _near(R.discounted_returns(r, gamma=0.99, bootstrap_value=boot, **kw), ret)
+    a, t = R.generalized_advantage_estimation(r, v, gamma=0.99, gae_lambda=0.95,
+                                              bootstrap_value=boot, **kw)
+    _near(a, gae)
+    _near(t, tgt)
+    a, _ = R.skip_observation_generalized_advantage_estimation(r, v, nv, gamma=0.99,
+                                                               gae_lambda=0.95, **kw)
+    _near(a, skip)
+
+
+def test_gae_infinite_value_stays_where_the_recurrence_has_it(device):
+    """An infinite value reaches its own step and, through the bootstrap and
+    the trace, the steps before it; a terminal step's products with zero make
+    NaN as the reference's do."""
+
+    r, v, nv, valid, term, boot = _inputs(2, 512, device)
+    valid[:], term[:] = True, False
+    v[0, 300] = float("inf")
+    ins = (r, v, nv, valid, term, boot)
+    _, gae, tgt, _ = _walk(*ins, 1.0, 0.0)
+    a, t = R.generalized_advantage_estimation(r, v, gamma=1.0, gae_lambda=0.0,
+                                              bootstrap_value=boot)
+    assert torch.equal(torch.isnan(a.cpu()), torch.isnan(gae))
+    assert torch.equal(torch.isinf(t.cpu()), torch.isinf(tgt))
+
+
+@pytest.mark.parametrize("B,T", [(1, 1), (1, 2047), (1, 2048), (3, 683), (7, 4099), (1, 2100000)])
+@pytest.mark.parametrize("layout", ["flat", "strided"])
+def test_whiten_tiles(device, B, T, layout):
+    """One tile of 2048 elements, a remainder, and more tiles than workgroups;
+    a large common offset, which a one-pass sum of squares would lose."""
+
+    g = torch.Generator(device=device).manual_seed(T)
+    x = 1000.0 + torch.randn(B, T, device=device, generator=g)
+    m = torch.rand(B, T, device=device, generator=g) < 0.6
+    m[0, 0] = True
+    if layout == "strided":
+        x = torch.stack([x, x], -1).reshape(B, -1)[:, ::2]
+    xd = x.double()[m]
+    sd = xd.var(unbiased=False).sqrt() if xd.numel() > 1 else xd.new_zeros(())
+    want = torch.where(m, (x.double() - xd.mean()) / (sd + 1e-3), 0.0)
+    got = R.masked_whiten(x, m, eps=1e-3)
+    # float32 mean of values near 1000: 1e-4 of a standard deviation
+    assert (got.double() - want).abs().max().item() <= 1e-3 * max(1.0, want.abs().max().item())
+    with pytest.raises(ValueError):
+        R.masked_whiten(x, torch.zeros_like(m))
