@@ -35,9 +35,12 @@
 //   6. the token's log-prob in the form the training row kernels use
 //      (finish_row), from pass 1's sums.
 // Greedy decoding is pass 1 alone; sampling without top-k / top-p is passes 1
-// and 5.  With top-k (k <= 1024), one pass after step 2 gathers the entries
-// at or above the k-th key into LDS and steps 3-5 run on that list, one
-// candidate per thread, without re-reading the row.
+// and 5 (log q's floor excess is summed on pass 5's own read).  Top-k (up to
+// the lanes that hold data) and top-p first try a candidate list: the entries
+// at or above a lane-maximum threshold, gathered in one pass after pass 1 by
+// the few lanes that hold any; steps 2-5 then run on the list.  A list that
+// overflows, or that ends before the nucleus does, leaves the row to the
+// passes above.
 // Ties at a top-k or top-p threshold are kept lowest index first; they are
 // located with the same vocabulary-order search over 0/1 weights.
 #include "row_common.hpp"
@@ -128,15 +131,20 @@ template <> struct Bits<TagF32> {
   static __device__ __forceinline__ uint32_t bits_of(float v) { return __float_as_uint(v); }
 };
 
-// Lane `tid`'s 16 bytes of slab k as stored (zeros past the row's end); a
-// row that is not 16-byte aligned, or the row's last partial vector, is read
-// element by element.
+// Lane `tid`'s 16 bytes of slab k as stored (zeros past the row's end); only
+// the row's last partial vector is read element by element.  A row need not
+// be 16-byte aligned: the copy below is one global_load_dwordx4 at any
+// element's address, where eight 2-byte loads per vector made an odd
+// vocabulary several times slower than an even one.
 template <class Tag>
-__device__ __forceinline__ uint4 load_raw(const typename Tag::S* row, int V, bool al16, int k,
-                                          int tid) {
+__device__ __forceinline__ uint4 load_raw(const typename Tag::S* row, int V, int k, int tid) {
   constexpr int VEC = Tag::VEC;
   const int e0 = (k * SNT + tid) * VEC;
-  if (al16 && e0 + VEC <= V) return *reinterpret_cast<const uint4*>(row + e0);
+  if (e0 + VEC <= V) {
+    uint4 v;
+    __builtin_memcpy(&v, row + e0, sizeof(v));
+    return v;
+  }
   uint32_t w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
   for (int i = 0; i < VEC; ++i) {
@@ -162,37 +170,40 @@ __device__ __forceinline__ void unpack_raw(const uint4& v, uint32_t (&u)[Tag::VE
   }
 }
 
-// f(k, e0, u, full) over the slabs of this lane, ten (f16: eight) slab loads
-// in flight at a time: a pass re-reads the row from memory, and each batch costs one
-// memory latency, so a 19-slab bf16 row of 151936 entries takes two per pass.
+// f(k, e0, u, full) over the slabs of this lane, ten (16-bit rows: eight) slab
+// loads in flight at a time: a pass re-reads the row from memory, and each
+// batch costs one memory latency, so a 19-slab bf16 row of 151936 entries
+// takes three per pass.
 // `full` is std::true_type for a slab that lies inside the row in every lane
 // (all but the last), so f's per-element bounds checks fold away there; the
-// row's last, partial slab gets std::false_type.
+// row's last, partial slab gets std::false_type.  Lanes that are not `active`
+// read nothing and skip f.
 template <class Tag, class F>
-__device__ __forceinline__ void for_slabs(const typename Tag::S* row, int V, bool al16, int nslab,
-                                          F&& f) {
+__device__ __forceinline__ void for_slabs(const typename Tag::S* row, int V, int nslab, F&& f,
+                                          bool active = true) {
   constexpr int VEC = Tag::VEC;
-  // f16's conversions need more registers per slab than bf16 or f32 shifts.
-  constexpr int UNR = std::is_same<Tag, TagF16>::value ? 8 : 10;
+  // 16-bit slabs unpack to twice the registers; ten in flight spill.
+  constexpr int UNR = VEC == 8 ? 8 : 10;
   const int tid = threadIdx.x;
   const int nfull = V / (SNT * VEC);
   for (int k0 = 0; k0 < nfull; k0 += UNR) {
     uint4 w[UNR];
 #pragma unroll
     for (int j = 0; j < UNR; ++j)
-      w[j] = (k0 + j < nfull) ? load_raw<Tag>(row, V, al16, k0 + j, tid) : make_uint4(0, 0, 0, 0);
+      w[j] = (active && k0 + j < nfull) ? load_raw<Tag>(row, V, k0 + j, tid)
+                                        : make_uint4(0, 0, 0, 0);
 #pragma unroll
     for (int j = 0; j < UNR; ++j) {
-      if (k0 + j < nfull) {
+      if (active && k0 + j < nfull) {
         uint32_t u[VEC];
         unpack_raw<Tag>(w[j], u);
         f(k0 + j, ((k0 + j) * SNT + tid) * VEC, u, std::true_type{});
       }
     }
   }
-  if (nfull < nslab) {
+  if (active && nfull < nslab) {
     uint32_t u[VEC];
-    unpack_raw<Tag>(load_raw<Tag>(row, V, al16, nfull, tid), u);
+    unpack_raw<Tag>(load_raw<Tag>(row, V, nfull, tid), u);
     f(nfull, (nfull * SNT + tid) * VEC, u, std::false_type{});
   }
 }
@@ -252,12 +263,12 @@ constexpr int TOPP_BINS = 4 * SNT;
 
 struct CandShared {
   int n;                          // entries gathered (may exceed KCAP: then unused)
-  int idx[KCAP];                  // vocabulary index: gathered, then dense candidates
+  alignas(16) int idx[KCAP];      // vocabulary index: gathered, then dense candidates
   uint32_t bits[KCAP];            // the entry as stored
-  int sidx[KCAP];                 // the gathered entries sorted by index
+  alignas(16) int sidx[KCAP];     // the gathered entries sorted by index
   uint32_t sbits[KCAP];
   unsigned long long mass[KCAP];  // top-p: fixed-point probability of candidate i
-  uint32_t key[KCAP];
+  alignas(16) uint32_t key[KCAP];
   int wave_cnt[SWAVES];
   double wave_sum[SWAVES];
   int found;                      // top-p threshold group
@@ -347,12 +358,12 @@ __device__ __forceinline__ int block_min_i32(int v) {
 // distribution without top-k / top-p), so the last positive element is V - 1
 // and is not tracked per element.
 template <class Tag, bool ALL_POSITIVE, class WFn, class TFn>
-__device__ __forceinline__ int vocab_search(const typename Tag::S* row, int V, bool al16,
-                                                  int nslab, WFn wfn, TFn tfn, SearchShared& sh) {
+__device__ __forceinline__ int vocab_search(const typename Tag::S* row, int V, int nslab,
+                                                  WFn wfn, TFn tfn, SearchShared& sh) {
   constexpr int VEC = Tag::VEC;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int last_pos = -1;
-  for_slabs<Tag>(row, V, al16, nslab, [&](int k, int e0, const uint32_t (&u)[VEC], auto full) {
+  for_slabs<Tag>(row, V, nslab, [&](int k, int e0, const uint32_t (&u)[VEC], auto full) {
     float facc = 0.0f;
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
@@ -398,7 +409,7 @@ __device__ __forceinline__ int vocab_search(const typename Tag::S* row, int V, b
 
   // Lane scan inside slab ks.
   uint32_t u[VEC];
-  unpack_raw<Tag>(load_raw<Tag>(row, V, al16, ks, tid), u);
+  unpack_raw<Tag>(load_raw<Tag>(row, V, ks, tid), u);
   const int e0 = (ks * SNT + tid) * VEC;
   float w8[VEC];
   float flw = 0.0f;
@@ -543,6 +554,25 @@ __device__ __forceinline__ bool mass_threshold(bool mine, uint32_t ck, unsigned 
   return true;
 }
 
+// How many of the n <= KCAP indices lie below this thread's (thread tid's
+// entry; meaningless past n).  Four indices per LDS read; the list is padded
+// to a multiple of four.
+__device__ __forceinline__ int rank_by_index(int* idx, int n) {
+  const int tid = threadIdx.x, n4 = (n + 3) >> 2;
+  if (tid >= n && tid < 4 * n4) idx[tid] = 0x7fffffff;
+  __syncthreads();
+  int rank = 0;
+  if (tid < n) {
+    const int e = idx[tid];
+    const int4* q = reinterpret_cast<const int4*>(idx);
+    for (int j = 0; j < n4; ++j) {
+      const int4 t = q[j];
+      rank += (t.x < e ? 1 : 0) + (t.y < e ? 1 : 0) + (t.z < e ? 1 : 0) + (t.w < e ? 1 : 0);
+    }
+  }
+  return rank;
+}
+
 template <class Tag>
 __device__ __forceinline__ void list_draw(CandShared& cs, float* sh_s, int n, uint32_t kth,
                                           int need_k, bool use_p, double top_p, float iT,
@@ -554,11 +584,9 @@ __device__ __forceinline__ void list_draw(CandShared& cs, float* sh_s, int n, ui
   // idx / bits in that order): an entry's rank is the number of smaller
   // indices.
   if (!sorted) {
+    const int rank = rank_by_index(cs.idx, n);
     if (tid < n) {
-      const int e = cs.idx[tid];
-      int rank = 0;
-      for (int j = 0; j < n; ++j) rank += cs.idx[j] < e ? 1 : 0;
-      cs.sidx[rank] = e;
+      cs.sidx[rank] = cs.idx[tid];
       cs.sbits[rank] = cs.bits[tid];
     }
     __syncthreads();
@@ -628,431 +656,6 @@ __device__ __forceinline__ void list_draw(CandShared& cs, float* sh_s, int n, ui
   __syncthreads();
 }
 
-// One row of the streaming path, by the whole workgroup (every thread calls
-// it): sample_kernel's body, and the register-resident top-k kernel's path
-// for a row whose candidate list overflows.  cs and hist: the caller's LDS.
-template <class Tag>
-__device__ __forceinline__ void sample_row(const SampleArgs& a, const int64_t r, CandShared& cs,
-                                           uint32_t* hist) {
-  using S = typename Tag::S;
-  constexpr int VEC = Tag::VEC;
-  constexpr int KB = Bits<Tag>::KB;
-  __shared__ SearchShared sh;
-  __shared__ unsigned long long histm[256];
-  __shared__ float sh_s[2 * SWAVES];
-  __shared__ float sh_x[SWAVES];
-  __shared__ int sh_e[SWAVES];
-  __shared__ uint32_t sh_digit;
-  __shared__ int sh_found;
-  __shared__ unsigned long long sh_above;
-
-  const S* row = static_cast<const S*>(a.logits) + r * a.stride;
-  const int V = (int)a.V;  // at most SNT * VEC * MAX_SLABS (checked on the host)
-  const bool al16 = (reinterpret_cast<uintptr_t>(row) & 15u) == 0;
-  const int nslab = (V + SNT * VEC - 1) / (SNT * VEC);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // x / T as x * (1/T): within an ulp of the division, and one multiply in
-  // the per-element work (the sampler is bound by its VALU issue rate).
-  const float iT = 1.0f / a.temp;
-
-  // 1. Per lane: the first maximum of the logits and its index, and the sum
-  // of exp((x - max) / T) over the lane's other entries.  A lane walks its
-  // slabs in increasing index order and keeps the first of equal maxima
-  // (strict >); fmaxf skips NaN, so NaN never wins, while NaN and +inf reach
-  // the sum (2^NaN, 2^(inf - inf)) and are caught there.  The maximum's own
-  // term (exactly 1) is kept out of the sum and added back per lane below, so
-  // S_other of the greedy token needs no subtraction and no second pass.
-  const float c2 = iT * kLog2e;  // exp(y / T) = 2^(y * c2)
-  float bx = -__builtin_huge_valf();
-  int bi32 = 0x7fffffff;
-  float sx = 0.0f;
-  for_slabs<Tag>(row, V, al16, nslab, [&](int, int e0, const uint32_t (&u)[VEC], auto full) {
-    float v[VEC];
-#pragma unroll
-    for (int i = 0; i < VEC; ++i)
-      v[i] = (full || e0 + i < V) ? Bits<Tag>::val(u[i]) : -__builtin_huge_valf();
-    float mc = v[0];
-#pragma unroll
-    for (int i = 1; i < VEC; ++i) mc = fmaxf(mc, v[i]);
-    int ic = VEC - 1;
-#pragma unroll
-    for (int i = VEC - 2; i >= 0; --i) ic = (v[i] == mc) ? i : ic;
-    const bool up = mc > bx;
-    const int skip = up ? ic : -1;  // the new maximum's own term stays out
-    const float mn = fmaxf(bx, mc);
-    const float mg = fmaxf(mn, -__FLT_MAX__);
-    float es = 0.0f;
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) es += (i == skip) ? 0.0f : exp2_hw((v[i] - mg) * c2);
-    // A replaced maximum joins the other entries with its term 1.
-    const float old_term = (up && bx > -__builtin_huge_valf()) ? 1.0f : 0.0f;
-    sx = __builtin_fmaf(sx + old_term, exp2_hw((bx - mg) * c2), es);
-    bi32 = up ? e0 + ic : bi32;
-    bx = mn;
-  });
-  const float lane_max = bx;
-  const int lane_arg = bi32;
-  int bi = bi32;
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ox = __shfl_xor(bx, o, 64);
-    const int oi = __shfl_xor(bi, o, 64);
-    argmax_merge(bx, bi, ox, oi);
-  }
-  if (lane == 0) {
-    sh_x[wave] = bx;
-    sh_e[wave] = bi;
-  }
-  __syncthreads();
-  bx = sh_x[0];
-  bi = sh_e[0];
-  for (int w = 1; w < SWAVES; ++w) argmax_merge(bx, bi, sh_x[w], sh_e[w]);
-  __syncthreads();
-  // Row totals relative to the row maximum: every entry (Z without top-k),
-  // and every entry but the argmax (the greedy token's S_other).
-  float tot[2];
-  {
-    const float own = lane_max > -__builtin_huge_valf() ? 1.0f : 0.0f;
-    const float f = bx > -__builtin_huge_valf() ? exp2_hw((lane_max - bx) * c2) : 0.0f;
-    tot[0] = (sx + own) * f;
-    tot[1] = (sx + (lane_arg == bi ? 0.0f : own)) * f;
-  }
-  block_sum<SNT, 2, float>(tot, sh_s);
-  const float os = tot[0], s_arg_other = tot[1];
-  const bool row_bad = bx == -__builtin_huge_valf() || bi >= V || os != os ||
-                       __builtin_fabsf(bx * iT) == __builtin_huge_valf();
-  if (row_bad) {
-    int tok_bad = bi < V ? bi : 0;
-    if (a.greedy && os != os) {
-      // Greedy decoding is torch.argmax, which ranks NaN above every number:
-      // the row's first NaN is its token.
-      int fn = 0x7fffffff;
-      for_slabs<Tag>(row, V, al16, nslab, [&](int, int e0, const uint32_t (&u)[VEC], auto full) {
-#pragma unroll
-        for (int i = VEC - 1; i >= 0; --i) {
-          const float v = Bits<Tag>::val(u[i]);
-          if ((full || e0 + i < V) && v != v) fn = min(fn, e0 + i);
-        }
-      });
-      fn = block_min_i32(fn);
-      if (fn < V) tok_bad = fn;
-    }
-    if (tid == 0) {
-      raise_flag(a.status, RRL_FLAG_BAD_PROBS);
-      a.token[r] = tok_bad;
-      a.logp[r] = __builtin_nanf("");
-      if (a.logq) a.logq[r] = __builtin_nanf("");
-    }
-    return;
-  }
-  const float m = bx * iT;  // max of x / T (scaling by 1/T > 0 is monotone)
-
-  int tok = bi;
-  float logq = 0.0f;
-  float s_other = s_arg_other;  // the argmax's; replaced below for another token
-  if (!a.greedy) {
-    // 2. top-k candidates: the k-th largest key by an MSB-first radix select.
-    const bool use_k = a.top_k > 0 && a.top_k < V;
-    uint32_t kth = 0;
-    int need_k = 0, cnt_k = 0;
-    int cut_k = -1;
-    bool listed = false;  // the top-k candidates sit in LDS (cs), in index order
-    if (use_k) {
-      uint32_t prefix = 0, pmask = 0;
-      int kk = (int)a.top_k;
-      for (int shift = KB - 8; shift >= 0; shift -= 8) {
-        for (int i = tid; i < 256; i += SNT) hist[i] = 0;
-        __syncthreads();
-        for_slabs<Tag>(row, V, al16, nslab, [&](int, int e0, const uint32_t (&u)[VEC], auto full) {
-#pragma unroll
-          for (int i = 0; i < VEC; ++i) {
-            const uint32_t key = float_key<KB>(u[i]);
-            if ((full || e0 + i < V) && (key & pmask) == prefix)
-              atomicAdd(&hist[(key >> shift) & 255u], 1u);
-          }
-        });
-        __syncthreads();
-        if (wave == 0) {
-          // lane l owns bins 4l..4l+3; counts above a bin = suffix sums.
-          uint32_t c[4];
-          for (int b = 0; b < 4; ++b) c[b] = hist[4 * lane + b];
-          const uint32_t t = c[0] + c[1] + c[2] + c[3];
-          uint32_t incl = t;
-          for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t y = __shfl_down(incl, o, 64);
-            if (lane + o < 64) incl += y;
-          }
-          uint32_t above = incl - t;
-          for (int b = 3; b >= 0; --b) {
-            if (above < (uint32_t)kk && (uint32_t)kk <= above + c[b]) {
-              sh_digit = 4 * lane + b;
-              sh_above = above;
-            }
-            above += c[b];
-          }
-        }
-        __syncthreads();
-        const uint32_t d = sh_digit;
-        kk -= (int)sh_above;
-        prefix |= d << shift;
-        pmask |= 255u << shift;
-        cnt_k = (int)hist[d];
-        __syncthreads();
-      }
-      kth = prefix;
-      need_k = kk;  // 1 <= need_k <= cnt_k tokens at the threshold are kept
-      // Gather every entry at or above the k-th key (k - need_k + cnt_k of
-      // them) into LDS: the rest of the draw then never re-reads the row.
-      if (a.top_k <= KCAP) {
-        if (tid == 0) cs.n = 0;
-        __syncthreads();
-        for_slabs<Tag>(row, V, al16, nslab, [&](int, int e0, const uint32_t (&u)[VEC], auto full) {
-#pragma unroll
-          for (int i = 0; i < VEC; ++i) {
-            if ((full || e0 + i < V) && float_key<KB>(u[i]) >= kth) {
-              const int p = atomicAdd(&cs.n, 1);
-              if (p < KCAP) {
-                cs.idx[p] = e0 + i;
-                cs.bits[p] = u[i];
-              }
-            }
-          }
-        });
-        __syncthreads();
-        listed = cs.n <= KCAP;
-      }
-      if (!listed && need_k < cnt_k) {
-        const double nth = (double)(need_k - 1);
-        cut_k = vocab_search<Tag, false>(
-            row, V, al16, nslab,
-            [&](int, uint32_t b) { return float_key<KB>(b) == kth ? 1.0f : 0.0f; },
-            [&](double) { return nth; }, sh);
-      }
-    }
-    const bool use_p = a.top_p > 0.0 && a.top_p < 1.0;
-    uint32_t c[4] = {(uint32_t)r, (uint32_t)((uint64_t)r >> 32), (uint32_t)a.offset,
-                     (uint32_t)(a.offset >> 32)};
-    philox4x32_10(c, (uint32_t)a.seed, (uint32_t)(a.seed >> 32));
-    const double u01 = (double)(c[0] >> 8) * 5.9604644775390625e-8;  // 2^-24
-
-    if (listed) {
-      uint32_t tok_bits;
-      list_draw<Tag>(cs, sh_s, cs.n, kth, need_k, use_p, a.top_p, iT, m,
-                     float_key<KB>(load_one<Tag>(row, bi)), u01, tok, logq, tok_bits);
-    } else {
-      auto cand = [&](int e, uint32_t key) {
-        return !use_k || key > kth || (key == kth && (need_k >= cnt_k || e <= cut_k));
-      };
-
-      // 3. Z over the candidates (the whole row's online sum without top-k).
-      float zs = os;  // relative to the row maximum
-      if (use_k) {
-        zs = 0.0f;
-        for_slabs<Tag>(row, V, al16, nslab, [&](int, int e0, const uint32_t (&u)[VEC], auto full) {
-#pragma unroll
-          for (int i = 0; i < VEC; ++i) {
-            if ((full || e0 + i < V) && cand(e0 + i, float_key<KB>(u[i])))
-              zs += expf(Bits<Tag>::val(u[i]) * iT - m);
-          }
-        });
-        float v1[1] = {zs};
-        block_sum<SNT, 1, float>(v1, sh_s);
-        zs = v1[0];
-      }
-      const float inv_z = 1.0f / zs;
-      auto ex = [&](uint32_t b) {
-        float e = expf(Bits<Tag>::val(b) * iT - m);
-        asm volatile("" : "+v"(e));
-        return e;
-      };
-      auto prob = [&](uint32_t b) { return ex(b) * inv_z; };
-
-      // 4. top-p: radix select over fixed-point mass in descending key order.
-      bool p_found = false;
-      uint32_t pth = 0;
-      unsigned long long n_keep = 0, cnt_p = 0;
-      int cut_p = -1;
-      if (use_p) {
-        const unsigned long long P = (unsigned long long)(a.top_p * kMassScale);
-        uint32_t prefix = 0, pmask = 0;
-        unsigned long long A = 0;
-        p_found = true;
-        for (int shift = KB - 8; shift >= 0; shift -= 8) {
-          for (int i = tid; i < 256; i += SNT) {
-            hist[i] = 0;
-            histm[i] = 0;
-          }
-          if (tid == 0) sh_found = 0;
-          __syncthreads();
-          for_slabs<Tag>(row, V, al16, nslab, [&](int, int e0, const uint32_t (&u)[VEC], auto full) {
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) {
-              const uint32_t key = float_key<KB>(u[i]);
-              if ((full || e0 + i < V) && (key & pmask) == prefix && cand(e0 + i, key)) {
-                const unsigned long long fx =
-                    (unsigned long long)((double)prob(u[i]) * kMassScale);
-                atomicAdd(&hist[(key >> shift) & 255u], 1u);
-                atomicAdd(&histm[(key >> shift) & 255u], fx);
-              }
-            }
-          });
-          __syncthreads();
-          if (wave == 0) {
-            unsigned long long c[4];
-            for (int b = 0; b < 4; ++b) c[b] = histm[4 * lane + b];
-            const unsigned long long t = c[0] + c[1] + c[2] + c[3];
-            unsigned long long incl = t;
-            for (int o = 1; o < 64; o <<= 1) {
-              const unsigned long long y = __shfl_down(incl, o, 64);
-              if (lane + o < 64) incl += y;
-            }
-            unsigned long long above = A + (incl - t);
-            for (int b = 3; b >= 0; --b) {
-              // the bin holding the first token whose inclusive mass passes P
-              if (c[b] > 0 && above <= P && P < above + c[b]) {
-                sh_digit = 4 * lane + b;
-                sh_above = above;
-                sh_found = 1;
-              }
-              above += c[b];
-            }
-          }
-          __syncthreads();
-          const bool f = sh_found != 0;
-          const uint32_t d = sh_digit;
-          const unsigned long long ab = sh_above;
-          const unsigned long long binm = histm[d], binc = hist[d];
-          __syncthreads();
-          if (!f) {  // every candidate fits under top_p
-            p_found = false;
-            break;
-          }
-          A = ab;
-          prefix |= d << shift;
-          pmask |= 255u << shift;
-          cnt_p = binc;
-          if (shift == 0) {
-            const unsigned long long each = binm / binc;  // equal keys, equal mass
-            n_keep = each > 0 ? (P - A) / each : binc;
-          }
-        }
-        if (p_found) {
-          pth = prefix;
-          // The first token in descending order (the row maximum) is always kept.
-          if (pth == float_key<KB>(load_one<Tag>(row, bi)) && n_keep == 0) n_keep = 1;
-          if (n_keep > 0 && n_keep < cnt_p) {
-            const double nth = (double)(n_keep - 1);
-            cut_p = vocab_search<Tag, false>(
-                row, V, al16, nslab,
-                [&](int e, uint32_t b) {
-                  const uint32_t key = float_key<KB>(b);
-                  return (key == pth && cand(e, key)) ? 1.0f : 0.0f;
-                },
-                [&](double) { return nth; }, sh);
-          }
-        }
-      }
-      auto kept = [&](int e, uint32_t key) {
-        return !p_found || key > pth ||
-               (key == pth && (n_keep >= cnt_p || (n_keep > 0 && e <= cut_p)));
-      };
-      // q weight of a top-k candidate, floored; 0 outside the candidates
-      auto qw = [&](int e, uint32_t b) {
-        const uint32_t key = float_key<KB>(b);
-        return cand(e, key) ? fmaxf(kept(e, key) ? ex(b) * inv_z : 0.0f, 1e-9f) : 0.0f;
-      };
-
-      // 5. inverse CDF with this row's uniform.
-      __shared__ double sh_total;
-      auto target = [&](double total) {
-        if (tid == 0) sh_total = total;
-        return u01 * total;
-      };
-      auto draw = [&](auto wfn, auto all_positive) {
-        tok = vocab_search<Tag, decltype(all_positive)::value>(row, V, al16, nslab, wfn, target,
-                                                               sh);
-        const double qtot = sh_total;
-        __syncthreads();
-        if (tok < 0 || tok >= V) tok = bi;  // no positive weight: cannot happen, q >= 1e-9
-        if (tid == 0) logq = (float)(log((double)wfn(tok, load_one<Tag>(row, tok))) - log(qtot));
-      };
-      if (!use_k && !p_found) {
-        // The floored softmax max(p, 1e-9) as sample_resident_kernel's
-        // mixture: p with probability 1 / (1 + G), else the floor's excess
-        // g = max(1e-9 - p, 0), chosen by the component uniform u1; G takes
-        // a pass of its own only when u1 < V * 1e-9 (>= G / (1 + G)) or
-        // log q is asked for.
-        const float lz = log2f(zs);
-        auto rho_of = [&](uint32_t b) {
-          return exp2_hw(__builtin_fmaf(Bits<Tag>::val(b) - bx, c2, -lz));
-        };
-        const double u1 = (double)(((uint64_t)c[1] << 21) | (c[2] >> 11)) * 0x1p-53;
-        const bool near = u1 < (double)V * 1.001e-9;
-        double G = 0.0;
-        if (a.logq || near) {
-          float gs = 0.0f;
-          for_slabs<Tag>(row, V, al16, nslab, [&](int, int e0, const uint32_t (&u)[VEC], auto full) {
-#pragma unroll
-            for (int i = 0; i < VEC; ++i)
-              if (full || e0 + i < V) gs += fmaxf(1e-9f - rho_of(u[i]), 0.0f);
-          });
-          double t[1] = {(double)gs};
-          block_sum<SNT, 1, double>(t, sh.wave_tot);
-          G = t[0];
-        }
-        const bool use_g = near && u1 < G / (1.0 + G);
-        tok = vocab_search<Tag, false>(
-            row, V, al16, nslab,
-            [&](int, uint32_t b) {
-              const float p = rho_of(b);
-              return use_g ? fmaxf(1e-9f - p, 0.0f) : p;
-            },
-            target, sh);
-        __syncthreads();
-        if (tok < 0 || tok >= V) tok = bi;  // no positive weight: cannot happen with p
-        if (tid == 0 && a.logq)
-          logq = (float)(log((double)fmaxf(rho_of(load_one<Tag>(row, tok)), 1e-9f)) - log1p(G));
-      } else {
-        draw(qw, std::false_type{});
-      }
-    }
-    // The token's S_other from pass 1: the sum without the maximum when the
-    // token is the argmax, else Z minus the token's own term.  S_other then
-    // holds the maximum's term 1 and e_tok <= 1, so the difference loses at
-    // most one bit.
-    if (tok != bi)
-      s_other = os - exp2_hw((Bits<Tag>::val(load_one<Tag>(row, tok)) - bx) * c2);
-  }
-
-  // 6. log_softmax(x / T) at the token, as the training row kernels form it:
-  // finish_row of the maximum, the sum over the other columns and the
-  // token's own value.
-  if (tid == 0) {
-    const float xt = Bits<Tag>::val(load_one<Tag>(row, tok)) * iT;
-    const RowLogprob<float> fr = finish_row<float>(m, s_other, xt);
-    a.token[r] = tok;
-    a.logp[r] = fr.logp;
-    if (a.logq) a.logq[r] = logq;
-  }
-}
-
-template <class Tag>
-__global__ __launch_bounds__(SNT) void sample_kernel(SampleArgs a) {
-  __shared__ CandShared cs;
-  __shared__ uint32_t hist[256];
-  const int64_t r = blockIdx.x;
-  if (r >= a.B) return;
-  // A fill-in launch redoes the rows the register-resident nucleus path
-  // handed over (token slot -1); the others return at once.
-  if (a.fill_in && __builtin_nontemporal_load(&a.token[r]) != -1) return;
-  sample_row<Tag>(a, r, cs, hist);
-}
-
-template <class Tag>
-int launch_sample(const SampleArgs& a, hipStream_t st) {
-  hipLaunchKernelGGL((sample_kernel<Tag>), dim3((unsigned)a.B), dim3(SNT), 0, st, a);
-  return check_launch("sample_kernel");
-}
-
 // ---------------------------------------------------------------------------
 // Register-resident rows of 16-bit logits made of whole 16-byte vectors
 // (V % 8 == 0, rows 16-byte aligned, V <= 8 * 1024 * RES_MAX_SLABS).  Lane j
@@ -1118,18 +721,17 @@ __device__ __forceinline__ float sum8(const float (&e)[8]) {
   return ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
 }
 
-// The k-th largest of NK 16-bit keys per thread (keys whose valid flag is
+// The k-th largest of NK KB-bit keys per thread (keys whose valid flag is
 // false take no part; 1 <= k <= the number of valid keys): MSB-first radix
 // select, 8 bits per pass, over an LDS histogram of 256 bins.
-template <int NK>
-__device__ __forceinline__ uint32_t block_kth_keys16(const uint32_t (&key)[NK],
-                                                     const bool (&valid)[NK], int k,
-                                                     uint32_t* hist, uint32_t* sh_digit,
-                                                     uint32_t* sh_above) {
+template <int KB, int NK>
+__device__ __forceinline__ uint32_t block_kth_keys(const uint32_t (&key)[NK],
+                                                   const bool (&valid)[NK], int k, uint32_t* hist,
+                                                   uint32_t* sh_digit, uint32_t* sh_above) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   uint32_t prefix = 0, pmask = 0;
   uint32_t kk = (uint32_t)k;
-  for (int shift = 8; shift >= 0; shift -= 8) {
+  for (int shift = KB - 8; shift >= 0; shift -= 8) {
     if (tid < 256) hist[tid] = 0;
     __syncthreads();
 #pragma unroll
@@ -1164,12 +766,12 @@ __device__ __forceinline__ uint32_t block_kth_keys16(const uint32_t (&key)[NK],
   }
   return prefix;
 }
-__device__ __forceinline__ uint32_t block_kth_key16(uint32_t key, bool valid, int k,
-                                                    uint32_t* hist, uint32_t* sh_digit,
-                                                    uint32_t* sh_above) {
+template <int KB>
+__device__ __forceinline__ uint32_t block_kth_key(uint32_t key, bool valid, int k, uint32_t* hist,
+                                                  uint32_t* sh_digit, uint32_t* sh_above) {
   const uint32_t ks[1] = {key};
   const bool vs[1] = {valid};
-  return block_kth_keys16<1>(ks, vs, k, hist, sh_digit, sh_above);
+  return block_kth_keys<KB, 1>(ks, vs, k, hist, sh_digit, sh_above);
 }
 
 // A value known to be the same in every active lane, moved to scalar
@@ -1412,6 +1014,634 @@ __device__ __forceinline__ void small_list_draw(CandShared& cs, SmallShared& ss,
   tok_bits = ss.bits;
 }
 
+// Lane maxima at or above the nucleus list's threshold: of 1024 lanes, 448
+// leave a list of about 590 entries of the 1024 that fit.
+constexpr int NUC_NUM = 7, NUC_DEN = 16;
+
+// Top-p without top-k from a list: cs holds n <= KCAP entries, every entry of
+// the row at or above some key.  If the nucleus ends inside the list (its
+// mass passes top_p there), the kept entries are all on it, every other entry
+// of the row weighs the floor 1e-9, and the draw needs no further pass: the
+// cumulative weight up to the kept entry at index e, the i-th in order, is
+// the kept weights' prefix plus (e - i) floors, and a target between two kept
+// entries names the floor entry by its distance.  The rules (exact
+// fixed-point masses, ties lowest index first, the row maximum always kept)
+// are the row passes' below.  Returns false, for every thread, when the list
+// ends first.
+template <class Tag>
+__device__ __forceinline__ bool nucleus_list_draw(CandShared& cs, int n, int V, double top_p,
+                                                  float iT, float m, float inv_z,
+                                                  uint32_t max_key, double u01, int& tok,
+                                                  float& logq) {
+  constexpr int KB = Bits<Tag>::KB;
+  const int tid = threadIdx.x;
+  const bool have = tid < n;
+  const int e = have ? cs.idx[tid] : 0;
+  const uint32_t b = have ? cs.bits[tid] : 0u;
+  const uint32_t ck = float_key<KB>(b);
+  const float pc = have ? expf(Bits<Tag>::val(b) * iT - m) * inv_z : 0.0f;
+  const unsigned long long P = (unsigned long long)(top_p * kMassScale);
+  const unsigned long long ms = have ? (unsigned long long)((double)pc * kMassScale) : 0ull;
+  if (!mass_threshold<KB>(have, ck, ms, P, cs)) return false;
+  const uint32_t pth = cs.pth;
+  const unsigned long long A0 = cs.A, C0 = (unsigned long long)cs.C;
+  const unsigned long long each = cs.M / C0;  // equal keys, equal mass
+  unsigned long long n_keep = each > 0 ? (P - A0) / each : C0;
+  if (pth == max_key && n_keep == 0) n_keep = 1;
+  const bool tie = have && ck == pth;
+  bool keep = have && (ck > pth || (tie && n_keep >= C0));
+  if (n_keep > 0 && n_keep < C0) {  // uniform: rank the ties among themselves
+    int* tied = reinterpret_cast<int*>(cs.key);
+    int nt = 0;
+    const int tp = block_excl_count(tie, cs.wave_cnt, nt);
+    if (tie) tied[tp] = e;
+    if (tid >= nt && tid < ((nt + 3) & ~3)) tied[tid] = 0x7fffffff;
+    __syncthreads();
+    if (tie) {
+      unsigned long long before = 0;
+      const int4* q = reinterpret_cast<const int4*>(tied);
+      for (int j = 0; j < (nt + 3) >> 2; ++j) {
+        const int4 t = q[j];
+        before += (t.x < e ? 1 : 0) + (t.y < e ? 1 : 0) + (t.z < e ? 1 : 0) + (t.w < e ? 1 : 0);
+      }
+      keep = before < n_keep;
+    }
+  }
+  // The kept entries in index order.
+  int nk = 0;
+  const int pos = block_excl_count(keep, cs.wave_cnt, nk);
+  if (keep) {
+    cs.sidx[pos] = e;
+    cs.sbits[pos] = b;
+  }
+  __syncthreads();
+  const int rank = rank_by_index(cs.sidx, nk);
+  if (tid < nk) {
+    cs.idx[rank] = cs.sidx[tid];
+    cs.bits[rank] = cs.sbits[tid];
+  }
+  __syncthreads();
+  const bool mine = tid < nk;
+  const int ei = mine ? cs.idx[tid] : V;
+  const int ep = mine && tid > 0 ? cs.idx[tid - 1] : -1;
+  const float wf =
+      mine ? fmaxf(expf(Bits<Tag>::val(cs.bits[tid]) * iT - m) * inv_z, 1e-9f) : 0.0f;
+  double incl, excl, tot;
+  block_scan_d((double)wf, cs.wave_sum, incl, excl, tot);
+  const double fl = (double)1e-9f;
+  const double total = tot + (double)(V - nk) * fl;
+  const double target = u01 * total;
+  // [lo, hi) of consecutive kept entries tile [0, the last one's hi): excl is
+  // the previous thread's incl itself.
+  const double lo = tid > 0 ? excl + (double)(ep - (tid - 1)) * fl : 0.0;
+  const double at = excl + (double)(ei - tid) * fl;
+  const double hi = incl + (double)(ei - tid) * fl;
+  const bool last = tid == nk - 1;
+  if (mine && lo <= target && (target < hi || last)) {
+    int t = ei;
+    float w = wf;
+    if (target < at) {  // a floor entry before this one
+      const int j = (int)((target - lo) / fl);
+      t = min(ep + 1 + j, ei - 1);
+      w = 1e-9f;
+    } else if (target >= hi && ei + 1 < V) {  // one after the last
+      const double j = (target - hi) / fl;
+      t = j < (double)(V - 1 - ei) ? ei + 1 + (int)j : V - 1;
+      w = 1e-9f;
+    }
+    cs.pick = t;
+    cs.logq = (float)(log((double)w) - log(total));
+  }
+  __syncthreads();
+  tok = cs.pick;
+  logq = cs.logq;
+  __syncthreads();
+  return true;
+}
+
+// One row of the streaming path, by the whole workgroup (every thread calls
+// it): sample_kernel's body, and the register-resident top-k kernel's path
+// for a row whose candidate list overflows.  cs, ss and hist: the caller's
+// LDS.  LIST: top-k and top-p try a candidate list from the lane maxima first
+// (the resident kernel has tried already).
+//
+// Reading the row bounds it, once per pass: a radix select over the row costs
+// four passes of float32 keys for top-k and four more, with exponentials and
+// 64-bit atomics, for top-p.  The list costs one pass, by the lanes whose
+// maximum reaches its threshold alone.  Before -> with the list, us for 256
+// rows of 151936 float32 entries: top-k 50 with top-p 0.9 177 -> 51, top-p 0.9
+// 255 -> 66; for 64 rows of 50257 bf16 entries (read by vectors now, too)
+// 88 -> 24 and 139 -> 32, the defaults 57 -> 25.
+template <class Tag, bool LIST>
+__device__ __forceinline__ void sample_row(const SampleArgs& a, const int64_t r, CandShared& cs,
+                                           SmallShared& ss, uint32_t* hist) {
+  using S = typename Tag::S;
+  constexpr int VEC = Tag::VEC;
+  constexpr int KB = Bits<Tag>::KB;
+  __shared__ SearchShared sh;
+  __shared__ unsigned long long histm[256];
+  __shared__ float sh_s[2 * SWAVES];
+  __shared__ float sh_x[SWAVES];
+  __shared__ int sh_e[SWAVES];
+  __shared__ uint32_t sh_digit;
+  __shared__ int sh_found;
+  __shared__ unsigned long long sh_above;
+  __shared__ uint32_t sh_above32;
+
+  const S* row = static_cast<const S*>(a.logits) + r * a.stride;
+  const int V = (int)a.V;  // at most SNT * VEC * MAX_SLABS (checked on the host)
+  const int nslab = (V + SNT * VEC - 1) / (SNT * VEC);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // x / T as x * (1/T): within an ulp of the division, and one multiply in
+  // the per-element work (the sampler is bound by its VALU issue rate).
+  const float iT = 1.0f / a.temp;
+
+  // 1. Per lane: the first maximum of the logits and its index, and the sum
+  // of exp((x - max) / T) over the lane's other entries.  A lane walks its
+  // slabs in increasing index order and keeps the first of equal maxima
+  // (strict >); fmaxf skips NaN, so NaN never wins, while NaN and +inf reach
+  // the sum (2^NaN, 2^(inf - inf)) and are caught there.  The maximum's own
+  // term (exactly 1) is kept out of the sum and added back per lane below, so
+  // S_other of the greedy token needs no subtraction and no second pass.
+  const float c2 = iT * kLog2e;  // exp(y / T) = 2^(y * c2)
+  float bx = -__builtin_huge_valf();
+  int bi32 = 0x7fffffff;
+  float sx = 0.0f;
+  for_slabs<Tag>(row, V, nslab, [&](int, int e0, const uint32_t (&u)[VEC], auto full) {
+    float v[VEC];
+#pragma unroll
+    for (int i = 0; i < VEC; ++i)
+      v[i] = (full || e0 + i < V) ? Bits<Tag>::val(u[i]) : -__builtin_huge_valf();
+    float mc = v[0];
+#pragma unroll
+    for (int i = 1; i < VEC; ++i) mc = fmaxf(mc, v[i]);
+    int ic = VEC - 1;
+#pragma unroll
+    for (int i = VEC - 2; i >= 0; --i) ic = (v[i] == mc) ? i : ic;
+    const bool up = mc > bx;
+    const int skip = up ? ic : -1;  // the new maximum's own term stays out
+    const float mn = fmaxf(bx, mc);
+    const float mg = fmaxf(mn, -__FLT_MAX__);
+    float es = 0.0f;
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) es += (i == skip) ? 0.0f : exp2_hw((v[i] - mg) * c2);
+    // A replaced maximum joins the other entries with its term 1.
+    const float old_term = (up && bx > -__builtin_huge_valf()) ? 1.0f : 0.0f;
+    sx = __builtin_fmaf(sx + old_term, exp2_hw((bx - mg) * c2), es);
+    bi32 = up ? e0 + ic : bi32;
+    bx = mn;
+  });
+  const float lane_max = bx;
+  const int lane_arg = bi32;
+  int bi = bi32;
+  for (int o = 32; o > 0; o >>= 1) {
+    const float ox = __shfl_xor(bx, o, 64);
+    const int oi = __shfl_xor(bi, o, 64);
+    argmax_merge(bx, bi, ox, oi);
+  }
+  if (lane == 0) {
+    sh_x[wave] = bx;
+    sh_e[wave] = bi;
+  }
+  __syncthreads();
+  bx = sh_x[0];
+  bi = sh_e[0];
+  for (int w = 1; w < SWAVES; ++w) argmax_merge(bx, bi, sh_x[w], sh_e[w]);
+  __syncthreads();
+  // Row totals relative to the row maximum: every entry (Z without top-k),
+  // and every entry but the argmax (the greedy token's S_other).
+  float tot[2];
+  {
+    const float own = lane_max > -__builtin_huge_valf() ? 1.0f : 0.0f;
+    const float f = bx > -__builtin_huge_valf() ? exp2_hw((lane_max - bx) * c2) : 0.0f;
+    tot[0] = (sx + own) * f;
+    tot[1] = (sx + (lane_arg == bi ? 0.0f : own)) * f;
+  }
+  block_sum<SNT, 2, float>(tot, sh_s);
+  const float os = tot[0], s_arg_other = tot[1];
+  const bool row_bad = bx == -__builtin_huge_valf() || bi >= V || os != os ||
+                       __builtin_fabsf(bx * iT) == __builtin_huge_valf();
+  if (row_bad) {
+    int tok_bad = bi < V ? bi : 0;
+    if (a.greedy && os != os) {
+      // Greedy decoding is torch.argmax, which ranks NaN above every number:
+      // the row's first NaN is its token.
+      int fn = 0x7fffffff;
+      for_slabs<Tag>(row, V, nslab, [&](int, int e0, const uint32_t (&u)[VEC], auto full) {
+#pragma unroll
+        for (int i = VEC - 1; i >= 0; --i) {
+          const float v = Bits<Tag>::val(u[i]);
+          if ((full || e0 + i < V) && v != v) fn = min(fn, e0 + i);
+        }
+      });
+      fn = block_min_i32(fn);
+      if (fn < V) tok_bad = fn;
+    }
+    if (tid == 0) {
+      raise_flag(a.status, RRL_FLAG_BAD_PROBS);
+      a.token[r] = tok_bad;
+      a.logp[r] = __builtin_nanf("");
+      if (a.logq) a.logq[r] = __builtin_nanf("");
+    }
+    return;
+  }
+  const float m = bx * iT;  // max of x / T (scaling by 1/T > 0 is monotone)
+
+  int tok = bi;
+  float logq = 0.0f;
+  float s_other = s_arg_other;  // the argmax's; replaced below for another token
+  if (!a.greedy) {
+    const bool use_k = a.top_k > 0 && a.top_k < V;
+    const bool use_p = a.top_p > 0.0 && a.top_p < 1.0;
+    uint32_t c[4] = {(uint32_t)r, (uint32_t)((uint64_t)r >> 32), (uint32_t)a.offset,
+                     (uint32_t)(a.offset >> 32)};
+    philox4x32_10(c, (uint32_t)a.seed, (uint32_t)(a.seed >> 32));
+    const double u01 = (double)(c[0] >> 8) * 5.9604644775390625e-8;  // 2^-24
+    const uint32_t max_key = float_key<KB>(load_one<Tag>(row, bi));
+    bool drawn = false;
+    if constexpr (LIST) {
+      // The kq-th largest lane maximum t0 has at least kq entries at or above
+      // it, so the entries at or above t0 hold the top kq and every tie.
+      const int nlanes = min(SNT, (V + VEC - 1) / VEC);
+      const int kq = use_k ? (int)min(a.top_k, (int64_t)SNT + 1)
+                           : (use_p ? max(1, nlanes * NUC_NUM / NUC_DEN) : SNT + 1);
+      if (kq <= nlanes) {
+        const uint32_t lkey = float_key<KB>(Bits<Tag>::bits_of(lane_max));
+        const bool in_row = tid < nlanes;
+        const uint32_t t0 = block_kth_key<KB>(lkey, in_row, kq, hist, &sh_digit, &sh_above32);
+        if (tid == 0) cs.n = 0;
+        __syncthreads();
+        for_slabs<Tag>(
+            row, V, nslab,
+            [&](int, int e0, const uint32_t (&u)[VEC], auto full) {
+#pragma unroll
+              for (int i = 0; i < VEC; ++i) {
+                if ((full || e0 + i < V) && float_key<KB>(u[i]) >= t0) {
+                  const int p = atomicAdd(&cs.n, 1);
+                  if (p < KCAP) {
+                    cs.idx[p] = e0 + i;
+                    cs.bits[p] = u[i];
+                  }
+                }
+              }
+            },
+            in_row && lkey >= t0);
+        __syncthreads();
+        const int n = cs.n;
+        uint32_t tok_bits;
+        if (n <= KCAP) {
+          if (!use_k) {
+            drawn = nucleus_list_draw<Tag>(cs, n, V, a.top_p, iT, m, 1.0f / os, max_key, u01, tok,
+                                           logq);
+          } else if (n <= 64) {
+            small_list_draw<Tag>(cs, ss, n, kq, use_p, a.top_p, iT, m, max_key, u01, tok, logq,
+                                 tok_bits);
+            drawn = true;
+          } else {
+            const bool mine = tid < n;
+            const uint32_t key = float_key<KB>(mine ? cs.bits[tid] : 0u);
+            const uint32_t kth = block_kth_key<KB>(key, mine, kq, hist, &sh_digit, &sh_above32);
+            int n_above = 0;
+            (void)block_excl_count(mine && key > kth, cs.wave_cnt, n_above);
+            list_draw<Tag>(cs, sh_s, n, kth, kq - n_above, use_p, a.top_p, iT, m, max_key, u01,
+                           tok, logq, tok_bits);
+            drawn = true;
+          }
+        }
+        __syncthreads();
+      }
+    }
+    if (!drawn) {
+    // 2. top-k candidates: the k-th largest key by an MSB-first radix select.
+    uint32_t kth = 0;
+    int need_k = 0, cnt_k = 0;
+    int cut_k = -1;
+    bool listed = false;  // the top-k candidates sit in LDS (cs), in index order
+    if (use_k) {
+      uint32_t prefix = 0, pmask = 0;
+      int kk = (int)a.top_k;
+      for (int shift = KB - 8; shift >= 0; shift -= 8) {
+        for (int i = tid; i < 256; i += SNT) hist[i] = 0;
+        __syncthreads();
+        for_slabs<Tag>(row, V, nslab, [&](int, int e0, const uint32_t (&u)[VEC], auto full) {
+#pragma unroll
+          for (int i = 0; i < VEC; ++i) {
+            const uint32_t key = float_key<KB>(u[i]);
+            if ((full || e0 + i < V) && (key & pmask) == prefix)
+              atomicAdd(&hist[(key >> shift) & 255u], 1u);
+          }
+        });
+        __syncthreads();
+        if (wave == 0) {
+          // lane l owns bins 4l..4l+3; counts above a bin = suffix sums.
+          uint32_t c[4];
+          for (int b = 0; b < 4; ++b) c[b] = hist[4 * lane + b];
+          const uint32_t t = c[0] + c[1] + c[2] + c[3];
+          uint32_t incl = t;
+          for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_down(incl, o, 64);
+            if (lane + o < 64) incl += y;
+          }
+          uint32_t above = incl - t;
+          for (int b = 3; b >= 0; --b) {
+            if (above < (uint32_t)kk && (uint32_t)kk <= above + c[b]) {
+              sh_digit = 4 * lane + b;
+              sh_above = above;
+            }
+            above += c[b];
+          }
+        }
+        __syncthreads();
+        const uint32_t d = sh_digit;
+        kk -= (int)sh_above;
+        prefix |= d << shift;
+        pmask |= 255u << shift;
+        cnt_k = (int)hist[d];
+        __syncthreads();
+      }
+      kth = prefix;
+      need_k = kk;  // 1 <= need_k <= cnt_k tokens at the threshold are kept
+      // Gather every entry at or above the k-th key (k - need_k + cnt_k of
+      // them) into LDS: the rest of the draw then never re-reads the row.
+      if (a.top_k <= KCAP) {
+        if (tid == 0) cs.n = 0;
+        __syncthreads();
+        for_slabs<Tag>(row, V, nslab, [&](int, int e0, const uint32_t (&u)[VEC], auto full) {
+#pragma unroll
+          for (int i = 0; i < VEC; ++i) {
+            if ((full || e0 + i < V) && float_key<KB>(u[i]) >= kth) {
+              const int p = atomicAdd(&cs.n, 1);
+              if (p < KCAP) {
+                cs.idx[p] = e0 + i;
+                cs.bits[p] = u[i];
+              }
+            }
+          }
+        });
+        __syncthreads();
+        listed = cs.n <= KCAP;
+      }
+      if (!listed && need_k < cnt_k) {
+        const double nth = (double)(need_k - 1);
+        cut_k = vocab_search<Tag, false>(
+            row, V, nslab,
+            [&](int, uint32_t b) { return float_key<KB>(b) == kth ? 1.0f : 0.0f; },
+            [&](double) { return nth; }, sh);
+      }
+    }
+    if (listed) {
+      uint32_t tok_bits;
+      list_draw<Tag>(cs, sh_s, cs.n, kth, need_k, use_p, a.top_p, iT, m,
+                     max_key, u01, tok, logq, tok_bits);
+    } else {
+      auto cand = [&](int e, uint32_t key) {
+        return !use_k || key > kth || (key == kth && (need_k >= cnt_k || e <= cut_k));
+      };
+
+      // 3. Z over the candidates (the whole row's online sum without top-k).
+      float zs = os;  // relative to the row maximum
+      if (use_k) {
+        zs = 0.0f;
+        for_slabs<Tag>(row, V, nslab, [&](int, int e0, const uint32_t (&u)[VEC], auto full) {
+#pragma unroll
+          for (int i = 0; i < VEC; ++i) {
+            if ((full || e0 + i < V) && cand(e0 + i, float_key<KB>(u[i])))
+              zs += expf(Bits<Tag>::val(u[i]) * iT - m);
+          }
+        });
+        float v1[1] = {zs};
+        block_sum<SNT, 1, float>(v1, sh_s);
+        zs = v1[0];
+      }
+      const float inv_z = 1.0f / zs;
+      auto ex = [&](uint32_t b) {
+        float e = expf(Bits<Tag>::val(b) * iT - m);
+        asm volatile("" : "+v"(e));
+        return e;
+      };
+      auto prob = [&](uint32_t b) { return ex(b) * inv_z; };
+
+      // 4. top-p: radix select over fixed-point mass in descending key order.
+      bool p_found = false;
+      uint32_t pth = 0;
+      unsigned long long n_keep = 0, cnt_p = 0;
+      int cut_p = -1;
+      if (use_p) {
+        const unsigned long long P = (unsigned long long)(a.top_p * kMassScale);
+        uint32_t prefix = 0, pmask = 0;
+        unsigned long long A = 0;
+        p_found = true;
+        for (int shift = KB - 8; shift >= 0; shift -= 8) {
+          for (int i = tid; i < 256; i += SNT) {
+            hist[i] = 0;
+            histm[i] = 0;
+          }
+          if (tid == 0) sh_found = 0;
+          __syncthreads();
+          for_slabs<Tag>(row, V, nslab, [&](int, int e0, const uint32_t (&u)[VEC], auto full) {
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) {
+              const uint32_t key = float_key<KB>(u[i]);
+              if ((full || e0 + i < V) && (key & pmask) == prefix && cand(e0 + i, key)) {
+                const unsigned long long fx =
+                    (unsigned long long)((double)prob(u[i]) * kMassScale);
+                atomicAdd(&hist[(key >> shift) & 255u], 1u);
+                atomicAdd(&histm[(key >> shift) & 255u], fx);
+              }
+            }
+          });
+          __syncthreads();
+          if (wave == 0) {
+            unsigned long long c[4];
+            for (int b = 0; b < 4; ++b) c[b] = histm[4 * lane + b];
+            const unsigned long long t = c[0] + c[1] + c[2] + c[3];
+            unsigned long long incl = t;
+            for (int o = 1; o < 64; o <<= 1) {
+              const unsigned long long y = __shfl_down(incl, o, 64);
+              if (lane + o < 64) incl += y;
+            }
+            unsigned long long above = A + (incl - t);
+            for (int b = 3; b >= 0; --b) {
+              // the bin holding the first token whose inclusive mass passes P
+              if (c[b] > 0 && above <= P && P < above + c[b]) {
+                sh_digit = 4 * lane + b;
+                sh_above = above;
+                sh_found = 1;
+              }
+              above += c[b];
+            }
+          }
+          __syncthreads();
+          const bool f = sh_found != 0;
+          const uint32_t d = sh_digit;
+          const unsigned long long ab = sh_above;
+          const unsigned long long binm = histm[d], binc = hist[d];
+          __syncthreads();
+          if (!f) {  // every candidate fits under top_p
+            p_found = false;
+            break;
+          }
+          A = ab;
+          prefix |= d << shift;
+          pmask |= 255u << shift;
+          cnt_p = binc;
+          if (shift == 0) {
+            const unsigned long long each = binm / binc;  // equal keys, equal mass
+            n_keep = each > 0 ? (P - A) / each : binc;
+          }
+        }
+        if (p_found) {
+          pth = prefix;
+          // The first token in descending order (the row maximum) is always kept.
+          if (pth == max_key && n_keep == 0) n_keep = 1;
+          if (n_keep > 0 && n_keep < cnt_p) {
+            const double nth = (double)(n_keep - 1);
+            cut_p = vocab_search<Tag, false>(
+                row, V, nslab,
+                [&](int e, uint32_t b) {
+                  const uint32_t key = float_key<KB>(b);
+                  return (key == pth && cand(e, key)) ? 1.0f : 0.0f;
+                },
+                [&](double) { return nth; }, sh);
+          }
+        }
+      }
+      auto kept = [&](int e, uint32_t key) {
+        return !p_found || key > pth ||
+               (key == pth && (n_keep >= cnt_p || (n_keep > 0 && e <= cut_p)));
+      };
+      // q weight of a top-k candidate, floored; 0 outside the candidates
+      auto qw = [&](int e, uint32_t b) {
+        const uint32_t key = float_key<KB>(b);
+        return cand(e, key) ? fmaxf(kept(e, key) ? ex(b) * inv_z : 0.0f, 1e-9f) : 0.0f;
+      };
+
+      // 5. inverse CDF with this row's uniform.
+      __shared__ double sh_total;
+      auto target = [&](double total) {
+        if (tid == 0) sh_total = total;
+        return u01 * total;
+      };
+      auto draw = [&](auto wfn, auto all_positive) {
+        tok = vocab_search<Tag, decltype(all_positive)::value>(row, V, nslab, wfn, target,
+                                                               sh);
+        const double qtot = sh_total;
+        __syncthreads();
+        if (tok < 0 || tok >= V) tok = bi;  // no positive weight: cannot happen, q >= 1e-9
+        if (tid == 0) logq = (float)(log((double)wfn(tok, load_one<Tag>(row, tok))) - log(qtot));
+      };
+      if (!use_k && !p_found) {
+        // The floored softmax max(p, 1e-9) as sample_resident_kernel's
+        // mixture: p with probability 1 / (1 + G), else the floor's excess
+        // g = max(1e-9 - p, 0), chosen by the component uniform u1; G takes
+        // a pass of its own only when u1 < V * 1e-9 (>= G / (1 + G)) or
+        // log q is asked for.
+        const float lz = log2f(zs);
+        auto rho_of = [&](uint32_t b) {
+          return exp2_hw(__builtin_fmaf(Bits<Tag>::val(b) - bx, c2, -lz));
+        };
+        const double u1 = (double)(((uint64_t)c[1] << 21) | (c[2] >> 11)) * 0x1p-53;
+        const bool near = u1 < (double)V * 1.001e-9;
+        // The rare near case needs G before it can choose the component; any
+        // other call for log q sums the excess on the draw's own pass.
+        double G = 0.0;
+        auto excess = [&](float gs) {
+          double t[1] = {(double)gs};
+          block_sum<SNT, 1, double>(t, sh.wave_tot);
+          return t[0];
+        };
+        if (near) {
+          float gs = 0.0f;
+          for_slabs<Tag>(row, V, nslab, [&](int, int e0, const uint32_t (&u)[VEC], auto full) {
+#pragma unroll
+            for (int i = 0; i < VEC; ++i)
+              if (full || e0 + i < V) gs += fmaxf(1e-9f - rho_of(u[i]), 0.0f);
+          });
+          G = excess(gs);
+        }
+        const bool use_g = near && u1 < G / (1.0 + G);
+        float gs = 0.0f, gs_row = 0.0f;  // gs_row: as the pass over the row left it
+        auto take_row = [&](double total) {
+          gs_row = gs;
+          return target(total);
+        };
+        if (a.logq && !near) {
+          tok = vocab_search<Tag, false>(
+              row, V, nslab,
+              [&](int, uint32_t b) {
+                const float p = rho_of(b);
+                gs += fmaxf(1e-9f - p, 0.0f);
+                return p;
+              },
+              take_row, sh);
+          __syncthreads();
+          G = excess(gs_row);
+        } else {
+          tok = vocab_search<Tag, false>(
+              row, V, nslab,
+              [&](int, uint32_t b) {
+                const float p = rho_of(b);
+                return use_g ? fmaxf(1e-9f - p, 0.0f) : p;
+              },
+              target, sh);
+        }
+        __syncthreads();
+        if (tok < 0 || tok >= V) tok = bi;  // no positive weight: cannot happen with p
+        if (tid == 0 && a.logq)
+          logq = (float)(log((double)fmaxf(rho_of(load_one<Tag>(row, tok)), 1e-9f)) - log1p(G));
+      } else {
+        draw(qw, std::false_type{});
+      }
+    }
+    }  // !drawn
+    // The token's S_other from pass 1: the sum without the maximum when the
+    // token is the argmax, else Z minus the token's own term.  S_other then
+    // holds the maximum's term 1 and e_tok <= 1, so the difference loses at
+    // most one bit.
+    if (tok != bi)
+      s_other = os - exp2_hw((Bits<Tag>::val(load_one<Tag>(row, tok)) - bx) * c2);
+  }
+
+  // 6. log_softmax(x / T) at the token, as the training row kernels form it:
+  // finish_row of the maximum, the sum over the other columns and the
+  // token's own value.
+  if (tid == 0) {
+    const float xt = Bits<Tag>::val(load_one<Tag>(row, tok)) * iT;
+    const RowLogprob<float> fr = finish_row<float>(m, s_other, xt);
+    a.token[r] = tok;
+    a.logp[r] = fr.logp;
+    if (a.logq) a.logq[r] = logq;
+  }
+}
+
+template <class Tag, bool LIST>
+__global__ __launch_bounds__(SNT) void sample_kernel(SampleArgs a) {
+  __shared__ CandShared cs;
+  __shared__ SmallShared ss;
+  __shared__ uint32_t hist[256];
+  const int64_t r = blockIdx.x;
+  if (r >= a.B) return;
+  // A fill-in launch redoes the rows the register-resident nucleus path
+  // handed over (token slot -1); the others return at once.
+  if (a.fill_in && __builtin_nontemporal_load(&a.token[r]) != -1) return;
+  sample_row<Tag, LIST>(a, r, cs, ss, hist);
+}
+
+template <class Tag>
+int launch_sample(const SampleArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL((sample_kernel<Tag, true>), dim3((unsigned)a.B), dim3(SNT), 0, st, a);
+  return check_launch("sample_kernel");
+}
+
+// The fill-in launch behind the nucleus path: its rows are too flat for a
+// list, and without one the workgroups that return at once start 1.6 us sooner.
+int launch_fill_in(const SampleArgs& a, hipStream_t st) {
+  SampleArgs f = a;
+  f.fill_in = 1;
+  hipLaunchKernelGGL((sample_kernel<TagBF16, false>), dim3((unsigned)f.B), dim3(SNT), 0, st, f);
+  return check_launch("sample_kernel");
+}
+
 template <class Tag, int SL>
 __global__ __launch_bounds__(SNT) void sample_resident_kernel(SampleArgs a) {
   static_assert(Tag::VEC == 8, "16-bit rows");
@@ -1550,7 +1780,7 @@ __global__ __launch_bounds__(SNT) void sample_resident_kernel(SampleArgs a) {
   // takes the streaming path (sample_row) in the same launch.
   const int kq = (int)a.top_k;
   constexpr int KB = Bits<Tag>::KB;
-  const uint32_t t0 = block_kth_key16(float_key<KB>(Bits<Tag>::bits_of(lm)), tid < nvec, kq,
+  const uint32_t t0 = block_kth_key<KB>(float_key<KB>(Bits<Tag>::bits_of(lm)), tid < nvec, kq,
                                       hist, &sh_digit, &sh_above);
   const uint32_t max_key = float_key<KB>(Bits<Tag>::bits_of(M));
   const float t0f = Bits<Tag>::val(key_bits<KB>(t0));
@@ -1606,7 +1836,7 @@ __global__ __launch_bounds__(SNT) void sample_resident_kernel(SampleArgs a) {
       eb[j] = !ev[j] ? 0u : (q < KCAP ? cs.bits[q] : rs.ovf.bits[q - KCAP]);
       ek[j] = float_key<KB>(eb[j]);
     }
-    const uint32_t kth = block_kth_keys16<NE>(ek, ev, kq, hist, &sh_digit, &sh_above);
+    const uint32_t kth = block_kth_keys<KB, NE>(ek, ev, kq, hist, &sh_digit, &sh_above);
     if (tid == 0) cs.n = 0;
     __syncthreads();
 #pragma unroll
@@ -1626,7 +1856,7 @@ __global__ __launch_bounds__(SNT) void sample_resident_kernel(SampleArgs a) {
     // The list still overflows (coarse logits, many ties at the threshold):
     // this row takes the streaming path, re-reading it from memory, in this
     // launch.  (The registers' row is not needed past the gather.)
-    sample_row<Tag>(a, r, cs, hist);
+    sample_row<Tag, false>(a, r, cs, ss, hist);
     return;
   }
   const bool use_p = a.top_p > 0.0 && a.top_p < 1.0;
@@ -1689,7 +1919,7 @@ __global__ __launch_bounds__(SNT) void sample_resident_kernel(SampleArgs a) {
     // The exact k-th key of the list (which holds every entry at or above
     // it), and how many of its ties the top k keep.
     const uint32_t key = float_key<KB>(eb);
-    const uint32_t kth = block_kth_key16(key, have, kq, hist, &sh_digit, &sh_above);
+    const uint32_t kth = block_kth_key<KB>(key, have, kq, hist, &sh_digit, &sh_above);
     int n_above = 0;
     (void)block_excl_count(have && key > kth, cs.wave_cnt, n_above);
     list_draw<Tag>(cs, sh_z, n, kth, kq - n_above, use_p, a.top_p, iT, M * iT, max_key, u01,
@@ -2578,9 +2808,7 @@ extern "C" int rrl_sample_logprobs(const void* logits, int32_t logits_dtype, int
       // fill-in launch of the streaming kernel (its other workgroups return).
       const int rc = launch_sample_blocks<TagBF16, true>(a, nslab, st);
       if (rc != RRL_OK) return rc;
-      SampleArgs f = a;
-      f.fill_in = 1;
-      return launch_sample<TagBF16>(f, st);
+      return launch_fill_in(a, st);
     }
     if (!res_topk)
       return logits_dtype == RRL_BF16 ? launch_sample_blocks<TagBF16, false>(a, nslab, st)
