@@ -191,6 +191,17 @@ def _addmm_into(acc: Tensor, a: Tensor, b: Tensor) -> None:
     acc.add_(torch.mm(a, b).to(acc.dtype))
 
 
+def _mm_wide(a: Tensor, b: Tensor) -> Tensor:
+    """a @ b, in float32 for 16-bit operands (the first block's share of a
+    float32 accumulator)."""
+
+    if a.dtype not in (torch.bfloat16, torch.float16):
+        return torch.mm(a, b)
+    acc = torch.zeros((a.shape[0], b.shape[1]), dtype=torch.float32, device=a.device)
+    _addmm_into(acc, a, b)
+    return acc
+
+
 def _transposed16(w: Tensor) -> Tensor:
     """A contiguous [H, V] copy of a 2-byte [V, H] matrix (rrl_transpose16)."""
 
@@ -201,24 +212,38 @@ def _transposed16(w: Tensor) -> Tensor:
     return out
 
 
+# From this many gradient rows the [H, V] copy of the weight repays itself
+# (V = 151,936, H = 1024: 127 us for the copy; d hidden from it 662 against
+# 669 us at 1,024 rows, 905 / 899 at 2,300, 1447 / 1464 at 4,096, 1694 / 1980
+# at 8,192 and 3320 / 3853 at 16,384).
+TRANSPOSE_ROWS = 6144
+
+
 class _Grads:
-    """d hidden rows and the d weight accumulator of one chunked backward.
+    """d hidden rows and the d weight accumulator of one chunked backward over
+    ``n`` gradient rows.
 
     For 16-bit weights both products take the operand layouts the GEMM library
     runs fastest on this GPU (measured on config 5's 16,384-token blocks):
     d hidden as ``dl @ wT.t()`` with ``wT`` a contiguous [H, V] copy of the
-    weight (3.25 ms against 3.78 ms for ``dl @ w``), and d weight as
-    ``acc += dl.t() @ xT.t()`` with ``xT`` the block's contiguous [H, n]
-    hidden states (4.29 ms against 4.81 ms for ``acc += dl.t() @ x``).
-    Other dtypes keep the plain forms."""
+    weight (3.25 ms against 3.78 ms for ``dl @ w``) where the rows repay the
+    copy, and d weight as ``acc += dl.t() @ xT.t()`` with ``xT`` the block's
+    contiguous [H, n] hidden states (4.29 ms against 4.81 ms for
+    ``acc += dl.t() @ x``).  One block's d weight is rounded to the weight
+    dtype by its GEMM, as the accumulator is at the end of several: the
+    float32 accumulator, its clearing and its conversion (V = 151,936,
+    H = 1024: 93 + 162 us and 160 us of the GEMM) are for several blocks,
+    whose first writes it instead of adding to zeros.  Other dtypes keep the
+    plain forms."""
 
-    def __init__(self, h2: Tensor, w: Tensor, need_h: bool, need_w: bool):
+    def __init__(self, h2: Tensor, w: Tensor, need_h: bool, need_w: bool, n: int, row_block: int):
         self.w = w
         self.wide = w.dtype in (torch.bfloat16, torch.float16)
         self.dh = torch.zeros_like(h2, memory_format=torch.contiguous_format) if need_h else None
-        self.wT = _transposed16(w) if (need_h and self.wide) else None
-        self.dw = (torch.zeros(w.shape, dtype=torch.float32 if self.wide else w.dtype,
-                               device=w.device) if need_w else None)
+        self.wT = _transposed16(w) if (need_h and self.wide and n >= TRANSPOSE_ROWS) else None
+        self.need_w = need_w
+        self.single = n <= row_block
+        self.dw: Optional[Tensor] = None
 
     def add_block(self, dl: Tensor, x_rows: Tensor, rows: Tensor) -> None:
         """dl [n, V] = d loss / d logits of the token rows ``rows``; x_rows
@@ -228,13 +253,20 @@ class _Grads:
             with nat.timed("lm_dhidden_gemm"):
                 w = self.wT.t() if self.wT is not None else self.w
                 self.dh.index_copy_(0, rows, torch.mm(dl, w))
-        if self.dw is not None:
+        if self.need_w:
             with nat.timed("lm_dweight_gemm"):
                 x = x_rows.t().contiguous().t() if self.wide else x_rows
-                _addmm_into(self.dw, dl.t(), x)
+                if self.single:
+                    self.dw = torch.mm(dl.t(), x)
+                elif self.dw is None:
+                    self.dw = _mm_wide(dl.t(), x)
+                else:
+                    _addmm_into(self.dw, dl.t(), x)
 
     def finish(self) -> Tuple[Optional[Tensor], Optional[Tensor]]:
         dw = self.dw
+        if self.need_w and dw is None:  # no gradient rows
+            dw = torch.zeros_like(self.w, memory_format=torch.contiguous_format)
         if dw is not None and dw.dtype != self.w.dtype:
             dw = dw.to(self.w.dtype)
         self.wT = None
@@ -281,9 +313,9 @@ def _chunked_backward(h2: Tensor, w: Tensor, tflat: Tensor, lse: Tensor, logp: T
 
     dev = h2.device
     V = w.shape[0]
-    grads = _Grads(h2, w, need_h, need_w)
     rows = torch.nonzero(g != 0).reshape(-1)
     n = rows.numel()
+    grads = _Grads(h2, w, need_h, need_w, n, row_block)
     if n:
         stream = nat.stream_ptr(dev)
         blocks = _Blocks(w, row_block, n)
@@ -480,8 +512,8 @@ class _ChunkedLinearPolicy(torch.autograd.Function):
         V = w.shape[0]
         stream = nat.stream_ptr(dev)
         pref = L.ctypes_ref(params)
-        grads = _Grads(h2, w, need_h, need_w)
         n = act.numel()
+        grads = _Grads(h2, w, need_h, need_w, n, row_block)
         if n == 0:
             return grads.finish()
         blocks = _Blocks(w, row_block, n)
