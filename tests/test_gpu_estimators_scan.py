@@ -97,7 +97,7 @@ def test_gae_infinite_value_stays_where_the_recurrence_has_it(device):
 
 
 @pytest.mark.parametrize("B,T", [(1, 1), (1, 2047), (1, 2048), (3, 683), (7, 4099), (1, 2100000)])
-@pytest.mark.parametrize("layout", ["flat", "strided"])
+@pytest.mark.parametrize("layout", ["flat", "offset", "strided"])
 def test_whiten_tiles(device, B, T, layout):
     """One tile of 2048 elements, a remainder, and more tiles than workgroups;
     a large common offset, which a one-pass sum of squares would lose."""
@@ -108,6 +108,8 @@ def test_whiten_tiles(device, B, T, layout):
     m[0, 0] = True
     if layout == "strided":
         x = torch.stack([x, x], -1).reshape(B, -1)[:, ::2]
+    elif layout == "offset":  # contiguous, but not at a 16-byte address
+        x = torch.cat([x.new_zeros(1), x.reshape(-1)])[1:].view(B, T)
     xd = x.double()[m]
     sd = xd.var(unbiased=False).sqrt() if xd.numel() > 1 else xd.new_zeros(())
     want = torch.where(m, (x.double() - xd.mean()) / (sd + 1e-3), 0.0)
