@@ -45,7 +45,8 @@ struct ScanArgs {
 template <int KIND> struct StateDim { static constexpr int D = KIND == 1 ? 2 : 1; };
 
 // A run of steps as a map on the carried state, S' = m S + c.  Padding is the
-// identity.
+// identity.  Maps and states between lanes are float64: composed in float32
+// they left 64 x 8192 advantages further from 64 bits than the serial walk.
 template <typename Acc, int KIND>
 struct Run {
   Acc m = Acc(1), c = Acc(0);
@@ -163,7 +164,7 @@ struct Step {
   static constexpr int D = StateDim<KIND>::D;
   Acc r, v, nv;
   bool valid, term;
-  __device__ __forceinline__ void add_to(Run<Acc, KIND>& f, Acc g, Acc gl) const {
+  __device__ __forceinline__ void add_to(Run<double, KIND>& f, Acc g, Acc gl) const {
     if (!valid) return;
     const Acc nt = term ? Acc(0) : Acc(1);
     if constexpr (KIND == 0) f.step(g * nt, r);
@@ -208,8 +209,8 @@ __global__ __launch_bounds__(NT) void reverse_scan_kernel(ScanArgs a) {
   constexpr int D = StateDim<KIND>::D;
   constexpr int NW = NT / 64;
   // Raw storage: the runs have initialisers, which LDS cannot.
-  __shared__ __align__(16) char sh_raw[2 * NW * sizeof(Run<Acc, KIND>)];
-  auto* sh_wave = reinterpret_cast<Run<Acc, KIND>*>(sh_raw);
+  __shared__ __align__(16) char sh_raw[2 * NW * sizeof(Run<double, KIND>)];
+  auto* sh_wave = reinterpret_cast<Run<double, KIND>*>(sh_raw);
   // gamma and gamma*lambda as the reference forms them: python float products
   // rounded to the tensor dtype.
   const Acc g = (Acc)a.gamma;
@@ -218,9 +219,9 @@ __global__ __launch_bounds__(NT) void reverse_scan_kernel(ScanArgs a) {
   const int64_t tile = (int64_t)NT * E;
   for (int64_t b = blockIdx.x; b < a.B; b += gridDim.x) {
     // The state behind the tile: at first the bootstrap value.
-    Acc C[D];
+    double C[D];
     C[0] = KIND != 2 && a.boot.present() ? a.boot.get<Acc>(b, 0) : Acc(0);
-    if (D == 2) C[D - 1] = Acc(0);
+    if (D == 2) C[D - 1] = 0.0;
     int buf = 0;
     for (int64_t base = (a.T - 1) / tile * tile; base >= 0; base -= tile, buf ^= 1) {
       const int64_t t0 = base + (int64_t)threadIdx.x * E;
@@ -241,7 +242,7 @@ __global__ __launch_bounds__(NT) void reverse_scan_kernel(ScanArgs a) {
         for (int i = 0; i < 4; ++i)
           st[e + i] = {r[i], v[i], nv[i], (ok >> i & 1u) && t + i < a.T, (term >> i & 1u) != 0};
       }
-      Run<Acc, KIND> f, later, whole;
+      Run<double, KIND> f, later, whole;
 #pragma unroll
       for (int e = E - 1; e >= 0; --e) st[e].add_to(f, g, gl);
       wave_suffix(f, later, whole);
@@ -249,18 +250,21 @@ __global__ __launch_bounds__(NT) void reverse_scan_kernel(ScanArgs a) {
       __syncthreads();
       // Every wave carries the tile's incoming state down to its own end, and
       // on through the rest for the next tile's.
-      Acc S[D];
+      double in[D];
 #pragma unroll
-      for (int i = 0; i < D; ++i) S[i] = C[i];
+      for (int i = 0; i < D; ++i) in[i] = C[i];
 #pragma unroll
       for (int w = NW - 1; w >= 0; --w) {
         if (w == wave) {
 #pragma unroll
-          for (int i = 0; i < D; ++i) S[i] = C[i];
+          for (int i = 0; i < D; ++i) in[i] = C[i];
         }
         sh_wave[buf * NW + w].apply(C);
       }
-      later.apply(S);
+      later.apply(in);
+      Acc S[D];
+#pragma unroll
+      for (int i = 0; i < D; ++i) S[i] = (Acc)in[i];
       Acc o0[E], o1[E];
 #pragma unroll
       for (int e = E - 1; e >= 0; --e) st[e].replay(g, gl, S, o0[e], o1[e]);
