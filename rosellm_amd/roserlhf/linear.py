@@ -232,9 +232,8 @@ class _Grads:
     ``acc += dl.t() @ x``).  One block's d weight is rounded to the weight
     dtype by its GEMM, as the accumulator is at the end of several: the
     float32 accumulator, its clearing and its conversion (V = 151,936,
-    H = 1024: 93 + 162 us and 160 us of the GEMM) are for several blocks,
-    whose first writes it instead of adding to zeros.  Other dtypes keep the
-    plain forms."""
+    H = 1024: 93 + 162 us and 160 us of the GEMM) are for several blocks.
+    Other dtypes keep the plain forms."""
 
     def __init__(self, h2: Tensor, w: Tensor, need_h: bool, need_w: bool, n: int, row_block: int):
         self.w = w
