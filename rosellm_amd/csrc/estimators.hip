@@ -203,7 +203,7 @@ struct Step {
 // state through the later waves' runs (up to 15 of them), so a
 // tile of NT * E steps costs one barrier; longer sequences go tile by tile
 // from the end.  rrl_gae at 64 x 8192: 57.7 us before (32-step chunks read
-// twice, 16 barriers), 9.2 us here.
+// twice, 16 barriers), 11.0 us here (9.2 with float32 maps).
 template <typename Acc, int KIND, int NT, int E, bool VEC>
 __global__ __launch_bounds__(NT) void reverse_scan_kernel(ScanArgs a) {
   constexpr int D = StateDim<KIND>::D;
@@ -489,8 +489,8 @@ __global__ __launch_bounds__(RED_NT) void masked_mean_bwd_kernel(RedArgs a) {
 // behind its type's branch) and the 64-bit division per element that strided
 // operands need bounded it: three launches took 24 us, two 15.7.  Float32
 // values with one-byte flags are read four at a time, and the second launch's
-// first tile is requested before the moments are merged: GAE + whitening of
-// 64 x 8192 50.2 -> 42.3 us per pass.
+// first tile is requested before the moments are merged: 7.8 us, and GAE +
+// whitening of 64 x 8192 50.2 -> 42.3 us per pass.
 constexpr int WH_E = 8;  // elements per lane and tile
 
 // (count, mean, M2) <- merged with another group's.
