@@ -39,6 +39,7 @@ namespace {
 
 constexpr int kMaxSlabs = 20;       // slabs per lane: 80 VGPRs of the 128 at 4 waves per SIMD
 constexpr int kWavesPerSimd = 4;
+constexpr float kFmaLse = 128.0f;   // |lse| up to which the one-FMA exponent keeps 5e-6
 
 // Per-token records for the resident kernel (TokenRecord): the views' dtype
 // and stride handling happens here, once per token, so that the row loop reads
@@ -224,17 +225,17 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
     if (EPV == 8 && tid == 0 && fabsf(lse) > 2e38f && fabsf(lse) != __builtin_huge_valf())
       raise_flag(a.status, RRL_FLAG_FAST_RANGE);
     // -g * exp(x - lse) = -sign(g) * exp2(x * log2e + (log2|g| - lse * log2e)):
-    // one FMA per 16-bit element (forming x - lse first costs 1-2% of the
-    // 151936-entry sweep), the difference first for float32, whose 1e-7 it
-    // keeps.  lse * log2e overflows past 2.3e38; logits there lie 1e36 apart,
-    // so e^(x - lse) is 1 or 0 and half the scale gives the same.  The sign is
-    // applied to the packed words with one XOR per dword.
+    // one FMA per 16-bit element, the difference first for float32, whose 1e-7
+    // it keeps.  The FMA leaves the rounding of lse * log2e in the exponent,
+    // 5e-6 at |lse| = 128 and doubling with it (at 3e38 nothing else is left),
+    // so 16-bit rows past that take the distance from the row's maximum, which
+    // is exact at any size, and the sum itself instead of lse, which float32
+    // cannot hold beside such a maximum.  The branch is uniform over the
+    // workgroup: forming the difference in every row costs 1-2% of the
+    // 151936-entry sweep.  The sign is applied to the packed words with one XOR
+    // per dword.
+    const bool wide = EPV == 8 && fabsf(lse) > kFmaLse && lse - lse == 0.0f;
     const float lg = __log2f(fabsf(gr));
-    const float sc = EPV == 8 && fabsf(lse) > 2e38f ? 0.5f * kLog2e : kLog2e;
-    const float cg = lg - lse * sc;
-    auto expo = [&](float xv) {
-      return EPV == 8 ? __builtin_fmaf(xv, sc, cg) : __builtin_fmaf(xv - lse, kLog2e, lg);
-    };
     const bool flip = gr > 0.0f;
     const uint32_t sgn = flip ? P::SGN2 : 0u;
     const float tgt_pre = flip ? -tgt_d : tgt_d;  // the XOR restores tgt_d
@@ -242,26 +243,39 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
     // row: there log2|g| = -inf and exp2(-inf) = 0 for every finite or -inf
     // logit (a +inf or NaN logit makes lse non-finite and the row NaN, as in
     // log_softmax), so zero-weight rows take no branch.
+    auto put_row = [&](auto expo) __attribute__((always_inline)) {
 #pragma unroll
-    for (int k = 0; k < SL; ++k) {
-      float d[EPV];
-      float v[EPV];
-      P::unpack(x[k], v);
+      for (int k = 0; k < SL; ++k) {
+        float d[EPV];
+        float v[EPV];
+        P::unpack(x[k], v);
 #pragma unroll
-      for (int i = 0; i < EPV; ++i) d[i] = exp2_hw(expo(v[i]));
-      if (rel == k * NT) {
+        for (int i = 0; i < EPV; ++i) d[i] = exp2_hw(expo(v[i]));
+        if (rel == k * NT) {
 #pragma unroll
-        for (int i = 0; i < EPV; ++i) d[i] = (i == ti) ? tgt_pre : d[i];
+          for (int i = 0; i < EPV; ++i) d[i] = (i == ti) ? tgt_pre : d[i];
+        }
+        u32x4 o = P::pack(d);
+        o.x ^= sgn; o.y ^= sgn; o.z ^= sgn; o.w ^= sgn;
+        store_b128_nt(o, dst, voff, k * NT * 16);
       }
-      u32x4 o = P::pack(d);
-      o.x ^= sgn; o.y ^= sgn; o.z ^= sgn; o.w ^= sgn;
-      store_b128_nt(o, dst, voff, k * NT * 16);
-    }
-    if constexpr (EXTRAS) {
-      const float dv = ex_tgt ? tgt_pre : exp2_hw(expo(P::one(xe)));
-      P::store_one(P::pack_one(dv) ^ (flip ? P::SGN1 : 0u), row_rsrc(drow, V32 * ESZ),
-                   extra_off(g));
-      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (EXTRAS) {
+        const float dv = ex_tgt ? tgt_pre : exp2_hw(expo(P::one(xe)));
+        P::store_one(P::pack_one(dv) ^ (flip ? P::SGN1 : 0u), row_rsrc(drow, V32 * ESZ),
+                     extra_off(g));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    if constexpr (EPV == 8) {
+      if (wide) {
+        const float cm = lg - __log2f(s + exp2_hw((xt - m) * kLog2e));
+        put_row([&](float xv) { return __builtin_fmaf(xv - m, kLog2e, cm); });
+      } else {
+        const float cg = lg - lse * kLog2e;
+        put_row([&](float xv) { return __builtin_fmaf(xv, kLog2e, cg); });
+      }
+    } else {
+      put_row([&](float xv) { return __builtin_fmaf(xv - lse, kLog2e, lg); });
     }
     // Then the next row's loads into the same registers: each CU issues its
     // row's stores as one burst and the next row's loads as another instead

@@ -715,10 +715,10 @@ def test_fused_many_rows_persistent(device, dtype, objective):
 
 def test_fused_extreme_logits(device):
     """Rows at the edge of the 16-bit range: an all -inf row but one entry, a
-    half -inf (masked vocabulary) row, and a row whose log-sum-exp (3e38)
-    exceeds the register-resident kernel's exponent range, which the generic
-    kernel launched behind it (RRL_POLICY_RERUN_FAST_RANGE) then redoes on the
-    device.  All must match the float64 oracle."""
+    half -inf (masked vocabulary) row, and rows with a log-sum-exp of 3e38 (the
+    maximum on the target, and off it under a clamped ratio, whose gradient is
+    0; test_gpu_value_range.py has the rows with a gradient).  All must match
+    the float64 oracle."""
 
     B, T, V = 4, 8, 4096
     x, t, old, adv, mask = _fused_inputs(35, B, T, V, torch.bfloat16)
