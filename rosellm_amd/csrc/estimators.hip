@@ -493,15 +493,23 @@ __global__ __launch_bounds__(RED_NT) void masked_mean_bwd_kernel(RedArgs a) {
 // whitening of 64 x 8192 50.2 -> 42.3 us per pass.
 constexpr int WH_E = 8;  // elements per lane and tile
 
-// (count, mean, M2) <- merged with another group's.
+// (count, mean, M2) <- merged with another group's.  The squared distance of
+// the means may pass the type's range where the deviations' squares do not, so
+// it is only formed times the weight; means further apart than the range keep a
+// finite mean and give an infinite M2, as the sum of squares would be.
 template <typename Acc>
 struct Moments {
   Acc n, mean, m2;
   __device__ __forceinline__ void merge(Acc n2, Acc mean2, Acc m22) {
     if (n2 == Acc(0)) return;
+    if (n == Acc(0)) {
+      n = n2, mean = mean2, m2 = m22;
+      return;
+    }
     const Acc nt = n + n2, d = mean2 - mean, f = n2 / nt;
-    mean += d * f;
-    m2 += m22 + d * d * n * f;
+    const bool apart = d - d != Acc(0) && mean - mean == Acc(0) && mean2 - mean2 == Acc(0);
+    mean = apart ? mean * (n / nt) + mean2 * f : mean + d * f;
+    m2 += m22 + (d * (n * f)) * d;
     n = nt;
   }
 };

@@ -118,3 +118,39 @@ def test_whiten_tiles(device, B, T, layout):
     assert (got.double() - want).abs().max().item() <= 1e-3 * max(1.0, want.abs().max().item())
     with pytest.raises(ValueError):
         R.masked_whiten(x, torch.zeros_like(m))
+
+
+@pytest.mark.parametrize("layout", ["flat", "strided"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_whiten_large_values(device, layout, dtype):
+    """Finite values whose squares overflow float32 while their deviations do
+    not, in one tile of 2048 elements and in several."""
+
+    def run(x, m):
+        if layout == "strided":
+            x = torch.stack([x, x], -1).reshape(x.shape[0], -1)[:, ::2]
+        return R.masked_whiten(x, m).double()
+
+    for n in (64, 4096):
+        m = torch.ones(1, n, dtype=torch.bool, device=device)
+        # deviations of 1e17 about 2e19
+        x = (2.0e19 + 1.0e17 * torch.randn(1, n, device=device)).to(dtype)
+        xd = x.double()
+        want = (xd - xd.mean()) / xd.var(unbiased=False).sqrt()
+        # float32 mean: 1e-6 of 2e19, 2e-4 of a deviation; bfloat16 results are
+        # rounded to 8 bits, 2^-9 of a value at most
+        bar = 1e-3 + (2.0 ** -9 if dtype == torch.bfloat16 else 0.0)
+        assert (run(x, m) - want).abs().max().item() <= bar * want.abs().max().item()
+        # one value 2^n times: its sum is exact, so nothing deviates
+        x = torch.full((1, n), 2.0 ** 100, dtype=dtype, device=device)
+        assert torch.equal(run(x, m), torch.zeros(1, n, dtype=torch.float64, device=device))
+    # two tiles with one value each: the means lie two deviations apart
+    m = torch.zeros(1, 4096, dtype=torch.bool, device=device)
+    m[0, 5] = m[0, 3000] = True
+    x = torch.zeros(1, 4096, dtype=dtype, device=device)
+    x[0, 5], x[0, 3000] = 2.0 ** 63.5, -(2.0 ** 63.5)
+    got = run(x, m)
+    assert abs(got[0, 5].item() - 1.0) <= 1e-2 and got[0, 3000].item() == -got[0, 5].item()
+    # a spread whose square no float32 holds: deviations over an infinite one
+    x[0, 5], x[0, 3000] = 3.0e38, -3.0e38
+    assert torch.equal(run(x, m), torch.zeros_like(got))
