@@ -658,7 +658,8 @@ int row_coef_args(PolicyArgs& a, const rrl_policy_params* params, int64_t B, int
   const bool gspo = params->kind == RRL_OBJ_GSPO || params->kind == RRL_OBJ_GSPO_TOKEN;
   RRL_REQUIRE(!gspo || !row_coef, RRL_EINVAL,
               "row coefficients exist for the token-local objectives only");
-  RRL_REQUIRE(workspace && (B == 0 || ((row_coef || gspo) && mask.ptr)), RRL_EINVAL,
+  // An empty mask has no address, and its rows are still counted (as empty).
+  RRL_REQUIRE(workspace && (B == 0 || row_coef || gspo) && (B * T == 0 || mask.ptr), RRL_EINVAL,
               "null pointer argument");
   RRL_REQUIRE(is_known_dtype(mask.dtype), RRL_EDTYPE, "unsupported mask dtype");
   RRL_REQUIRE(params->kind != RRL_OBJ_NLL || mask.dtype == RRL_I32 || mask.dtype == RRL_I64,
@@ -675,7 +676,9 @@ extern "C" int rrl_policy_row_coef(const rrl_policy_params* params, int64_t B, i
                                    void* workspace, int32_t* status, void* stream) {
   clear_error();
   PolicyArgs a{};
-  RRL_REQUIRE(B == 0 || row_coef, RRL_EINVAL, "null pointer argument");
+  RRL_REQUIRE(B == 0 || (row_coef && mask.ptr), RRL_EINVAL, "null pointer argument");
+  RRL_REQUIRE(!params || (params->kind != RRL_OBJ_GSPO && params->kind != RRL_OBJ_GSPO_TOKEN),
+              RRL_EINVAL, "row coefficients exist for the token-local objectives only");
   if (int rc = row_coef_args(a, params, B, T, mask, acc_dtype, row_coef, workspace, status))
     return rc;
   hipStream_t st = as_stream(stream);

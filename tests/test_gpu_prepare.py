@@ -14,7 +14,9 @@ import pytest
 import torch
 
 from rosellm_amd import _native as nat
+from rosellm_amd import roserlhf as R
 from rosellm_amd.roserlhf import losses as L
+from rosellm_amd.rosetrainer import cross_entropy
 
 pytestmark = pytest.mark.gpu
 
@@ -118,3 +120,36 @@ def test_prepare_and_forward(device, B, T, kind):
              grad.data_ptr(), nat.stream_ptr(device))
     (want,) = torch.autograd.grad((0.5 - 2.0) * obj + 0.25 * mean, lp)
     assert torch.allclose(grad.double(), want, rtol=1e-5, atol=1e-6 * want.abs().max().item())
+
+
+@pytest.mark.parametrize("objective", ["gspo", "gspo_token"])
+def test_sequences_without_positions(device, objective):
+    """[B, 0]: no sequence has an action token, fused as composed."""
+
+    B, V = 3, 16
+    x = torch.zeros(B, 0, V, device=device)
+    t = torch.zeros(B, 0, dtype=torch.int64, device=device)
+    z = torch.zeros(B, 0, device=device)
+    adv = torch.zeros(B, device=device) if objective == "gspo" else z
+    mask = torch.zeros(B, 0, dtype=torch.bool, device=device)
+    composed = R.gspo_policy_loss if objective == "gspo" else R.gspo_token_policy_loss
+    with pytest.raises(ValueError, match="at least one action token"):
+        composed(R.gather_token_logprobs(x, t), z, adv, mask, clip_low=0.1, clip_high=0.1)
+    with pytest.raises(ValueError, match="at least one action token"):
+        R.fused_policy_loss(x, t, z, adv, mask, objective=objective, clip_low=0.1)
+
+
+def test_token_objectives_without_positions(device):
+    """[B, 0] through the single-pass objectives: the composed loss's error,
+    and torch's own values for a cross-entropy over nothing."""
+
+    x = torch.zeros(3, 0, 16, device=device)
+    t = torch.zeros(3, 0, dtype=torch.int64, device=device)
+    z = torch.zeros(3, 0, device=device)
+    with pytest.raises(ValueError, match="empty mask"):
+        R.fused_policy_loss(x, t, z, z, t.bool(), clip_low=0.1)
+    with pytest.raises(ValueError, match="at least one action token"):
+        R.fused_policy_loss(x, t, z, z, t.bool(), objective="sapo", tau_positive=1.0,
+                            tau_negative=1.0)
+    assert torch.isnan(cross_entropy(x, t))
+    assert cross_entropy(x, t, reduction="sum").item() == 0.0
