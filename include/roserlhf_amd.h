@@ -64,6 +64,14 @@ enum rrl_status {
   RRL_EALIGN = -4   /* pointer alignment below the element size */
 };
 
+/* Added to the address of a `status` word in host memory that the GPU can write
+ * (hipHostMalloc): rrl_masked_mean_fwd, rrl_sequence_log_ratio_fwd,
+ * rrl_broadcast_turn and rrl_masked_whiten set its bits with plain stores, as
+ * host memory has no GPU atomics.  The word is cleared by the caller, serves one
+ * call at a time and is read behind an event.  A word passed without it is
+ * device memory, OR-ed atomically, and may be shared by calls on any streams. */
+#define RRL_STATUS_HOST 1
+
 /* Bits written (OR-ed) into the device `status` word. */
 enum rrl_flag {
   RRL_FLAG_EMPTY_MASK = 1,       /* global mask weight sum is zero        (losses.py:48-49)   */

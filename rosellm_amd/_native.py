@@ -49,6 +49,8 @@ POLICY_SUM = 4
 POLICY_RERUN_FAST_RANGE = 8
 POLICY_RECORDS_READY = 16
 
+STATUS_HOST = 1  # RRL_STATUS_HOST, added to a host status word's address
+
 # rrl_objective
 OBJ_PPO, OBJ_SAO, OBJ_GSPO, OBJ_GSPO_TOKEN, OBJ_SAPO, OBJ_NLL = range(6)
 NSCALARS = 8
@@ -364,24 +366,24 @@ def read_status(status: torch.Tensor) -> int:
 
 class HostStatus:
     """A status word in host memory that a kernel stores (rrl_policy_prepare,
-    rrl_targets_status, rrl_policy_forward) and the host reads without waiting
+    rrl_targets_status, rrl_policy_forward) or, cleared first, sets bits of (the
+    estimators' entry points) and the host reads without waiting
     for anything queued behind that kernel: ``record()`` marks the place on the
     current stream, ``read()`` waits for the mark alone.  As a context manager
     it waits on the way out, so the word outlives its writer on every path."""
 
-    __slots__ = ("_word", "_event")
+    __slots__ = ("_word", "_event", "ptr")
 
     def __init__(self, zero: bool = False):
-        """``zero``: cleared first, for kernels that only set bits."""
+        """``zero``: cleared first, for kernels that only set bits; ``ptr`` then
+        says that they must do so without atomics."""
 
         self._word = torch.empty(1, dtype=torch.int32, pin_memory=True)
+        self.ptr = self._word.data_ptr()
         if zero:
             self._word.zero_()
+            self.ptr += STATUS_HOST
         self._event = None
-
-    @property
-    def ptr(self) -> int:
-        return self._word.data_ptr()
 
     def record(self, device: torch.device) -> None:
         self._event = torch.cuda.Event()

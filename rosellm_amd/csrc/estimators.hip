@@ -17,14 +17,18 @@ namespace rrl {
 
 namespace {
 
-// Sets a bit of the caller's cleared status word without an atomic, so that
-// the word may be host memory: every writer in one of these launches sets the
-// same single bit.
+// Sets a bit of the caller's status word: with an atomic, or (RRL_STATUS_HOST in
+// its address) with plain stores to a word in host memory, which has no atomics
+// from here and belongs to this call alone; every writer in one of these
+// launches sets the same single bit.
 __device__ __forceinline__ void or_flag(int32_t* status, int32_t bit) {
-  if (status) {
-    volatile int32_t* p = status;
+  const uintptr_t at = reinterpret_cast<uintptr_t>(status);
+  if (at & RRL_STATUS_HOST) {
+    volatile int32_t* p = reinterpret_cast<volatile int32_t*>(at - RRL_STATUS_HOST);
     *p = *p | bit;
     __threadfence_system();
+  } else {
+    raise_flag(status, bit);
   }
 }
 

@@ -153,3 +153,55 @@ def test_token_objectives_without_positions(device):
                             tau_negative=1.0)
     assert torch.isnan(cross_entropy(x, t))
     assert cross_entropy(x, t, reduction="sum").item() == 0.0
+
+
+def _flagging_calls(device, B=64, T=2048):
+    """(entry point's call on a status address, its bit) for the entry points
+    that OR a bit: every token, row or mask of the inputs is a bad one."""
+
+    x = torch.ones(B, T, device=device)
+    none = torch.zeros(B, T, dtype=torch.bool, device=device)
+    live = ~none
+    ids = torch.full((B, T), 7, dtype=torch.int64, device=device)
+    ws = torch.empty(nat.lib().rrl_reduce_workspace_bytes(B * T), dtype=torch.uint8, device=device)
+    out, cnt = torch.empty_like(x), torch.empty_like(x)
+    s = lambda: nat.stream_ptr(device)  # noqa: E731
+    v = _view
+    return [
+        (lambda p: nat.call("rrl_masked_whiten", B, T, v(x), v(none), 1e-8, 1, nat.F32,
+                            ws.data_ptr(), out.data_ptr(), nat.F32, p, s()), nat.FLAG_EMPTY_MASK),
+        (lambda p: nat.call("rrl_masked_mean_fwd", B, T, v(x), v(none), nat.F32, ws.data_ptr(),
+                            out.data_ptr(), p, s()), nat.FLAG_EMPTY_MASK),
+        (lambda p: nat.call("rrl_sequence_log_ratio_fwd", B, T, v(x), v(x), v(none), 1, nat.F32,
+                            out.data_ptr(), cnt.data_ptr(), p, s()), nat.FLAG_EMPTY_ROW),
+        (lambda p: nat.call("rrl_broadcast_turn", B, 1, T, nat.rows_view(x[:, :1], B, 1)[0], v(ids),
+                            v(live), cnt.data_ptr(), nat.F32, p, s()), nat.FLAG_INVALID_TURN),
+    ]
+
+
+def test_status_word_shared_between_streams(device):
+    """A device status word takes bits from calls on several streams at once and
+    keeps those already set; a host word (RRL_STATUS_HOST) is set without
+    atomics; a null one is not written."""
+
+    calls = _flagging_calls(device)
+    for f, bit in calls:
+        word = torch.full((1,), 64, dtype=torch.int32, device=device)
+        f(word.data_ptr())
+        f(None)
+        assert int(word.item()) == 64 | bit
+        with nat.HostStatus(zero=True) as host:
+            f(host.ptr)
+            host.record(device)
+            assert host.read() == bit
+    # different bits from the last two and the first, each on its own stream
+    (a, ab), (b, bb), (c, cb) = calls[0], calls[2], calls[3]
+    streams = [torch.cuda.Stream(device) for _ in range(3)]
+    words = torch.zeros(50, dtype=torch.int32, device=device)
+    torch.cuda.synchronize()
+    for i in range(words.numel()):
+        for f, st in zip((a, b, c), streams):
+            with torch.cuda.stream(st):
+                f(words[i:].data_ptr())
+    torch.cuda.synchronize()
+    assert words.tolist() == [ab | bb | cb] * words.numel()
