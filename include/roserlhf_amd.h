@@ -78,10 +78,8 @@ enum rrl_flag {
   RRL_FLAG_EMPTY_ROW = 2,        /* some row has no action token          (losses.py:250-251) */
   RRL_FLAG_TARGET_RANGE = 4,     /* target id outside [0, V)              (gather, losses.py:36) */
   RRL_FLAG_INVALID_TURN = 8,     /* unmasked token with invalid turn id   (advantages.py:284-286) */
-  RRL_FLAG_FAST_RANGE = 16,      /* rrl_fused_logprob_policy's 16-bit register-resident kernel met a
-                                    row with finite |log-sum-exp| > 2e38.  Its outputs are the exact
-                                    ones; callers that refuse such logits read it (no reference
-                                    counterpart) */
+  RRL_FLAG_FAST_RANGE = 16,      /* not raised any more: rrl_fused_logprob_policy forms rows of any
+                                    finite log-sum-exp in its one launch (no reference counterpart) */
   RRL_FLAG_BAD_PROBS = 32,       /* rrl_sample_logprobs: a row holds NaN or +inf logits (torch.multinomial
                                     rejects such probabilities, roseinfer/engine.py:1155,1169) */
   RRL_FLAG_LM_RANGE = 64         /* rrl_lm_head_fwd without mref_in: a token's logits rose more than 64
@@ -99,12 +97,10 @@ enum rrl_policy_flag {
                                  lse as 0 (equal to the reference for finite logits, where such a
                                  row contributes exactly 0; no reference counterpart) */
   RRL_POLICY_SUM = 4,         /* RRL_OBJ_NLL: reduction "sum" instead of "mean" */
-  RRL_POLICY_RERUN_FAST_RANGE = 8, /* rrl_fused_logprob_policy: launch the generic row kernel as a
-                                 conditional rerun of the call just made with the same arguments
-                                 on the same stream and status word (status required): its
-                                 workgroups return at once unless the status word holds
-                                 RRL_FLAG_FAST_RANGE, so a caller need not read the status between
-                                 the two launches (no reference counterpart) */
+  RRL_POLICY_RERUN_FAST_RANGE = 8, /* rrl_fused_logprob_policy: the rerun, for rows flagged
+                                 FAST_RANGE, of the call just made with the same arguments (status
+                                 required).  No row is flagged: the arguments are checked and
+                                 nothing is launched (no reference counterpart) */
   RRL_POLICY_RECORDS_READY = 16 /* rrl_fused_logprob_policy: rrl_policy_prepare has packed the
                                  records (no reference counterpart) */
 };

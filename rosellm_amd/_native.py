@@ -38,7 +38,6 @@ FLAG_EMPTY_MASK = 1
 FLAG_EMPTY_ROW = 2
 FLAG_TARGET_RANGE = 4
 FLAG_INVALID_TURN = 8
-FLAG_FAST_RANGE = 16
 FLAG_BAD_PROBS = 32
 FLAG_LM_RANGE = 64
 
@@ -219,12 +218,10 @@ def timed(name: str) -> _TimedSpan:
     return _TimedSpan(name)
 
 
-def call(name: str, *args, timed: bool = True) -> None:
-    """Call an entry point and raise on a non-zero return code.  ``timed=False``
-    keeps the call out of ``time_calls``' records: a launch that is not the
-    entry point's own work (the conditional rerun behind a single-pass sweep)."""
+def call(name: str, *args) -> None:
+    """Call an entry point and raise on a non-zero return code."""
 
-    events = _timed.get(name) if _timed and timed else None
+    events = _timed.get(name) if _timed else None
     if events is not None:
         start = _event()
         start.record()

@@ -222,8 +222,6 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
     // Sweep 2: dlogits, then refill the register slabs with the next row.
     const S* drow = dl + (int64_t)b * a.ds_b + (int64_t)t * a.ds_t;
     const __amdgpu_buffer_rsrc_t dst = row_rsrc(drow + g.head, g.nbody * 16);
-    if (EPV == 8 && tid == 0 && fabsf(lse) > 2e38f && fabsf(lse) != __builtin_huge_valf())
-      raise_flag(a.status, RRL_FLAG_FAST_RANGE);
     // -g * exp(x - lse) = -sign(g) * exp2(x * log2e + (log2|g| - lse * log2e)):
     // one FMA per 16-bit element, the difference first for float32, whose 1e-7
     // it keeps.  The FMA leaves the rounding of lse * log2e in the exponent,

@@ -463,17 +463,6 @@ class _ChunkedLinearPolicy(torch.autograd.Function):
                               row_block)
             grads = _ChunkedLinearPolicy._sweep(params, h2, w, tflat, ok, ak, mk, coef, act, T,
                                                 lse, logp, need_h, need_w, row_block, status)
-            flags = nat.read_status(status)
-            if flags & nat.FLAG_FAST_RANGE:
-                # A row's log-sum-exp beyond the register-resident kernel's
-                # exponent range (bf16 logits near 2e38): redo the sweep on the
-                # generic row kernel (the block's logits were overwritten).
-                generic = nat.RrlPolicyParams.from_buffer_copy(params)
-                generic.flags |= nat.POLICY_GENERIC
-                status.zero_()
-                grads = _ChunkedLinearPolicy._sweep(generic, h2, w, tflat, ok, ak, mk, coef, act,
-                                                    T, lse, logp, need_h, need_w, row_block,
-                                                    status)
         else:
             live = mk.reshape(N) != 0
             _logprob_rows(h2, w, tflat, torch.nonzero(live).reshape(-1), lse, logp, status,

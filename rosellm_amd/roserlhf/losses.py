@@ -827,8 +827,7 @@ class _Sweep:
     The host waits for the errors once.  Out of place it waits behind
     everything queued: the wait ends when the prepare kernels do, and the sweep
     is already next in line.  In place the errors are read before the sweep
-    overwrites the logits, except for bfloat16, whose log-sum-exp range
-    (FAST_RANGE) is known after it."""
+    overwrites the logits."""
 
     def __init__(self, params, x, geom, tview, ov, av, mv, dev):
         self.params, self.x, self.dev = params, x, dev
@@ -849,7 +848,7 @@ class _Sweep:
         self.logp = torch.empty(B * T, dtype=self.acc, device=dev)
         self.lse = torch.empty(B * T, dtype=self.acc, device=dev)
 
-    def run(self, dl_ptr: int, d_b: int, d_t: int, inplace: bool, outs, trusted, inplace_error):
+    def run(self, dl_ptr: int, d_b: int, d_t: int, inplace: bool, outs, trusted):
         """Launch everything; raises the call's data errors."""
 
         B, T, V = self.B, self.T, self.V
@@ -858,25 +857,21 @@ class _Sweep:
         p = nat.RrlPolicyParams.from_buffer_copy(self.params)
         p.flags |= nat.POLICY_RECORDS_READY
         pref = ctypes_ref(p)
-        late = inplace and self.x.dtype == torch.bfloat16
-        sweep_status = nat.new_status(self.dev) if late else None
         with nat.HostStatus() as status:
             nat.call("rrl_policy_prepare", pref, B, T, V, self.tview, self.ov, self.av, self.mv,
                      self.acc_code, self.coef_ptr, self.rec_ptr, self.ws_ptr, status.ptr, stream)
             status.record(self.dev)
-            if inplace and not late:
+            if inplace:
                 _raise_flags(status.read(), p.kind)
             nat.call("rrl_fused_logprob_policy", pref, self.x.data_ptr(), code, B, T, V, self.s_b,
                      self.s_t, self.tview, self.ov, self.av, self.mv, self.coef_ptr,
                      self.rec_ptr, self.logp.data_ptr(), self.lse.data_ptr(), dl_ptr, code, d_b,
-                     d_t, nat.ptr(sweep_status), stream)
+                     d_t, None, stream)
             lview = nat.RrlView(self.logp.data_ptr(), self.acc_code, T, 1)
             nat.call("rrl_policy_forward", pref, B, T, lview, self.ov, self.av, self.mv,
                      self.acc_code, self.ws_ptr, ctypes.byref(nat.scalars(outs)), None,
                      nat.ptr(trusted), None, stream)
-            if late and nat.read_status(sweep_status) & nat.FLAG_FAST_RANGE:
-                raise RuntimeError(inplace_error)
-            if late or not inplace:
+            if not inplace:
                 _raise_flags(status.read(), p.kind)
 
 
@@ -922,9 +917,7 @@ class _FusedPolicy(torch.autograd.Function):
         trusted = torch.empty(B * T if kind == nat.OBJ_SAO else 0, dtype=torch.bool, device=dev)
         logp, lse, ws = sweep.logp, sweep.lse, sweep.scratch
         outs = _scalar_outputs(_scalar_dtypes(kind, logp, old, adv), dev)
-        sweep.run(dl.data_ptr(), d_b, d_t, inplace, outs, trusted if trusted.numel() else None,
-                  "fused_policy_loss(inplace=True): logits beyond +-2e38 need the generic "
-                  "kernel, which cannot rerun over overwritten logits; call with inplace=False")
+        sweep.run(dl.data_ptr(), d_b, d_t, inplace, outs, trusted if trusted.numel() else None)
 
         ctx.params = params
         ctx.inplace = inplace

@@ -98,9 +98,7 @@ class _CrossEntropyRows(torch.autograd.Function):
                 d_b, d_t = T * V, V
             dptr = dl.data_ptr()
         loss = torch.empty((), dtype=sweep.acc, device=dev)
-        sweep.run(dptr, d_b, d_t, inplace, (None, None, None, None, loss), None,
-                  "cross-entropy with inplace=True: logits beyond +-2e38 need the generic "
-                  "kernel, which cannot rerun over overwritten logits; call with inplace=False")
+        sweep.run(dptr, d_b, d_t, inplace, (None, None, None, None, loss), None)
         if shift and logits.shape[1] > 0:
             dl[:, -1].zero_()  # the last position predicts nothing
         del tkeep

@@ -750,13 +750,11 @@ def test_fused_extreme_logits(device):
 
 
 @pytest.mark.parametrize("V", [4096, 151936])
-def test_fused_rerun_only_when_flagged(device, V):
-    """The conditional generic launch queued behind an out-of-place bfloat16
-    sweep returns at once when no row was flagged: log-probs, loss and
-    dlogits equal the register-resident kernel's own (an in-place call, which
-    queues no rerun) bit for bit."""
+def test_fused_inplace_is_bit_identical(device, V):
+    """Out of place and in place run the same single-pass kernel: log-probs and
+    dlogits are equal bit for bit."""
 
-    print(f"[rerun-if-flagged] V={V}", flush=True)
+    print(f"[fused-inplace] V={V}", flush=True)
     B, T = 4, 8
     x, t, old, adv, mask = _fused_inputs(73, B, T, V, torch.bfloat16)
     d = lambda v: v.to(device)  # noqa: E731
@@ -769,7 +767,7 @@ def test_fused_rerun_only_when_flagged(device, V):
                                       inplace=True, **kw)
     assert torch.equal(lp, lp_i)
     _close(out_i.loss, out.loss, 1e-6, 1e-8, "loss")
-    assert torch.equal(buf.detach(), xd.grad), "dlogits differ from the resident kernel's"
+    assert torch.equal(buf.detach(), xd.grad), "in-place dlogits differ"
 
 
 @pytest.mark.parametrize("dtype,V", [(torch.bfloat16, 151936), (torch.bfloat16, 20000),

@@ -205,3 +205,28 @@ def test_status_word_shared_between_streams(device):
                 f(words[i:].data_ptr())
     torch.cuda.synchronize()
     assert words.tolist() == [ab | bb | cb] * words.numel()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_inplace_errors_leave_the_logits(device, dtype):
+    """A bad target id or an empty mask raises before the logits are
+    overwritten."""
+
+    B, T, V = 2, 5, 4096
+    x = torch.randn(B, T, V, device=device).to(dtype)
+    keep = x.clone()
+    t = torch.randint(0, V, (B, T), device=device)
+    old = adv = torch.zeros(B, T, device=device)
+    mask = torch.ones(B, T, dtype=torch.bool, device=device)
+    bad = t.clone()
+    bad[-1, -1] = V
+    kw = dict(clip_low=0.2, inplace=True)
+    with pytest.raises(RuntimeError, match="index out of bounds"):
+        R.fused_policy_loss(x, bad, old, adv, mask, **kw)
+    assert torch.equal(x, keep)
+    with pytest.raises(ValueError, match="empty mask"):
+        R.fused_policy_loss(x, t, old, adv, torch.zeros_like(mask), **kw)
+    assert torch.equal(x, keep)
+    with pytest.raises(IndexError):
+        cross_entropy(x, bad, inplace=True)
+    assert torch.equal(x, keep)

@@ -56,6 +56,9 @@ def test_maximum_off_the_label(device, dtype, top, V):
     xg = x.clone().requires_grad_()
     (dl,) = torch.autograd.grad(cross_entropy(xg, t, reduction="sum"), xg)
     _near(dl, want, dtype)
+    buf = x.clone()
+    loss = cross_entropy(buf.requires_grad_(), t, reduction="sum", inplace=True)
+    assert torch.equal(buf.detach(), dl) and not torch.isnan(loss)
 
 
 @pytest.mark.parametrize("dtype,top", TOPS)
@@ -86,3 +89,75 @@ def test_tied_maxima(device, dtype, top, V, objective):
     want = -g * lp.exp()
     want.scatter_add_(-1, t[..., None], g)
     _near(dl, want, dtype)
+    buf = x.clone()
+    out_i = R.fused_policy_loss(buf.requires_grad_(), t, old, adv, mask, objective=objective,
+                                inplace=True, **kw)
+    assert torch.equal(buf.detach(), dl) and torch.equal(out_i.loss, out.loss)
+
+
+@pytest.mark.parametrize("top", [1.0e8, 3.0e38])
+def test_lm_head_logits(device, top):
+    """The chunked LM head over logits as large, one tied with the target's:
+    d weight = d logits^T @ hidden."""
+
+    V, H = 512, 64
+    g = torch.Generator(device=device).manual_seed(5)
+    h = torch.zeros(1, 4, H, device=device)
+    h[0, :, 0] = torch.tensor([1.0, 1.0, 0.0, 0.0], device=device)
+    h[0, :, 1:] = 0.01 * torch.randn(4, H - 1, device=device, generator=g)
+    w = torch.zeros(V, H, device=device)
+    w[3, 0] = w[7, 0] = top
+    h, w = h.bfloat16().requires_grad_(), w.bfloat16().requires_grad_()
+    t = torch.tensor([[3, 9, 3, 9]], device=device)
+    x = (h.detach().double()[0] @ w.detach().double().t()).bfloat16().double()
+    lp = torch.log_softmax(x, dim=-1)
+    old = lp.gather(-1, t[0][:, None]).float().view(1, 4).clamp_min(-80.0)
+    adv = torch.tensor([[1.0, 0.0, -0.5, 2.0]], device=device)
+    mask = torch.ones_like(t, dtype=torch.bool)
+    out = R.fused_linear_policy_loss(h, w, t, old, adv, mask, objective="clipped", clip_low=0.2)
+    dh, dw = torch.autograd.grad(out.loss, (h, w))
+    assert torch.isfinite(dw).all()
+    up = -adv.double()[0][:, None] / 4
+    dl = -up * lp.exp()
+    dl.scatter_add_(-1, t[0][:, None], up)
+    want = dl.t() @ h.detach().double()[0]
+    # d logits and the product are each rounded to bfloat16
+    assert ((dw.double() - want).abs() <= 2.0 ** -6 * want.abs().max()).all()
+
+
+def test_rerun_flag_launches_nothing(device):
+    """RRL_POLICY_RERUN_FAST_RANGE (C callers): the first call's outputs stand
+    and its status word stays clear; without one the call is refused."""
+
+    import ctypes
+
+    from rosellm_amd import _native as nat
+    from rosellm_amd.roserlhf import losses as L
+
+    B, T, V = 1, 6, 4096
+    x, t = _rows(torch.bfloat16, V, device)
+    x[0, 2, 9] = 3.0e38
+    t[0, 2] = 11
+    z, one = torch.zeros(B, T, device=device), torch.ones(B, T, device=device)
+    mask = torch.ones_like(t, dtype=torch.bool)
+    coef = torch.full((B,), 1.0 / T, device=device)
+    rec = torch.empty(nat.lib().rrl_fused_records_bytes(B, T), dtype=torch.uint8, device=device)
+    lp, lse, dl = torch.empty_like(z), torch.empty_like(z), torch.empty_like(x)
+    status = nat.new_status(device)
+    p = L._params(nat.OBJ_PPO, clip_low=0.2, clip_high=0.2, mask_is_weight=True)
+
+    def call(flags, word):
+        p.flags = flags
+        v = [nat.rows_view(q, B, T)[0] for q in (t, z, one, mask)]
+        nat.call("rrl_fused_logprob_policy", ctypes.byref(p), x.data_ptr(), nat.BF16, B, T, V,
+                 T * V, V, *v, coef.data_ptr(), rec.data_ptr(), lp.data_ptr(), lse.data_ptr(),
+                 dl.data_ptr(), nat.BF16, T * V, V, word, nat.stream_ptr(device))
+
+    call(0, status.data_ptr())
+    first = (lp.clone(), lse.clone(), dl.clone())
+    assert int(status.item()) == 0 and torch.isfinite(dl).all()
+    call(nat.POLICY_RERUN_FAST_RANGE, status.data_ptr())
+    assert all(torch.equal(a, b) for a, b in zip(first, (lp, lse, dl)))
+    assert int(status.item()) == 0
+    with pytest.raises(RuntimeError, match="status word"):
+        call(nat.POLICY_RERUN_FAST_RANGE, None)
