@@ -36,11 +36,11 @@
 //      (finish_row), from pass 1's sums.
 // Greedy decoding is pass 1 alone; sampling without top-k / top-p is passes 1
 // and 5 (log q's floor excess is summed on pass 5's own read).  Top-k (up to
-// the lanes that hold data) and top-p first try a candidate list: the entries
-// at or above a lane-maximum threshold, gathered in one pass after pass 1 by
-// the few lanes that hold any; steps 2-5 then run on the list.  A list that
-// overflows, or that ends before the nucleus does, leaves the row to the
-// passes above.
+// list_top_k) and top-p (where the row's mass lies in few entries, NUC_SLACK)
+// first try a candidate list: the entries at or above a lane-maximum
+// threshold, gathered in one pass after pass 1 by the few lanes that hold any;
+// steps 2-5 then run on the list.  A list that overflows, or that ends before
+// the nucleus does, leaves the row to the passes above.
 // Ties at a top-k or top-p threshold are kept lowest index first; they are
 // located with the same vocabulary-order search over 0/1 weights.
 #include "row_common.hpp"
@@ -1017,6 +1017,33 @@ __device__ __forceinline__ void small_list_draw(CandShared& cs, SmallShared& ss,
 // Lane maxima at or above the nucleus list's threshold: of 1024 lanes, 448
 // leave a list of about 590 entries of the 1024 that fit.
 constexpr int NUC_NUM = 7, NUC_DEN = 16;
+// A list tried in vain costs its select and its pass over the row: 26 us
+// against 21 for 2000 float32 entries, 39 / 31 for 8192, 282 / 259 for 151936.
+// So the mass it can hold is estimated first, in one sum over the lanes: a
+// lane's largest term, or the lane's sum less twice the row's mean term for each
+// of its other entries (where large entries share a lane).  Where the list's
+// mass is 0.3 of the row or more, it is at most 1.02 times this sum over
+// independent normal logits of any spread, and 1.05 times with 64 candidates
+// side by side (1.00 with them scattered).
+constexpr float NUC_SLACK = 1.03f;
+
+// The largest top_k drawn from a lane-maximum list, by the bytes of a row.  The
+// list costs a select over the lanes, a pass and a rank among its 1.0-1.6 top_k
+// entries; without it a row takes 2 or 4 select passes and one more, which a
+// short row gets cheaply.  Up to 50 the short draw wins at any length; past 600
+// of 1024 lanes the list overflows.  us with the list / without, 64 rows:
+//   bytes per row        8 KB          16 KB         32 KB         64 KB        608 KB
+//   top_k =  50  f32  12.7 / 17.5   13.5 / 20.4   14.3 / 23.4   16.1 / 29.9    40 / 138
+//            100      18.8 / 18.1   19.8 / 21.0   20.6 / 24.2   22.5 / 30.6    47 / 139
+//            300      22.5 / 20.4   22.8 / 23.3   23.7 / 26.6   25.9 / 33.4    52 / 142
+//            400      28.2 / 21.4   24.3 / 24.3   26.9 / 27.5   29.9 / 34.5    57 / 143
+//            600            -       33.5 / 28.9   35.7 / 32.2   38.7 / 39.3    67 / 149
+//            100  f16  17.5 / 17.3  19.1 / 20.1        -        23.0 / 30.7       -
+//            300       21.2 / 19.7  22.0 / 22.7        -        27.2 / 33.8       -
+//            400       29.2 / 20.8  23.6 / 23.8        -        31.2 / 35.1       -
+__device__ __forceinline__ int list_top_k(int64_t row_bytes) {
+  return row_bytes < (12 << 10) ? 50 : row_bytes < (24 << 10) ? 300 : row_bytes < (48 << 10) ? 400 : 600;
+}
 
 // Top-p without top-k from a list: cs holds n <= KCAP entries, every entry of
 // the row at or above some key.  If the nucleus ends inside the list (its
@@ -1091,8 +1118,10 @@ __device__ __forceinline__ bool nucleus_list_draw(CandShared& cs, int n, int V, 
   const double fl = (double)1e-9f;
   const double total = tot + (double)(V - nk) * fl;
   const double target = u01 * total;
-  // [lo, hi) of consecutive kept entries tile [0, the last one's hi): excl is
-  // the previous thread's incl itself.
+  // [lo, hi) of consecutive kept entries tile [0, the last one's hi), so one
+  // thread claims: excl is the previous thread's incl itself, and a count times
+  // the floor is exact in float64 (24 bits by at most 20), fused with the sum
+  // or not.  Without floor entries in between, at = lo for the same reason.
   const double lo = tid > 0 ? excl + (double)(ep - (tid - 1)) * fl : 0.0;
   const double at = excl + (double)(ei - tid) * fl;
   const double hi = incl + (double)(ei - tid) * fl;
@@ -1210,13 +1239,15 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a, const int64_t r,
   __syncthreads();
   // Row totals relative to the row maximum: every entry (Z without top-k),
   // and every entry but the argmax (the greedy token's S_other).
-  float tot[2];
+  float tot[2], lane_top;
   {
     const float own = lane_max > -__builtin_huge_valf() ? 1.0f : 0.0f;
     const float f = bx > -__builtin_huge_valf() ? exp2_hw((lane_max - bx) * c2) : 0.0f;
+    lane_top = own * f;
     tot[0] = (sx + own) * f;
     tot[1] = (sx + (lane_arg == bi ? 0.0f : own)) * f;
   }
+  const float lane_sum = tot[0];
   block_sum<SNT, 2, float>(tot, sh_s);
   const float os = tot[0], s_arg_other = tot[1];
   const bool row_bad = bx == -__builtin_huge_valf() || bi >= V || os != os ||
@@ -1263,13 +1294,29 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a, const int64_t r,
       // The kq-th largest lane maximum t0 has at least kq entries at or above
       // it, so the entries at or above t0 hold the top kq and every tie.
       const int nlanes = min(SNT, (V + VEC - 1) / VEC);
-      const int kq = use_k ? (int)min(a.top_k, (int64_t)SNT + 1)
-                           : (use_p ? max(1, nlanes * NUC_NUM / NUC_DEN) : SNT + 1);
-      if (kq <= nlanes) {
-        const uint32_t lkey = float_key<KB>(Bits<Tag>::bits_of(lane_max));
-        const bool in_row = tid < nlanes;
-        const uint32_t t0 = block_kth_key<KB>(lkey, in_row, kq, hist, &sh_digit, &sh_above32);
-        if (tid == 0) cs.n = 0;
+      int kq = SNT + 1;
+      if (use_k) kq = a.top_k <= list_top_k((int64_t)V * sizeof(S)) ? (int)a.top_k : kq;
+      else if (use_p) kq = max(1, nlanes * NUC_NUM / NUC_DEN);
+      const uint32_t lkey = float_key<KB>(Bits<Tag>::bits_of(lane_max));
+      const bool in_row = tid < nlanes;
+      const uint32_t ninf = float_key<KB>(Bits<Tag>::bits_of(-__builtin_huge_valf()) &
+                                          (KB == 16 ? 0xffffu : 0xffffffffu));
+      bool worth = kq <= nlanes;
+      if (worth && !use_k) {
+        const float rest = 2.0f * (float)(nslab * VEC - 1) * os / (float)V;
+        const float held = wave_sum_dpp(fmaxf(lane_top, lane_sum - rest));
+        if (lane == 0) sh_s[wave] = held;
+        __syncthreads();  // sh_s is written again behind other barriers
+        float all = 0.0f;
+        for (int w = 0; w < SWAVES; ++w) all += sh_s[w];
+        worth = NUC_SLACK * all >= (float)a.top_p * os;
+      }
+      if (worth) {
+        uint32_t t0 = block_kth_key<KB>(lkey, in_row, kq, hist, &sh_digit, &sh_above32);
+        // With fewer finite lanes than kq top-k's list would hold the -inf
+        // entries, too, and is left out.  Top-p's need not, as they weigh nothing.
+        if (!use_k) t0 = max(t0, ninf + 1);
+        if (tid == 0) cs.n = t0 > ninf ? 0 : KCAP + 1;
         __syncthreads();
         for_slabs<Tag>(
             row, V, nslab,
@@ -1285,7 +1332,7 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a, const int64_t r,
                 }
               }
             },
-            in_row && lkey >= t0);
+            in_row && lkey >= t0 && t0 > ninf);
         __syncthreads();
         const int n = cs.n;
         uint32_t tok_bits;

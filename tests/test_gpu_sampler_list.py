@@ -29,6 +29,11 @@ def _rows(kind, B, V, dtype):
         x *= 0.01
     elif kind == "ties":  # a few values: thresholds are large tie groups
         x = torch.round(2.0 * x)
+    elif kind == "masked":  # fewer finite entries than lanes
+        x[torch.rand(B, V, generator=g) < 1.0 - 90.0 / V] = -float("inf")
+        x[:, V // 2] = 1.0
+    elif kind == "clump":  # the candidates share lanes
+        x[:, V // 3:V // 3 + 40] += 7.0
     return x.to(dtype)
 
 
@@ -53,6 +58,29 @@ def test_lists(device, dtype, V, kind, top_k, top_p):
         for got, w in ((out.logprobs, want["logp"]), (out.sampling_logprobs, want["logq"])):
             w = torch.from_numpy(w)[sure]
             assert torch.allclose(got.cpu().double()[sure], w, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("kind", ["peaked", "masked", "clump"])
+@pytest.mark.parametrize("kb", [12, 24, 48])
+@pytest.mark.parametrize("side", [-1, 1])
+def test_list_or_passes(device, kind, kb, side):
+    """Row lengths on both sides of the top-k list's limits, at each limit and one
+    past it, and nuclei that end inside and beyond the list."""
+
+    for dtype, size in ((torch.float32, 4), (torch.float16, 2)):
+        V = (kb << 10) // size + side
+        print(f"[sampler list] {dtype} V={V} {kind}", flush=True)
+        x = _rows(kind, 4, V, dtype)
+        for top_k, top_p in [(50, 1.0), (51, 0.9), (300, 1.0), (301, 1.0), (400, 0.95), (401, 1.0),
+                             (600, 1.0), (601, 1.0), (0, 0.5), (0, 0.8), (0, 0.97)]:
+            kw = dict(temperature=0.8, top_k=top_k, top_p=top_p, do_sample=True)
+            want = so.sample_rows(x.float().numpy(), seed=7, offset=2, **kw)
+            out = RI.sample_next_token_batch(x.to(device), seed=7, offset=2, **kw)
+            sure = torch.from_numpy((want["margin"] > 1e-5) & (want["p_margin"] > 1e-6))
+            assert torch.equal(out.token_ids.cpu()[sure], torch.from_numpy(want["token"])[sure])
+            for got, w in ((out.logprobs, want["logp"]), (out.sampling_logprobs, want["logq"])):
+                w = torch.from_numpy(w)[sure]
+                assert torch.allclose(got.cpu().double()[sure], w, rtol=1e-5, atol=1e-5)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
