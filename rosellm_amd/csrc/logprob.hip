@@ -1,15 +1,20 @@
 // Token log-probs over the vocabulary (losses.py:14-38), their backward, and the
 // single-pass log-prob + token-local objective gradient.
 //
-// One workgroup owns one logits row (b, t).  Sweep 1 streams the row with
-// 16-byte loads and keeps an online (max, sum exp) pair per lane, combined
-// across the wave with shuffles and across waves through LDS.  Sweep 2 (backward
-// and single pass) writes dlogits = g * (onehot - exp(x - lse)), so no softmax
-// tensor is ever materialised.  The register-resident kernels
-// (logprob_resident.hip) keep the whole row in registers between the sweeps for
-// bf16, f16 and float32 rows up to 163840 (16-bit) or 81920 (float32) entries;
-// this file is the generic path for float64, longer rows, accumulation and
-// dlogits rows laid out differently from the logits rows.
+// The generic kernel: one workgroup owns one logits row (b, t).  Sweep 1 streams
+// the row with 16-byte loads and keeps an online (max, sum exp) pair per lane,
+// combined across the wave with shuffles and across waves through LDS.  Sweep 2
+// (backward and single pass) writes dlogits = g * (onehot - exp(x - lse)), so no
+// softmax tensor is ever materialised.
+//
+// It takes every float64 row, and of bf16, f16 and float32 rows those of calls
+// that ask for it, give no log-probs (backward) or records (single pass), or want
+// dlogits laid out otherwise than the logits (another dtype, accumulation, rows
+// neither 16-byte aligned nor at their logits row's offset from a 128-byte
+// boundary) or rows of 2 GB.  The others run in
+// logprob_fwd.hip (the forward), logprob_resident.hip (single pass and backward
+// from registers; the backward of longer rows in pieces) and logprob_long.hip
+// (single pass of rows past 163840 16-bit or 81920 float32 entries).
 #include <mutex>
 
 #include "policy_math.hpp"

@@ -10,11 +10,11 @@
 //     rows, many of them per CU) to 1024 (one row per CU); see launch_variant.
 //   * A row of V 16-bit logits is held in VGPRs as SL slabs of one 16-byte
 //     vector per lane: slab k, lane j holds vector k*NT + j.  V = 151936
-//     (bf16) is 18992 vectors, 19 slabs of the NT = 1024, SL = 20 variant,
-//     i.e. 80 VGPRs.
-//   * Per-row scalars (target, old log-prob, advantage, mask weight * 1/M)
-//     come from a packed 16-byte record per token (pack_records_kernel), read
-//     a row ahead through the scalar cache.
+//     (bf16) is 18992 vectors, 19 slabs of 1024 lanes, i.e. 76 VGPRs.
+//   * Per-row scalars (target, old log-prob, advantage, mask weight) come from
+//     a packed 16-byte record per token (pack_records_kernel, or
+//     rrl_policy_prepare), the row coefficient from its array, both read a row
+//     ahead through the scalar cache.
 //   * Sweep 1 (registers only): online max / sum of exp over the non-target
 //     columns per lane, slab by slab as the loads land, then one LDS combine
 //     across the workgroup's waves.
@@ -542,22 +542,31 @@ int launch_resident(int mode, const RowArgs& a, int32_t nvec, int cus, hipStream
 // reduction and finish_row's serial chain, then its stores; a CU hides that
 // only behind other rows, so a short row takes a small workgroup and the CU
 // holds many (24 rows of 4096 bf16 entries with one wave each).  Measured
-// with 8192 rows, us for the fused pass (lanes per row 64 / 128 / 256 / 512 /
-// 1024; 1024 lanes and slabs in steps of four for every row before):
-//   V =  4096 bf16 (  512 vectors)   26 /  32 /  43 /  70 / 145
-//   V =  8192 bf16 ( 1024)           52 /  50 /  54 /  76 / 163
-//   V = 16000 bf16 ( 2000)            - / 102 /  99 / 102 / 173
-//   V = 24000 bf16 ( 3000)            - /   - / 150 / 143 / 221
-//   V = 32000 bf16 ( 4000)            - /   - / 204 / 190 / 218
-//   V = 50304 bf16 ( 6288)            - /   - /   - / 301 / 300
-//   V = 65536 bf16 ( 8192, 4096 rows) - /   - /   - / 186 / 204
-//   V = 20000 f32  ( 5000)            - /   - / 248 / 236 / 242
-//   V = 32000 f32  ( 8000, 4096 rows) - /   - /   - / 189 / 184
+// with 8192 rows, us at no fewer than 64 / 128 / 256 / 512 / 1024 lanes per
+// row, the fused pass and the backward (which has no reduction, and would take
+// 256 lanes where the fused pass takes fewer; it shares the fused pass's table):
+//   V =  4096 bf16 (  512 vectors)   20 /  29 /  35 /  84 / 198    24 /  24 /  24 /  50 / 123
+//   V =  8192 bf16 ( 1024)           47 /  47 /  51 /  88 / 214    45 /  45 /  44 /  53 / 125
+//   V = 16000 bf16 ( 2000)            - /  95 /  95 / 107 / 225     - /  92 /  92 /  97 / 129
+//   V = 24000 bf16 ( 3000)            - /   - / 146 / 139 / 237     - /   - / 140 / 142 / 153
+//   V = 32000 bf16 ( 4000)            - /   - / 185 / 186 / 250     - /   - / 193 / 192 / 195
+//   V = 50304 bf16 ( 6288)            - /   - /   - / 294 / 317     - /   - /   - / 306 / 305
+//   V = 65536 bf16 ( 8192, 4096 rows) - /   - /   - / 183 / 197     - /   - /   - / 184 / 185
+//   V = 20000 f32  ( 5000)            - /   - /   - / 233 / 247     - /   - /   - / 241 / 241
+//   V = 32000 f32  ( 8000, 4096 rows) - /   - /   - /   - / 183     - /   - /   - /   - / 186
 // A slab past the row's end costs its issue slots though it moves nothing:
 // 4000 vectors took 228 us with 13 slabs of 512 lanes against 190 with 8, so
-// the slab counts step by at most a sixth from 5 up.  With fewer than 2048
-// rows one- and two-wave workgroups leave the chip idle, and 256 lanes finish
-// each row sooner (512 rows of V = 8192: 11.5 / 10.7 / 9.1 / 10.1 / 15.3 us).
+// the slab counts step by one or two from 4 up.  With few rows one- and two-wave
+// workgroups leave the chip idle, and 256 lanes finish each row sooner; the fused
+// pass's lines cross between 1024 and 2048 rows, the backward's not at all, by
+// little (us with one wave, or two at 12000, against 256 lanes):
+//   rows            512          1024         1536         2048         4096
+//   V =  4096  6.5 /  5.5   7.2 /  7.0   8.6 /  8.9   8.9 / 10.4  11.8 / 18.1  fused
+//              4.3 /  4.4   4.9 /  4.3   6.0 /  5.9   7.4 /  6.8  12.5 / 11.7  backward
+//   V =  8192  8.5 /  6.5   9.0 /  8.9  11.6 / 10.7  11.9 / 13.8  20.2 / 26.4  fused
+//              5.3 /  4.5   7.2 /  6.8  10.0 /  9.7  12.2 / 11.6  23.3 / 22.6  backward
+//   V = 12000 10.4 /  8.1  11.3 / 11.1  15.9 / 14.0  16.5 / 16.9  36.8 / 36.3  fused
+//              6.4 /  5.3   8.8 /  9.2  13.7 / 12.8  17.4 / 17.1  35.8 / 33.1  backward
 template <class Tag, bool EXTRAS>
 int launch_variant(int mode, const RowArgs& a, int32_t nvec, hipStream_t stream) {
   int cus = 0;
