@@ -1041,7 +1041,7 @@ constexpr float NUC_SLACK = 1.03f;
 //            100  f16  17.5 / 17.3  19.1 / 20.1        -        23.0 / 30.7       -
 //            300       21.2 / 19.7  22.0 / 22.7        -        27.2 / 33.8       -
 //            400       29.2 / 20.8  23.6 / 23.8        -        31.2 / 35.1       -
-__device__ __forceinline__ int list_top_k(int64_t row_bytes) {
+inline int list_top_k(int64_t row_bytes) {
   return row_bytes < (12 << 10) ? 50 : row_bytes < (24 << 10) ? 300 : row_bytes < (48 << 10) ? 400 : 600;
 }
 
@@ -1151,8 +1151,10 @@ __device__ __forceinline__ bool nucleus_list_draw(CandShared& cs, int n, int V, 
 // One row of the streaming path, by the whole workgroup (every thread calls
 // it): sample_kernel's body, and the register-resident top-k kernel's path
 // for a row whose candidate list overflows.  cs, ss and hist: the caller's
-// LDS.  LIST: top-k and top-p try a candidate list from the lane maxima first
-// (the resident kernel has tried already).
+// LDS.  LIST: which candidate list from the lane maxima is tried first (kNoList:
+// the settings have none, or the resident kernel has tried).  Each list has a
+// kernel of its own: with the code of both in one, every setting took 1% longer
+// (64 x 151936 float32: the defaults 51.9 -> 52.5 us, top-k 50 41.7 -> 42.2).
 //
 // Reading the row bounds it, once per pass: a radix select over the row costs
 // four passes of float32 keys for top-k and four more, with exponentials and
@@ -1161,7 +1163,8 @@ __device__ __forceinline__ bool nucleus_list_draw(CandShared& cs, int n, int V, 
 // rows of 151936 float32 entries: top-k 50 with top-p 0.9 177 -> 51, top-p 0.9
 // 255 -> 66; for 64 rows of 50257 bf16 entries (read by vectors now, too)
 // 88 -> 24 and 139 -> 32, the defaults 57 -> 25.
-template <class Tag, bool LIST>
+enum List { kNoList, kTopKList, kNucleusList };
+template <class Tag, List LIST>
 __device__ __forceinline__ void sample_row(const SampleArgs& a, const int64_t r, CandShared& cs,
                                            SmallShared& ss, uint32_t* hist) {
   using S = typename Tag::S;
@@ -1239,15 +1242,13 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a, const int64_t r,
   __syncthreads();
   // Row totals relative to the row maximum: every entry (Z without top-k),
   // and every entry but the argmax (the greedy token's S_other).
-  float tot[2], lane_top;
+  float tot[2];
   {
     const float own = lane_max > -__builtin_huge_valf() ? 1.0f : 0.0f;
     const float f = bx > -__builtin_huge_valf() ? exp2_hw((lane_max - bx) * c2) : 0.0f;
-    lane_top = own * f;
     tot[0] = (sx + own) * f;
     tot[1] = (sx + (lane_arg == bi ? 0.0f : own)) * f;
   }
-  const float lane_sum = tot[0];
   block_sum<SNT, 2, float>(tot, sh_s);
   const float os = tot[0], s_arg_other = tot[1];
   const bool row_bad = bx == -__builtin_huge_valf() || bi >= V || os != os ||
@@ -1282,41 +1283,43 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a, const int64_t r,
   float logq = 0.0f;
   float s_other = s_arg_other;  // the argmax's; replaced below for another token
   if (!a.greedy) {
-    const bool use_k = a.top_k > 0 && a.top_k < V;
-    const bool use_p = a.top_p > 0.0 && a.top_p < 1.0;
+    // As launch_sample chose the kernel.
+    const bool use_k = LIST != kNucleusList && a.top_k > 0 && a.top_k < V;
+    const bool use_p = LIST == kNucleusList || (a.top_p > 0.0 && a.top_p < 1.0);
     uint32_t c[4] = {(uint32_t)r, (uint32_t)((uint64_t)r >> 32), (uint32_t)a.offset,
                      (uint32_t)(a.offset >> 32)};
     philox4x32_10(c, (uint32_t)a.seed, (uint32_t)(a.seed >> 32));
     const double u01 = (double)(c[0] >> 8) * 5.9604644775390625e-8;  // 2^-24
     const uint32_t max_key = float_key<KB>(load_one<Tag>(row, bi));
     bool drawn = false;
-    if constexpr (LIST) {
+    if constexpr (LIST != kNoList) {
       // The kq-th largest lane maximum t0 has at least kq entries at or above
       // it, so the entries at or above t0 hold the top kq and every tie.
       const int nlanes = min(SNT, (V + VEC - 1) / VEC);
-      int kq = SNT + 1;
-      if (use_k) kq = a.top_k <= list_top_k((int64_t)V * sizeof(S)) ? (int)a.top_k : kq;
-      else if (use_p) kq = max(1, nlanes * NUC_NUM / NUC_DEN);
-      const uint32_t lkey = float_key<KB>(Bits<Tag>::bits_of(lane_max));
-      const bool in_row = tid < nlanes;
-      const uint32_t ninf = float_key<KB>(Bits<Tag>::bits_of(-__builtin_huge_valf()) &
-                                          (KB == 16 ? 0xffffu : 0xffffffffu));
+      const int kq = LIST == kTopKList ? (int)a.top_k : max(1, nlanes * NUC_NUM / NUC_DEN);
       bool worth = kq <= nlanes;
-      if (worth && !use_k) {
+      if constexpr (LIST == kNucleusList) {
         const float rest = 2.0f * (float)(nslab * VEC - 1) * os / (float)V;
-        const float held = wave_sum_dpp(fmaxf(lane_top, lane_sum - rest));
+        const float top = exp2_hw((lane_max - bx) * c2);  // 0 where all is -inf
+        const float held = wave_sum_dpp(fmaxf(top, __builtin_fmaf(sx, top, top - rest)));
         if (lane == 0) sh_s[wave] = held;
-        __syncthreads();  // sh_s is written again behind other barriers
+        __syncthreads();  // sh_s is not written again in this kernel
         float all = 0.0f;
         for (int w = 0; w < SWAVES; ++w) all += sh_s[w];
         worth = NUC_SLACK * all >= (float)a.top_p * os;
       }
       if (worth) {
+        const uint32_t lkey = float_key<KB>(Bits<Tag>::bits_of(lane_max));
+        const bool in_row = tid < nlanes;
         uint32_t t0 = block_kth_key<KB>(lkey, in_row, kq, hist, &sh_digit, &sh_above32);
-        // With fewer finite lanes than kq top-k's list would hold the -inf
-        // entries, too, and is left out.  Top-p's need not, as they weigh nothing.
-        if (!use_k) t0 = max(t0, ninf + 1);
-        if (tid == 0) cs.n = t0 > ninf ? 0 : KCAP + 1;
+        if constexpr (LIST == kNucleusList) {
+          // -inf entries weigh nothing: with fewer finite lanes than kq the list
+          // holds every finite entry.
+          const uint32_t ninf = float_key<KB>(Bits<Tag>::bits_of(-__builtin_huge_valf()) &
+                                              (KB == 16 ? 0xffffu : 0xffffffffu));
+          t0 = max(t0, ninf + 1);
+        }
+        if (tid == 0) cs.n = 0;
         __syncthreads();
         for_slabs<Tag>(
             row, V, nslab,
@@ -1332,12 +1335,12 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a, const int64_t r,
                 }
               }
             },
-            in_row && lkey >= t0 && t0 > ninf);
+            in_row && lkey >= t0);
         __syncthreads();
         const int n = cs.n;
         uint32_t tok_bits;
         if (n <= KCAP) {
-          if (!use_k) {
+          if constexpr (LIST == kNucleusList) {
             drawn = nucleus_list_draw<Tag>(cs, n, V, a.top_p, iT, m, 1.0f / os, max_key, u01, tok,
                                            logq);
           } else if (n <= 64) {
@@ -1661,7 +1664,7 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a, const int64_t r,
   }
 }
 
-template <class Tag, bool LIST>
+template <class Tag, List LIST>
 __global__ __launch_bounds__(SNT) void sample_kernel(SampleArgs a) {
   __shared__ CandShared cs;
   __shared__ SmallShared ss;
@@ -1674,10 +1677,20 @@ __global__ __launch_bounds__(SNT) void sample_kernel(SampleArgs a) {
   sample_row<Tag, LIST>(a, r, cs, ss, hist);
 }
 
+template <class Tag, List LIST>
+int launch_sample_as(const SampleArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL((sample_kernel<Tag, LIST>), dim3((unsigned)a.B), dim3(SNT), 0, st, a);
+  return check_launch("sample_kernel");
+}
+
 template <class Tag>
 int launch_sample(const SampleArgs& a, hipStream_t st) {
-  hipLaunchKernelGGL((sample_kernel<Tag, true>), dim3((unsigned)a.B), dim3(SNT), 0, st, a);
-  return check_launch("sample_kernel");
+  if (!a.greedy && a.top_k > 0 && a.top_k < a.V)
+    return a.top_k <= list_top_k(a.V * (int64_t)sizeof(typename Tag::S))
+               ? launch_sample_as<Tag, kTopKList>(a, st)
+               : launch_sample_as<Tag, kNoList>(a, st);
+  if (!a.greedy && a.top_p > 0.0 && a.top_p < 1.0) return launch_sample_as<Tag, kNucleusList>(a, st);
+  return launch_sample_as<Tag, kNoList>(a, st);
 }
 
 // The fill-in launch behind the nucleus path: its rows are too flat for a
@@ -1685,7 +1698,7 @@ int launch_sample(const SampleArgs& a, hipStream_t st) {
 int launch_fill_in(const SampleArgs& a, hipStream_t st) {
   SampleArgs f = a;
   f.fill_in = 1;
-  hipLaunchKernelGGL((sample_kernel<TagBF16, false>), dim3((unsigned)f.B), dim3(SNT), 0, st, f);
+  hipLaunchKernelGGL((sample_kernel<TagBF16, kNoList>), dim3((unsigned)f.B), dim3(SNT), 0, st, f);
   return check_launch("sample_kernel");
 }
 
@@ -1903,7 +1916,7 @@ __global__ __launch_bounds__(SNT) void sample_resident_kernel(SampleArgs a) {
     // The list still overflows (coarse logits, many ties at the threshold):
     // this row takes the streaming path, re-reading it from memory, in this
     // launch.  (The registers' row is not needed past the gather.)
-    sample_row<Tag, false>(a, r, cs, ss, hist);
+    sample_row<Tag, kNoList>(a, r, cs, ss, hist);
     return;
   }
   const bool use_p = a.top_p > 0.0 && a.top_p < 1.0;
