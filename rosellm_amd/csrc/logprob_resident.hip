@@ -39,7 +39,7 @@ namespace {
 
 constexpr int kMaxSlabs = 20;       // slabs per lane: 80 VGPRs of the 128 at 4 waves per SIMD
 constexpr int kWavesPerSimd = 4;
-constexpr float kFmaLse = 128.0f;   // |lse| up to which the one-FMA exponent keeps 5e-6
+constexpr uint32_t kFmaLse = 0x43000000u;  // 128.0f: up to here the one-FMA exponent keeps 5e-6
 
 // Per-token records for the resident kernel (TokenRecord): the views' dtype
 // and stride handling happens here, once per token, so that the row loop reads
@@ -232,7 +232,10 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
     // workgroup: forming the difference in every row costs 1-2% of the
     // 151936-entry sweep.  The sign is applied to the packed words with one XOR
     // per dword.
-    const bool wide = EPV == 8 && fabsf(lse) > kFmaLse && lse - lse == 0.0f;
+    // kFmaLse < |lse| < inf, compared as bits in scalar registers.
+    const uint32_t lse_bits =
+        (uint32_t)__builtin_amdgcn_readfirstlane((int)(__float_as_uint(lse) & 0x7fffffffu));
+    const bool wide = EPV == 8 && lse_bits > kFmaLse && lse_bits < 0x7f800000u;
     const float lg = __log2f(fabsf(gr));
     const bool flip = gr > 0.0f;
     const uint32_t sgn = flip ? P::SGN2 : 0u;
@@ -265,7 +268,7 @@ __global__ __launch_bounds__(NT, kWavesPerSimd) void resident_fused_kernel(RowAr
       }
     };
     if constexpr (EPV == 8) {
-      if (wide) {
+      if (__builtin_expect(wide, 0)) {
         const float cm = lg - __log2f(s + exp2_hw((xt - m) * kLog2e));
         put_row([&](float xv) { return __builtin_fmaf(xv - m, kLog2e, cm); });
       } else {
