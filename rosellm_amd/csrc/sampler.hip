@@ -1152,9 +1152,11 @@ __device__ __forceinline__ bool nucleus_list_draw(CandShared& cs, int n, int V, 
 // it): sample_kernel's body, and the register-resident top-k kernel's path
 // for a row whose candidate list overflows.  cs, ss and hist: the caller's
 // LDS.  LIST: which candidate list from the lane maxima is tried first (kNoList:
-// the settings have none, or the resident kernel has tried).  Each list has a
-// kernel of its own: with the code of both in one, every setting took 1% longer
-// (64 x 151936 float32: the defaults 51.9 -> 52.5 us, top-k 50 41.7 -> 42.2).
+// the settings have none, or the resident kernel has tried; kGreedy: no draw).
+// Each has a kernel of its own: with the code of both lists in one, every setting
+// took 1% longer (64 x 151936 float32: the defaults 51.9 -> 52.5 us, top-k 50
+// 41.7 -> 42.2), and greedy decoding 1% beside the draws alone (64 x 50257
+// 11.1 -> 11.2).
 //
 // Reading the row bounds it, once per pass: a radix select over the row costs
 // four passes of float32 keys for top-k and four more, with exponentials and
@@ -1163,7 +1165,7 @@ __device__ __forceinline__ bool nucleus_list_draw(CandShared& cs, int n, int V, 
 // rows of 151936 float32 entries: top-k 50 with top-p 0.9 177 -> 51, top-p 0.9
 // 255 -> 66; for 64 rows of 50257 bf16 entries (read by vectors now, too)
 // 88 -> 24 and 139 -> 32, the defaults 57 -> 25.
-enum List { kNoList, kTopKList, kNucleusList };
+enum List { kNoList, kTopKList, kNucleusList, kGreedy };
 template <class Tag, List LIST>
 __device__ __forceinline__ void sample_row(const SampleArgs& a, const int64_t r, CandShared& cs,
                                            SmallShared& ss, uint32_t* hist) {
@@ -1282,7 +1284,7 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a, const int64_t r,
   int tok = bi;
   float logq = 0.0f;
   float s_other = s_arg_other;  // the argmax's; replaced below for another token
-  if (!a.greedy) {
+  if (LIST != kGreedy && !a.greedy) {
     // As launch_sample chose the kernel.
     const bool use_k = LIST != kNucleusList && a.top_k > 0 && a.top_k < V;
     const bool use_p = LIST == kNucleusList || (a.top_p > 0.0 && a.top_p < 1.0);
@@ -1292,7 +1294,7 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a, const int64_t r,
     const double u01 = (double)(c[0] >> 8) * 5.9604644775390625e-8;  // 2^-24
     const uint32_t max_key = float_key<KB>(load_one<Tag>(row, bi));
     bool drawn = false;
-    if constexpr (LIST != kNoList) {
+    if constexpr (LIST == kTopKList || LIST == kNucleusList) {
       // The kq-th largest lane maximum t0 has at least kq entries at or above
       // it, so the entries at or above t0 hold the top kq and every tie.
       const int nlanes = min(SNT, (V + VEC - 1) / VEC);
@@ -1685,11 +1687,12 @@ int launch_sample_as(const SampleArgs& a, hipStream_t st) {
 
 template <class Tag>
 int launch_sample(const SampleArgs& a, hipStream_t st) {
-  if (!a.greedy && a.top_k > 0 && a.top_k < a.V)
+  if (a.greedy) return launch_sample_as<Tag, kGreedy>(a, st);
+  if (a.top_k > 0 && a.top_k < a.V)
     return a.top_k <= list_top_k(a.V * (int64_t)sizeof(typename Tag::S))
                ? launch_sample_as<Tag, kTopKList>(a, st)
                : launch_sample_as<Tag, kNoList>(a, st);
-  if (!a.greedy && a.top_p > 0.0 && a.top_p < 1.0) return launch_sample_as<Tag, kNucleusList>(a, st);
+  if (a.top_p > 0.0 && a.top_p < 1.0) return launch_sample_as<Tag, kNucleusList>(a, st);
   return launch_sample_as<Tag, kNoList>(a, st);
 }
 
